@@ -893,56 +893,43 @@ struct GreenBatch {
   Green gr[2];
 };
 
-// A block is 64 consecutive i (coalesced rows) x 4 segments of NCH chunks of
-// GQ points of the line; each thread slides a register window of GQ + 2 KT
-// values along its segment, GQ new values per chunk, so every input is read
-// about (NCH GQ + 2 KT) / (NCH GQ) times (the halo rows of neighbouring
-// segments mostly from L2).  Coefficients beyond the system's K are zero.
-// Needs n1 % 64 == 0 and N % (4 GQ NCH) == 0.
-constexpr int GQ = 16;
-
-template <int DIR, typename R, int KT, int NCH>
+// One thread per column i and run of Q consecutive points of the line (i
+// fastest over the threads, so every load and store is coalesced): it loads
+// the Q + 2 KT values its outputs reach in one batch and filters them from
+// registers.  Coefficients beyond the system's K are zero.  Needs N % Q == 0
+// and 2 KT < N.
+template <int DIR, typename R, int KT, int Q>
 __global__ __launch_bounds__(256) void k_green(GreenBatch<R> B, int n1, int n2, int n3) {
   const int f = blockIdx.y;
   const int N = DIR == 1 ? n2 : n3;
   const int s = DIR == 1 ? n1 : n1 * n2;
-  const int nsg = N / (4 * GQ * NCH), nit = n1 / 64;
-  unsigned b = xcd_block(blockIdx.x, gridDim.x);
-  const int sg = (int)(b % nsg), rest = (int)(b / nsg);
-  const int it = rest % nit, other = rest / nit;   // other: k (DIR 1) or j (DIR 2)
-  const int i = it * 64 + (threadIdx.x & 63);
-  const int p0 = (sg * 4 + (threadIdx.x >> 6)) * GQ * NCH;
+  const unsigned runs = (unsigned)(N / Q), other_n = (unsigned)(DIR == 1 ? n3 : n2);   // other: k (DIR 1) or j (DIR 2)
+  const unsigned t = xcd_block(blockIdx.x, gridDim.x) * 256u + threadIdx.x;
+  if (t >= (unsigned)n1 * runs * other_n) return;
+  const int i = (int)(t % (unsigned)n1);
+  const unsigned rest = t / (unsigned)n1;
+  const int p0 = (int)(rest % runs) * Q, other = (int)(rest / runs);
   const int base = i + (DIR == 1 ? n1 * n2 * other : n1 * other);
   const Green& G = B.gr[B.which[f]];
+  const R* __restrict__ d = B.src[f];
+  R v[Q + 2 * KT];   // positions p0 - KT .. p0 + Q + KT - 1
+#pragma unroll
+  for (int q = 0; q < Q + 2 * KT; ++q) {
+    int p = p0 - KT + q;
+    p = p < 0 ? p + N : (p >= N ? p - N : p);
+    v[q] = d[base + p * s];
+  }
   double g[KT + 1];
 #pragma unroll
   for (int m = 0; m <= KT; ++m) g[m] = m <= G.K ? G.g[m] : 0.0;
-  const R* __restrict__ d = B.src[f];
-  auto at = [&](int p) {
-    p = p < 0 ? p + N : (p >= N ? p - N : p);
-    return (double)d[base + p * s];
-  };
-  double v[GQ + 2 * KT];   // window of positions pc - KT .. pc + GQ + KT - 1
 #pragma unroll
-  for (int q = 0; q < GQ + 2 * KT; ++q) v[q] = at(p0 - KT + q);
+  for (int q = 0; q < Q; ++q) {
+    double x = g[0] * (double)v[q + KT];
 #pragma unroll
-  for (int ch = 0; ch < NCH; ++ch) {
-    const int pc = p0 + ch * GQ;
-#pragma unroll
-    for (int q = 0; q < GQ; ++q) {
-      double x = g[0] * v[q + KT];
-#pragma unroll
-      for (int m = 1; m <= KT; ++m) x += g[m] * (v[q + KT - m] + v[q + KT + m]);
-      const int c = base + (pc + q) * s;
-      if (B.qadd[f]) B.qadd[f][c] = B.qadd[f][c] + (R)x;
-      else B.dst[f][c] = (R)x;
-    }
-    if (ch + 1 < NCH) {   // slide by GQ: the last 2 KT values become the head
-#pragma unroll
-      for (int q = 0; q < 2 * KT; ++q) v[q] = v[q + GQ];
-#pragma unroll
-      for (int q = 0; q < GQ; ++q) v[2 * KT + q] = at(pc + GQ + KT + q);
-    }
+    for (int m = 1; m <= KT; ++m) x += g[m] * ((double)v[q + KT - m] + (double)v[q + KT + m]);
+    const int c = base + (p0 + q) * s;
+    if (B.qadd[f]) B.qadd[f][c] = B.qadd[f][c] + (R)x;
+    else B.dst[f][c] = (R)x;
   }
 }
 
@@ -1455,13 +1442,23 @@ int launch_solve(melt_ctx* ctx, int dir, void* const* fields, int nfield, const 
 
 // y/z solves of the fused substep as Green filters: returns 1 (and launches
 // nothing) when a system needs the cyclic reduction instead.
+constexpr size_t GREEN_THREADS = 196608;
+
+// Truncation of the y and z filters: round-off of FP64; below half an ulp of
+// FP32 storage, and far below it on the grids only the one-thread-per-run
+// filter takes (they had the cyclic reduction's full accuracy before).
+double green_tol(const melt_ctx* ctx) {
+  if (!ctx->fp32) return 2e-17;
+  return ctx->n1 % 64 || ctx->n2 % 8 || ctx->n3 % 16 ? 1e-10 : 1e-8;
+}
+
 template <typename R>
 int launch_green(melt_ctx* ctx, int dir, void* const* src, void* const* dst, void* const* qadd, const double* betadx, int nfield,
                  int* used) {
   *used = 0;
   if (ctx->no_green) return 0;
   const int N = dir == 1 ? ctx->n2 : ctx->n3;
-  const double tol = ctx->fp32 ? 1e-8 : 2e-17;
+  const double tol = green_tol(ctx);
   GreenBatch<R> B{};
   int ng = 0;
   double bseen[2] = {0.0, 0.0};
@@ -1482,19 +1479,19 @@ int launch_green(melt_ctx* ctx, int dir, void* const* src, void* const* dst, voi
   }
   int kmax = std::max(B.gr[0].K, ng > 1 ? B.gr[1].K : 0);
   int KT = kmax <= 4 ? 4 : kmax <= 8 ? 8 : 12;
-  // KT < N / 2 keeps every window inside one period
-  if (ctx->n1 % 64 || N % (4 * GQ) || 2 * KT >= N) return 0;
-  // chunks per thread along z (the longest segment that tiles the line; along
-  // y single chunks measured faster, the extra blocks outweigh the halo)
-  const int nch = dir == 1 ? 1 : N % (16 * GQ) == 0 ? 4 : N % (8 * GQ) == 0 ? 2 : 1;
-  const int nsg = N / (4 * GQ * nch), nit = ctx->n1 / 64, other = dir == 1 ? ctx->n3 : ctx->n2;
-  dim3 grid((unsigned)(nsg * nit * other), nfield);
-#define GREEN_CASE(D, KK, NC) hipLaunchKernelGGL((k_green<D, R, KK, NC>), grid, dim3(256), 0, ctx->stream, B, ctx->n1, ctx->n2, ctx->n3)
-#define GREEN_NCH(D, KK) \
-  do { if (nch == 4) GREEN_CASE(D, KK, 4); else if (nch == 2) GREEN_CASE(D, KK, 2); else GREEN_CASE(D, KK, 1); } while (0)
-  if (dir == 1) { if (KT == 4) GREEN_NCH(1, 4); else if (KT == 8) GREEN_NCH(1, 8); else GREEN_NCH(1, 12); }
-  else { if (KT == 4) GREEN_NCH(2, 4); else if (KT == 8) GREEN_NCH(2, 8); else GREEN_NCH(2, 12); }
-#undef GREEN_NCH
+  if (2 * KT >= N) return 0;   // every window inside one period
+  // points per thread: longer runs read each value fewer times ((Q + 2 KT) / Q),
+  // as long as about three waves per SIMD are left (64^3 FP64, y + z: 4 points
+  // 9.7 + 11.0 us, 16 points 9.2 + 14.6; 96^3: 4 points 16.9 + 21.8, 8 points 13.7 + 19.9)
+  int Q = 4;
+  for (int c : {16, 8})
+    if (N % c == 0 && ctx->nc * (size_t)nfield / c >= GREEN_THREADS) { Q = c; break; }
+  const dim3 grid(nblocks(ctx->nc / Q, 256), nfield);
+#define GREEN_CASE(D, KK, QQ) hipLaunchKernelGGL((k_green<D, R, KK, QQ>), grid, dim3(256), 0, ctx->stream, B, ctx->n1, ctx->n2, ctx->n3)
+#define GREEN_Q(D, KK) do { if (Q == 16) GREEN_CASE(D, KK, 16); else if (Q == 8) GREEN_CASE(D, KK, 8); else GREEN_CASE(D, KK, 4); } while (0)
+  if (dir == 1) { if (KT == 4) GREEN_Q(1, 4); else if (KT == 8) GREEN_Q(1, 8); else GREEN_Q(1, 12); }
+  else { if (KT == 4) GREEN_Q(2, 4); else if (KT == 8) GREEN_Q(2, 8); else GREEN_Q(2, 12); }
+#undef GREEN_Q
 #undef GREEN_CASE
   MELT_HIP(hipGetLastError());
   *used = 1;
@@ -1504,11 +1501,27 @@ int launch_green(melt_ctx* ctx, int dir, void* const* src, void* const* dst, voi
 // The y and z solves of the fused substep as one pass (k_green_yz): returns 0
 // with *used = 0 (launching nothing) when the shapes or the systems do not fit,
 // and the caller runs the two passes instead.  Tuning key yz_jb: 0 default
-// (8 rows per block), 8 or 16 rows, 1 = always two passes.
-// planes per z segment at most: whole 256-plane lines measured fastest for
-// 8-byte values; 4-byte values (two columns per thread, half the blocks) need
-// the extra blocks of 128-plane segments (0.243 -> 0.169 ms at 256^3)
-constexpr int YZ_SEG_MAX8 = 256, YZ_SEG_MAX4 = 128;
+// (the rules below), 8 or 16 rows per block, 1 = always two passes.
+//
+// Two 8-wave blocks are resident on a CU, and a block's time is the planes it
+// marches, seg + 2 KT, so the pass takes about ceil(blocks / 512) (seg + 2 KT)
+// plane times (0.63 to 1.2 us each): the segment length that makes this least
+// is taken.  Measured at 128^3 FP64, 16 / 32 / 64 / 128 planes: 63 / 52 / 74 /
+// 124 us; 128^3 FP32: 29 / 38 / 61 / 108; 192^3 FP64, 48 / 64 / 96 / 192: 199 /
+// 173 / 221 / 212; 256^3 FP64, 64 / 128 / 256: 391 / 347 / 330; 384^3 FP64, 64 /
+// 128 / 192 / 384: 1390 / 1282 / 1278 / 1409.
+constexpr int YZ_SLOTS = 512;   // resident blocks on 256 CUs
+int yz_segment(int n1, int n2, int n3, int cols, int jb, int nfield, int KT) {
+  int best = 0;
+  long cost = 0;
+  for (int seg = 8; seg <= n3; seg += 8) {
+    if (n3 % seg) continue;
+    const long blocks = (long)(n3 / seg) * (n2 / jb) * (n1 / cols) * nfield;
+    const long c = (blocks + YZ_SLOTS - 1) / YZ_SLOTS * (seg + 2 * KT);
+    if (!best || c <= cost) { best = seg; cost = c; }
+  }
+  return best;
+}
 
 template <typename R>
 int launch_green_yz(melt_ctx* ctx, void* const* src, void* const* qadd, const double* by, const double* bz, int nfield, int* used) {
@@ -1516,7 +1529,12 @@ int launch_green_yz(melt_ctx* ctx, void* const* src, void* const* qadd, const do
   const int jb = ctx->tune[TUNE_YZ_JB] == 0 ? 8 : ctx->tune[TUNE_YZ_JB];
   if (ctx->no_green || (jb != 8 && jb != 16)) return 0;
   const int n1 = ctx->n1, n2 = ctx->n2, n3 = ctx->n3;
-  const double tol = ctx->fp32 ? 1e-8 : 2e-17;
+  // 8-byte values on narrow grids: the staged rows (8 + 2 KT for 8 filtered) and
+  // the few blocks cost more than a second pass over data that stays in the
+  // caches (64 x 64 x 64: 21 us fused, 20 as two passes; 64 x 64 x 256: 50 and 40;
+  // 128 x 128 x 96: 44 and 50; 4-byte values at 64^3: 13.6 and 16)
+  if (ctx->tune[TUNE_YZ_JB] == 0 && sizeof(R) == 8 && n1 < 128) return 0;
+  const double tol = green_tol(ctx);
   GreenYZ<R> B{};
   int ng = 0;
   double seen[2][2] = {};
@@ -1543,11 +1561,8 @@ int launch_green_yz(melt_ctx* ctx, void* const* src, void* const* qadd, const do
   // two columns per thread for 4-byte values where the rows allow it
   constexpr int C2 = sizeof(R) == 4 ? 2 : 1;   // (no 2-column instantiation for 8-byte values)
   const int C = C2 == 2 && n1 % 128 == 0 ? 2 : 1;
-  if (n1 % 64 || n2 % jb || n3 % GQ || 2 * KT >= n2 || 2 * KT >= n3) return 0;
-  // planes per z segment: the longest of the maximum above, 64, 32, 16 that tiles the line
-  int seg = GQ;
-  for (int s : {sizeof(R) == 4 ? YZ_SEG_MAX4 : YZ_SEG_MAX8, 64, 32})
-    if (n3 % s == 0) { seg = s; break; }
+  if (n1 % 64 || n2 % jb || n3 % 8 || 2 * KT >= n2 || 2 * KT >= n3) return 0;
+  const int seg = yz_segment(n1, n2, n3, 64 * C, jb, nfield, KT);
   dim3 grid((unsigned)((n3 / seg) * (n2 / jb) * (n1 / (64 * C))), nfield);
 #define YZ_CASE(KK, JB, CC) hipLaunchKernelGGL((k_green_yz<R, KK, JB, CC>), grid, dim3(64 * JB), 0, ctx->stream, B, n1, n2, n3, seg)
 #define YZ_JB(KK) \
