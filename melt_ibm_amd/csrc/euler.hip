@@ -1444,12 +1444,16 @@ int launch_solve(melt_ctx* ctx, int dir, void* const* fields, int nfield, const 
 // nothing) when a system needs the cyclic reduction instead.
 constexpr size_t GREEN_THREADS = 196608;
 
-// Truncation of the y and z filters: round-off of FP64; below half an ulp of
-// FP32 storage, and far below it on the grids only the one-thread-per-run
-// filter takes (they had the cyclic reduction's full accuracy before).
-double green_tol(const melt_ctx* ctx) {
-  if (!ctx->fp32) return 2e-17;
-  return ctx->n1 % 64 || ctx->n2 % 8 || ctx->n3 % 16 ? 1e-10 : 1e-8;
+// Truncation of the y (dir 1) and z (dir 2) filters: round-off of FP64, below
+// half an ulp of FP32 storage.  Grids off the 64-column (and, for z, 16-plane)
+// raster were solved by cyclic reduction: FP32 takes the filter there at FP64
+// round-off (the stored floats are the same but for rounding ties; 96^3 y + z 46
+// -> 22 us), FP64 keeps the cyclic reduction (0), whose last bits the surface
+// motion amplifies to 1e-9 within a few steps.
+double green_tol(const melt_ctx* ctx, int dir) {
+  const bool raster = ctx->n1 % 64 == 0 && (dir == 1 || ctx->n3 % 16 == 0);
+  if (!ctx->fp32) return raster ? 2e-17 : 0.0;
+  return raster ? 1e-8 : 2e-17;
 }
 
 template <typename R>
@@ -1458,7 +1462,8 @@ int launch_green(melt_ctx* ctx, int dir, void* const* src, void* const* dst, voi
   *used = 0;
   if (ctx->no_green) return 0;
   const int N = dir == 1 ? ctx->n2 : ctx->n3;
-  const double tol = green_tol(ctx);
+  const double tol = green_tol(ctx, dir);
+  if (tol == 0.0) return 0;
   GreenBatch<R> B{};
   int ng = 0;
   double bseen[2] = {0.0, 0.0};
@@ -1534,7 +1539,8 @@ int launch_green_yz(melt_ctx* ctx, void* const* src, void* const* qadd, const do
   // caches (64 x 64 x 64: 21 us fused, 20 as two passes; 64 x 64 x 256: 50 and 40;
   // 128 x 128 x 96: 44 and 50; 4-byte values at 64^3: 13.6 and 16)
   if (ctx->tune[TUNE_YZ_JB] == 0 && sizeof(R) == 8 && n1 < 128) return 0;
-  const double tol = green_tol(ctx);
+  if (n1 % 64 || n2 % jb || n3 % 16) return 0;
+  const double tol = green_tol(ctx, 2);
   GreenYZ<R> B{};
   int ng = 0;
   double seen[2][2] = {};
@@ -1561,7 +1567,7 @@ int launch_green_yz(melt_ctx* ctx, void* const* src, void* const* qadd, const do
   // two columns per thread for 4-byte values where the rows allow it
   constexpr int C2 = sizeof(R) == 4 ? 2 : 1;   // (no 2-column instantiation for 8-byte values)
   const int C = C2 == 2 && n1 % 128 == 0 ? 2 : 1;
-  if (n1 % 64 || n2 % jb || n3 % 8 || 2 * KT >= n2 || 2 * KT >= n3) return 0;
+  if (2 * KT >= n2 || 2 * KT >= n3) return 0;
   const int seg = yz_segment(n1, n2, n3, 64 * C, jb, nfield, KT);
   dim3 grid((unsigned)((n3 / seg) * (n2 / jb) * (n1 / (64 * C))), nfield);
 #define YZ_CASE(KK, JB, CC) hipLaunchKernelGGL((k_green_yz<R, KK, JB, CC>), grid, dim3(64 * JB), 0, ctx->stream, B, n1, n2, n3, seg)
