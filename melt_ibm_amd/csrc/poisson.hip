@@ -5,8 +5,8 @@
 // divergence of divg.f90 in the fused substep), y and z, division by the
 // modified wavenumbers -(ak3 + ak1 + ak2) (phini.f90:35-55) after the 1/N^3
 // normalisation (phcalc.f90:48-60), and the inverse transforms.  Each transform
-// is a Stockham radix-4/2/3 FFT of a tile of lines held in LDS, so each pass
-// reads and writes the spectrum once.  The z pass does forward FFT, division
+// is a radix-4/2/3 FFT of a tile of lines held in registers (32 to 512 points)
+// or LDS, so each pass reads and writes the spectrum once.  The z pass does forward FFT, division
 // and inverse FFT in one visit.
 //
 // The real transforms along x pack two real lines into one complex line
@@ -18,6 +18,7 @@
 // up to a multiple of 8 so every row starts on a 128-byte boundary.
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "common.h"
 
@@ -287,14 +288,31 @@ __global__ __launch_bounds__(FFT_NT) void k_fft_x_bwd(SpecArgs<T> S, FftPlan P, 
 }
 
 // ---------------------------------------------------------------- register FFTs
-// For lines of N = P*P points (P = 8 or 16) the y and z passes use the
-// two-level form X[k1 + P k2] = sum_b W_P^(b k2) W_N^(b k1) sum_a x[b + P a] W_P^(a k1):
-// thread b of a line loads x[b + P a] straight from HBM, does a P-point DFT in
-// registers, scales by W_N^(b k1) (twiddles of N staged in LDS), and one LDS
-// transpose hands it the P values of its k1 for the second P-point DFT, after
-// which it holds X[k1 + P k2] for every k2.  The inverse runs the same steps
-// from that layout in reverse.  One exchange (two barriers) per transform
-// instead of one per radix stage.
+// Lines of N = P*Q points are transformed in two stages with one LDS exchange
+// (two barriers a component) between them instead of one per radix: thread
+// b < Q of a line loads x[b + Q a], a < P, straight from HBM and transforms them
+// in registers (stage A); thread k < P then receives the Q values of its k,
+// finishes them in registers (stage B) and holds X[k + P q] for every q.
+//
+// 64 = 8 * 8 and 256 = 16 * 16: stage A is a P-point DFT and the twiddles
+// W_N^(b k), stage B a second DFT, X[k1 + P k2] = sum_b W_Q^(b k2) W_N^(b k1)
+// sum_a x[b + Q a] W_P^(a k1); the inverse runs the same steps from that layout
+// in reverse.
+//
+// The other lengths group the radix stages of lds_fft: stage A is its first
+// radices (product P), stage B the rest, each on the values a thread holds, with
+// the same twiddles, butterflies and order, so the results are those of lds_fft
+// to the last bit.  (In Stockham's order the first stages with product P
+// combine x[b + Q a] only, and the stages after them, from Ns = P on, the
+// elements k + P a only.)
+//
+// Where P and Q differ one stage runs on a part of the threads (whole waves);
+// the passes are bound by HBM or, on small grids, by the chain of barriers, so
+// the shorter chain is what counts.  All five passes of a solve against the
+// staged transforms above, us (FP64 / FP32): 48^3 64 -> 37 / 58 -> 36, 96^3 98 ->
+// 56 / 84 -> 44, 128^3 127 -> 82 / 106 -> 64, 192^3 258 -> 166 / 193 -> 109, 384^3
+// 2009 -> 1272 / 1152 -> 700, 512^3 5138 -> 2716 / 2755 -> 1599 (384^3 FP64 moves
+// 5.4 GB of spectrum and velocity: 1140 us at the rate of a copy).
 
 // cos(pi m / 8) and sin(pi m / 8), m = 0..15 (W_16^m = cos - i sin forward)
 template <typename T>
@@ -316,12 +334,28 @@ __device__ __forceinline__ cx<T> mul_w16(cx<T> v, bool inv) {
   else return cmul(v, w16<T>(m, inv));
 }
 
-// 4-point DFT of (v[o], v[o+s], v[o+2s], v[o+3s]) in place, natural order.
+// DFT of R values in place, natural order (the butterflies of fft_stage)
 template <typename T>
 __device__ __forceinline__ void dft4(cx<T>& x0, cx<T>& x1, cx<T>& x2, cx<T>& x3, bool inv) {
   cx<T> a0 = cadd(x0, x2), a1 = csub(x0, x2), a2 = cadd(x1, x3), d = csub(x1, x3);
   cx<T> a3 = inv ? mkc<T>(-d.y, d.x) : mkc<T>(d.y, -d.x);
   x0 = cadd(a0, a2); x1 = cadd(a1, a3); x2 = csub(a0, a2); x3 = csub(a1, a3);
+}
+template <typename T, int R>
+__device__ __forceinline__ void butterfly(cx<T> (&v)[R], bool inv) {
+  if constexpr (R == 4) {
+    dft4(v[0], v[1], v[2], v[3], inv);
+  } else if constexpr (R == 2) {
+    const cx<T> e = v[0], f = v[1];
+    v[0] = cadd(e, f); v[1] = csub(e, f);
+  } else {
+    static_assert(R == 3, "radix 2, 3 or 4");
+    const T c = T(-0.5), sn = (inv ? T(1) : T(-1)) * T(0.86602540378443864676);
+    const cx<T> sm = cadd(v[1], v[2]), df = csub(v[1], v[2]);
+    const cx<T> t1 = mkc<T>(v[0].x + c * sm.x, v[0].y + c * sm.y), t2 = mkc<T>(-sn * df.y, sn * df.x);   // t2 = i sn df
+    v[0] = cadd(v[0], sm);
+    v[1] = cadd(t1, t2); v[2] = csub(t1, t2);
+  }
 }
 
 // P-point DFT (P = 8, 16) of v[0..P-1] in registers; result in natural order.
@@ -360,264 +394,438 @@ __device__ __forceinline__ void dft_reg(cx<T> (&v)[P], bool inv) {
   }
 }
 
-constexpr int RF_NC = 8;   // kx columns per register-FFT block (8 x 16 B = one 128-byte line per row)
-constexpr int RF_NCZ = 8;  // the same for the z pass (16 and 32 measured slower)
+// Radix of the next stage of a plan with M points left (make_plan's order).
+constexpr int next_radix(int M) { return M % 4 == 0 ? 4 : M % 2 == 0 ? 2 : 3; }
 
-// LDS image of one block of NC lines: the exchange tile (NC x P rows of
-// pitch P+1) and the N twiddles.
-template <typename T, int P, int NC>
-struct RegFftLds {
-  static constexpr int lines = NC;
-  // The transposes move the real and then the imaginary parts through one
-  // tile of T (half the LDS of a complex tile, so more blocks fit per CU).
-  // Column c's P x (P+1) tile starts at c * CS; CS = 2 mod 16 puts the 16
-  // lanes of a 64-bit access in distinct bank pairs in both thread layouts
-  // (y/z: 8 columns x 2 threads per lane group; x: 16 threads of one column).
-  static constexpr int CS = P * (P + 1) + ((2 - P * (P + 1) % 16) + 16) % 16;
-  T ex[NC * CS];
-  cx<T> tw[P * P];
-};
-
-// v[q] of thread b of column c becomes v[b] of thread q (a P x P transpose
-// within the column), one component at a time.  The tile must be free on
-// entry (callers put a barrier after any earlier read of it).
-template <typename T, int P, int NC>
-__device__ __forceinline__ void reg_transpose(cx<T> (&v)[P], RegFftLds<T, P, NC>& L, int c, int b) {
-  T* e = L.ex + c * L.CS;
+// The stages of an N-point Stockham transform from Ns = P0 on, with product M, on
+// the M values v[a] = element k0 + P0 a a thread holds (L: product of those done;
+// k0 < P0 the thread's, 0 for the first stages).  The butterflies with twiddle 1
+// skip the product (1 - 0 i), which changes no value.
+template <typename T, int N, int P0, int M, int L = 1>
+__device__ __forceinline__ void stockham(cx<T> (&v)[M], const cx<T>* tw, int k0, bool inv) {
+  if constexpr (L < M) {
+    constexpr int R = next_radix(M / L), step = N / (P0 * L * R);
+    cx<T> o[M];
 #pragma unroll
-  for (int k1 = 0; k1 < P; ++k1) e[k1 * (P + 1) + b] = v[k1].x;
-  __syncthreads();
+    for (int j = 0; j < M / R; ++j) {
+      const int kk = j % L, k = k0 + P0 * kk;
+      cx<T> x[R];
 #pragma unroll
-  for (int q = 0; q < P; ++q) v[q].x = e[b * (P + 1) + q];
-  __syncthreads();
+      for (int r = 0; r < R; ++r) {
+        x[r] = v[j + r * (M / R)];
+        if (r > 0 && !(P0 == 1 && kk == 0)) {
+          cx<T> w = tw[k * r * step];
+          if (inv) w.y = -w.y;
+          x[r] = cmul(x[r], w);
+        }
+      }
+      butterfly<T, R>(x, inv);
 #pragma unroll
-  for (int k1 = 0; k1 < P; ++k1) e[k1 * (P + 1) + b] = v[k1].y;
-  __syncthreads();
+      for (int r = 0; r < R; ++r) o[(j / L) * L * R + kk + r * L] = x[r];
+    }
 #pragma unroll
-  for (int q = 0; q < P; ++q) v[q].y = e[b * (P + 1) + q];
+    for (int q = 0; q < M; ++q) v[q] = o[q];
+    // (keeps the next stage's twiddles from being loaded, and held, before this one is done)
+    if constexpr (M >= 24) __builtin_amdgcn_sched_barrier(0);
+    stockham<T, N, P0, M, L * R>(v, tw, k0, inv);
+  }
 }
 
-// One transform of the lines (column c, thread b) held as v[a] = x[b + P a]:
-// on return v[k2] = X[k1 + P k2] for k1 = b.
-template <typename T, int P, int NC>
-__device__ __forceinline__ void reg_fft_fwd(cx<T> (&v)[P], RegFftLds<T, P, NC>& L, int c, int b, bool inv) {
-  constexpr int N = P * P;
+// P-point DFT and the twiddles W_N^(b k1) of the square lengths
+template <typename T, int P>
+__device__ __forceinline__ void dft_twiddle(cx<T> (&v)[P], const cx<T>* tw, int b, bool inv) {
   dft_reg<T, P>(v, inv);
 #pragma unroll
   for (int k1 = 1; k1 < P; ++k1) {
-    cx<T> w = L.tw[(b * k1) % N];
+    cx<T> w = tw[b * k1];
     if (inv) w.y = -w.y;
     v[k1] = cmul(v[k1], w);
   }
-  reg_transpose<T, P, NC>(v, L, c, b);
-  dft_reg<T, P>(v, inv);
 }
 
-// Inverse of that layout: v[k2] = X[k1 + P k2] with k1 = b in, v[n2] =
-// x[b + P n2] out (unnormalised, like FFTW_BACKWARD when inv, else forward).
-template <typename T, int P, int NC>
-__device__ __forceinline__ void reg_fft_back(cx<T> (&v)[P], RegFftLds<T, P, NC>& L, int c, int b, bool inv) {
-  constexpr int N = P * P;
-  dft_reg<T, P>(v, inv);   // over k2: v[n1] = Z[k1 = b][n1]
+// Stage A of thread b and stage B of thread k.
+template <typename T, int P, int Q>
+__device__ __forceinline__ void stage_a(cx<T> (&v)[P], const cx<T>* tw, int b, bool inv) {
+  if constexpr (P == Q) dft_twiddle<T, P>(v, tw, b, inv);
+  else stockham<T, P * Q, 1, P>(v, tw, 0, inv);
+}
+template <typename T, int P, int Q>
+__device__ __forceinline__ void stage_b(cx<T> (&u)[Q], const cx<T>* tw, int k, bool inv) {
+  if constexpr (P == Q) dft_reg<T, Q>(u, inv);
+  else stockham<T, P * Q, P, Q>(u, tw, k, inv);
+}
+
+constexpr int RF_NC = 8;   // kx columns per register-FFT block (8 x 16 B = one 128-byte line per row; 16 and 32 measured slower)
+
+// LDS image of one block of NC lines: the exchange tile (per line P rows of
+// pitch Q+1) and the N twiddles.
+template <typename T, int P, int Q, int NC>
+struct RegFftLds {
+  // The exchanges move the real and then the imaginary parts through one
+  // tile of T (half the LDS of a complex tile, so more blocks fit per CU).
+  // Line c's tile starts at c * CS; CS = 2 mod 16 puts the 16 lanes of a
+  // 64-bit access in distinct bank pairs in both thread layouts (y/z: 8
+  // columns x 2 threads per lane group; x: the threads of one line).
+  static constexpr int CS = P * (Q + 1) + ((2 - P * (Q + 1) % 16) + 16) % 16;
+  T ex[NC * CS];
+  cx<T> tw[P * Q];
+};
+
+// Thread (c, b) of stage A (b < Q) holds v[k1], k1 < P; thread (d, k) of stage B
+// (k < P) receives u[q] = v[k] of thread (d, q), one component at a time.  The
+// tile must be free on entry (callers put a barrier after any earlier read of
+// it).  Every thread of the block calls this; those past their stage's count
+// only take part in the barriers.
+template <typename T, int P, int Q, int NC>
+__device__ __forceinline__ void exchange_ab(const cx<T> (&v)[P], cx<T> (&u)[Q], RegFftLds<T, P, Q, NC>& L, int c, int b, bool inA, int d, int k,
+                                            bool inB) {
+  T* ea = L.ex + c * L.CS + b;
+  const T* eb = L.ex + d * L.CS + k * (Q + 1);
+  if (inA)
 #pragma unroll
-  for (int n1 = 1; n1 < P; ++n1) {
-    cx<T> w = L.tw[(b * n1) % N];
-    if (inv) w.y = -w.y;
-    v[n1] = cmul(v[n1], w);
-  }
-  __syncthreads();   // every thread has read its forward exchange
-  reg_transpose<T, P, NC>(v, L, c, b);
-  dft_reg<T, P>(v, inv);   // over k1: v[n2] = x[b + P n2]
+    for (int k1 = 0; k1 < P; ++k1) ea[k1 * (Q + 1)] = v[k1].x;
+  __syncthreads();
+  if (inB)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) u[q].x = eb[q];
+  __syncthreads();
+  if (inA)
+#pragma unroll
+    for (int k1 = 0; k1 < P; ++k1) ea[k1 * (Q + 1)] = v[k1].y;
+  __syncthreads();
+  if (inB)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) u[q].y = eb[q];
+}
+// The reverse: thread (c, b) receives v[k1] = u[b] of thread (c, k1).
+template <typename T, int P, int Q, int NC>
+__device__ __forceinline__ void exchange_ba(cx<T> (&v)[P], const cx<T> (&u)[Q], RegFftLds<T, P, Q, NC>& L, int c, int b, bool inA, int d, int k,
+                                            bool inB) {
+  const T* ea = L.ex + c * L.CS + b;
+  T* eb = L.ex + d * L.CS + k * (Q + 1);
+  if (inB)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) eb[q] = u[q].x;
+  __syncthreads();
+  if (inA)
+#pragma unroll
+    for (int k1 = 0; k1 < P; ++k1) v[k1].x = ea[k1 * (Q + 1)];
+  __syncthreads();
+  if (inB)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) eb[q] = u[q].y;
+  __syncthreads();
+  if (inA)
+#pragma unroll
+    for (int k1 = 0; k1 < P; ++k1) v[k1].y = ea[k1 * (Q + 1)];
 }
 
-// y pass (N2 = P*P) with register FFTs: RF_NC kx columns x P threads per block.
-template <typename T, int P>
-__global__ __launch_bounds__(RF_NC * P) void k_fft_y_reg(SpecArgs<T> S, const cx<T>* __restrict__ tw, int inv, const int* __restrict__ gate) {
+// From stage B's order (thread b holds element b + P q in u[q]) to stage A's
+// (thread b holds element b + Q a in v[a]).
+template <typename T, int P, int Q, int NC>
+__device__ __forceinline__ void reorder_ba(cx<T> (&v)[P], const cx<T> (&u)[Q], RegFftLds<T, P, Q, NC>& L, int c, int b, bool inA, bool inB) {
+  T* e = L.ex + c * L.CS + b;
+  if (inB)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) e[P * q] = u[q].x;
+  __syncthreads();
+  if (inA)
+#pragma unroll
+    for (int a = 0; a < P; ++a) v[a].x = e[Q * a];
+  __syncthreads();
+  if (inB)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) e[P * q] = u[q].y;
+  __syncthreads();
+  if (inA)
+#pragma unroll
+    for (int a = 0; a < P; ++a) v[a].y = e[Q * a];
+}
+
+// Threads of a block of NC lines.
+constexpr int rf_threads(int P, int Q, int NC) { return NC * (P > Q ? P : Q); }
+
+// Element b + q of column c of a block's lines (rows rs apart): a block-uniform
+// base plus one 32-bit lane offset, so the P or Q addresses of a thread live in
+// scalar registers (as 64-bit lane addresses they take 2 P vector registers).
+template <typename T>
+struct Column {
+  char* base;
+  size_t row;     // bytes from row to row
+  unsigned off;   // of this thread (below 32 rows of 1024 x 520 bins: under 4 GiB)
+  __device__ __forceinline__ Column(cx<T>* p, size_t rs, int c, int b)
+      : base(reinterpret_cast<char*>(p)), row(rs * sizeof(cx<T>)), off((unsigned)(((size_t)b * rs + (size_t)c) * sizeof(cx<T>))) {}
+  __device__ __forceinline__ cx<T>& at(int q) const { return *reinterpret_cast<cx<T>*>(base + row * (size_t)q + off); }
+};
+
+// y pass (N2 = P*Q): RF_NC kx columns per block.
+template <typename T, int P, int Q, bool INV>
+__global__ __launch_bounds__(rf_threads(P, Q, RF_NC)) void k_fft_y_reg(SpecArgs<T> S, const cx<T>* __restrict__ tw, const int* __restrict__ gate) {
   if (gate && *gate == 0) return;
-  __shared__ RegFftLds<T, P, RF_NC> L;
-  constexpr int N = P * P;
+  __shared__ RegFftLds<T, P, Q, RF_NC> L;
+  constexpr int N = P * Q, NT = rf_threads(P, Q, RF_NC);
   const int t = threadIdx.x, c = t % RF_NC, b = t / RF_NC;
+  const bool inA = b < Q, inB = b < P;
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
   const int ntm = S.n1hp / RF_NC;
   const int m0 = (int)(blk % (unsigned)ntm) * RF_NC, k = (int)(blk / (unsigned)ntm);
-  for (int q = t; q < N; q += RF_NC * P) L.tw[q] = tw[q];
-  cx<T>* base = S.spec + (size_t)m0 + c + (size_t)S.n1hp * N * k;
-  const size_t rs = (size_t)S.n1hp;
-  cx<T> v[P];
+  for (int q = t; q < N; q += NT) L.tw[q] = tw[q];
+  const Column<T> col(S.spec + (size_t)m0 + (size_t)S.n1hp * N * k, (size_t)S.n1hp, c, b);
+  cx<T> v[P], u[Q];
+  if (inA)
 #pragma unroll
-  for (int a = 0; a < P; ++a) v[a] = base[rs * (b + P * a)];
+    for (int a = 0; a < P; ++a) v[a] = col.at(Q * a);
   __syncthreads();   // twiddles
-  reg_fft_fwd<T, P>(v, L, c, b, inv != 0);
+  if (inA) stage_a<T, P, Q>(v, L.tw, b, INV);
+  exchange_ab<T, P, Q, RF_NC>(v, u, L, c, b, inA, c, b, inB);
+  if (!inB) return;
+  stage_b<T, P, Q>(u, L.tw, b, INV);
 #pragma unroll
-  for (int k2 = 0; k2 < P; ++k2) base[rs * (b + P * k2)] = v[k2];
+  for (int k2 = 0; k2 < Q; ++k2) col.at(P * k2) = u[k2];
 }
 
 // z pass with register FFTs: forward FFT, 1/(N1 N2 N3), division by
 // -(ak3+ak1+ak2) with the zero mode set to 0 (phcalc.f90:40-73), inverse FFT.
-template <typename T, int P, int NC = RF_NCZ>
-__global__ __launch_bounds__(NC * P) void k_fft_z_solve_reg(SpecArgs<T> S, const cx<T>* __restrict__ tw, const double* __restrict__ ak1,
-                                                               const double* __restrict__ ak2, const double* __restrict__ ak3, double nrm,
-                                                               const int* __restrict__ gate) {
+template <typename T, int P, int Q>
+__global__ __launch_bounds__(rf_threads(P, Q, RF_NC), P * Q == 512 ? 2 : 1) void k_fft_z_solve_reg(SpecArgs<T> S, const cx<T>* __restrict__ tw,
+                                                                             const double* __restrict__ ak1, const double* __restrict__ ak2,
+                                                                             const double* __restrict__ ak3, double nrm,
+                                                                             const int* __restrict__ gate) {
   if (gate && *gate == 0) return;
-  __shared__ RegFftLds<T, P, NC> L;
-  constexpr int N = P * P;
-  const int t = threadIdx.x, c = t % NC, b = t / NC;
+  constexpr int N = P * Q, NT = rf_threads(P, Q, RF_NC);
+  __shared__ RegFftLds<T, P, Q, RF_NC> L;
+  __shared__ double lak[N];
+  const int t = threadIdx.x, c = t % RF_NC, b = t / RF_NC;
+  const bool inA = b < Q, inB = b < P;
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-  const int ntm = (S.n1hp + NC - 1) / NC;   // the last block may overhang the row
-  const int m0 = (int)(blk % (unsigned)ntm) * NC, j = (int)(blk / (unsigned)ntm);
-  for (int q = t; q < N; q += NC * P) L.tw[q] = tw[q];
-  const int m = m0 + c;
-  const bool col = m < S.n1hp;   // columns past the row transform zeros and store nothing
-  cx<T>* base = S.spec + (size_t)(col ? m : 0) + (size_t)S.n1hp * j;
-  const size_t rs = (size_t)S.n1hp * S.g.n2;
-  cx<T> v[P];
+  const int ntm = S.n1hp / RF_NC;
+  const int m0 = (int)(blk % (unsigned)ntm) * RF_NC, m = m0 + c, j = (int)(blk / (unsigned)ntm);
+  const double a1 = ak1[m], a2 = ak2[j];   // (the padding bins n1h <= m < n1hp are below n1)
+  for (int q = t; q < N; q += NT) {
+    L.tw[q] = tw[q];
+    lak[q] = ak3[q];
+  }
+  const Column<T> col(S.spec + (size_t)m0 + (size_t)S.n1hp * j, (size_t)S.n1hp * S.g.n2, c, b);
+  cx<T> v[P], u[Q];
+  if (inA)
 #pragma unroll
-  for (int a = 0; a < P; ++a) v[a] = col ? base[rs * (b + P * a)] : mkc<T>(0, 0);
+    for (int a = 0; a < P; ++a) v[a] = col.at(Q * a);
   __syncthreads();
-  reg_fft_fwd<T, P>(v, L, c, b, false);
+  if (inA) stage_a<T, P, Q>(v, L.tw, b, false);
+  exchange_ab<T, P, Q, RF_NC>(v, u, L, c, b, inA, c, b, inB);
+  if (inB) {
+    stage_b<T, P, Q>(u, L.tw, b, false);
 #pragma unroll
-  for (int k2 = 0; k2 < P; ++k2) {
-    const int p = b + P * k2;
-    if (m < S.n1h) {
-      double ev = -ak3[p] - ak1[m] - ak2[j];
-      double vx = (double)v[k2].x / nrm, vy = (double)v[k2].y / nrm;
-      if (m == 0 && j == 0 && p == 0) { vx = 0.0; vy = 0.0; }
-      else { vx = vx / ev; vy = vy / ev; }
-      v[k2] = mkc<T>((T)vx, (T)vy);
-    } else {
-      v[k2] = mkc<T>(0, 0);
+    for (int k2 = 0; k2 < Q; ++k2) {
+      // selected, not branched over: a branch per point keeps every operand of
+      // every division live (166 -> 138 registers at 256 points of FP64)
+      const int p = b + P * k2;
+      const double ev = -lak[p] - a1 - a2;
+      const double vx = (double)u[k2].x / nrm / ev, vy = (double)u[k2].y / nrm / ev;
+      const bool zero = m >= S.n1h || (m == 0 && j == 0 && p == 0);
+      u[k2] = mkc<T>(zero ? T(0) : (T)vx, zero ? T(0) : (T)vy);
     }
   }
-  reg_fft_back<T, P>(v, L, c, b, true);
+  if constexpr (P == Q) {   // back through the same steps in reverse
+    if (inB) dft_twiddle<T, Q>(u, L.tw, b, true);   // over k2: u[n1] = W_N^-(k1 n1) Z[k1 = b][n1]
+    __syncthreads();   // every thread has read its forward exchange
+    exchange_ba<T, P, Q, RF_NC>(v, u, L, c, b, inA, c, b, inB);
+    if (!inA) return;
+    dft_reg<T, P>(v, true);   // over k1: v[n2] = x[b + Q n2]
 #pragma unroll
-  for (int n2 = 0; n2 < P; ++n2)
-    if (col) base[rs * (b + P * n2)] = v[n2];
+    for (int n2 = 0; n2 < P; ++n2) col.at(Q * n2) = v[n2];
+  } else {   // the points in natural order, then the same two stages
+    __syncthreads();
+    reorder_ba<T, P, Q, RF_NC>(v, u, L, c, b, inA, inB);
+    if (inA) stage_a<T, P, Q>(v, L.tw, b, true);
+    __syncthreads();   // the reordered values are read
+    exchange_ab<T, P, Q, RF_NC>(v, u, L, c, b, inA, c, b, inB);
+    if (!inB) return;
+    stage_b<T, P, Q>(u, L.tw, b, true);
+#pragma unroll
+    for (int k2 = 0; k2 < Q; ++k2) col.at(P * k2) = u[k2];
+  }
 }
 
-// x pass, forward, with register FFTs (N1 = P*P): RF_XT threads per block,
-// thread (c, b) owns line pair c of the block (lines j, j+1 packed as real and
-// imaginary part, divergence formed at load as k_fft_x_fwd) and points
-// b + P a.  After the transform the two half spectra are separated with the
-// mirror bins N-m, exchanged through LDS.
-constexpr int RF_XT = 128;
+// Line pairs per block of the x passes: about 128 threads, and 2 NPB lines that
+// divide N (the passes have n1 = n2).
+constexpr int x_pairs(int N) { return N == 64 ? 16 : N == 512 ? 4 : 8; }
 
-template <typename Rf, typename T, int P>
-__global__ __launch_bounds__(RF_XT) void k_fft_x_fwd_reg(SpecArgs<T> S, const cx<T>* __restrict__ tw, const Rf* __restrict__ vx,
-                                                         const Rf* __restrict__ vy, const Rf* __restrict__ vz, const Rf* __restrict__ src,
-                                                         T usdtal, const int* __restrict__ gate, unsigned long long* __restrict__ div_slots) {
+// x pass, forward, with register FFTs (N1 = P*Q): thread (c, b) of stage A owns
+// line pair c of the block (lines j, j+1 packed as real and imaginary part,
+// divergence formed at load as k_fft_x_fwd) and points b + Q a.  After the
+// transform the two half spectra are separated with the mirror bins N-m,
+// exchanged through LDS.
+template <typename Rf, typename T, int P, int Q>
+__global__ __launch_bounds__(rf_threads(P, Q, x_pairs(P * Q))) void k_fft_x_fwd_reg(
+    SpecArgs<T> S, const cx<T>* __restrict__ tw, const Rf* __restrict__ vx, const Rf* __restrict__ vy, const Rf* __restrict__ vz,
+    const Rf* __restrict__ src, T usdtal, const int* __restrict__ gate, unsigned long long* __restrict__ div_slots) {
   if (gate && *gate == 0) return;
-  constexpr int N = P * P, NPB = RF_XT / P;   // line pairs per block
-  __shared__ RegFftLds<T, P, NPB> L;
+  constexpr int N = P * Q, NPB = x_pairs(N), NT = rf_threads(P, Q, NPB), TB = NT / NPB;
+  static_assert(N % (2 * NPB) == 0, "whole line pairs per block");
+  __shared__ RegFftLds<T, P, Q, NPB> L;
   static_assert(NPB * N <= (int)(sizeof(L.ex) / sizeof(L.ex[0])), "mirror exchange fits the transpose tile");
   const Grid& g = S.g;
-  const int t = threadIdx.x, b = t % P, c = t / P;
+  // stage A: TB threads a line, b < Q; stage B: the first NPB * P threads, P a line
+  const int t = threadIdx.x, b = t % TB, c = t / TB, kb = t % P, d = t / P;
+  const bool inA = b < Q, inB = d < NPB;
   int jt, k;
   tiled_2d(xcd_block(blockIdx.x, gridDim.x), g.n2 / (2 * NPB), g.n3, 16, 8, jt, k);  // the divergence reads rows j+1 and planes k+1
   const int j = jt * 2 * NPB + 2 * c, kp = k == g.n3 - 1 ? 0 : k + 1;
-  for (int q = t; q < N; q += RF_XT) L.tw[q] = tw[q];
+  for (int q = t; q < N; q += NT) L.tw[q] = tw[q];
   const T dx1 = (T)g.dx1, dx2 = (T)g.dx2, dx3 = (T)g.dx3;
   double dmax = 0.0;
-  cx<T> v[P];
+  cx<T> v[P], u[Q];
+  if (inA) {
+    // lines j0.. of the block start at a uniform base; a lane's two lines and
+    // their y neighbours at 32-bit offsets from it (j is even and n2 is, so only
+    // the row after the second line can wrap)
+    const size_t line = (size_t)N * ((size_t)(j - 2 * c) + (size_t)g.n2 * k), up = (size_t)N * ((size_t)(j - 2 * c) + (size_t)g.n2 * kp);
+    const int o = N * 2 * c + b, jw = j + 2 == g.n2 ? N * (2 - g.n2) : 2 * N;   // to the row after the second line
+    const Rf *px = vx + line, *py = vy + line, *pz = vz + line, *pu = vz + up, *ps = src + line;
 #pragma unroll
-  for (int a = 0; a < P; ++a) {
-    const int i = b + P * a, ip = i == N - 1 ? 0 : i + 1;
-    T z[2];
-#pragma unroll
-    for (int l = 0; l < 2; ++l) {
-      const int jj = j + l, jp = jj == g.n2 - 1 ? 0 : jj + 1;
-      const size_t idx = (size_t)i + (size_t)N * ((size_t)jj + (size_t)g.n2 * k);
+    for (int a = 0; a < P; ++a) {
+      const int i = o + Q * a;
+      T z[2];
       if (src) {
-        z[l] = (T)src[idx];
+        z[0] = (T)ps[i];
+        z[1] = (T)ps[i + N];
       } else {
-        const Rf x0 = vx[idx], x1 = vx[idx - i + ip], y0 = vy[idx], y1 = vy[(size_t)i + (size_t)N * ((size_t)jp + (size_t)g.n2 * k)];
-        const Rf z0 = vz[idx], z1 = vz[(size_t)i + (size_t)N * ((size_t)jj + (size_t)g.n2 * kp)];
-        T dq = ((T)x1 - (T)x0) * dx1 + ((T)y1 - (T)y0) * dx2 + ((T)z1 - (T)z0) * dx3;
-        z[l] = dq * usdtal;
-        if (div_slots)
-          dmax = fmax(dmax, fabs(((double)x1 - (double)x0) * g.dx1 + ((double)y1 - (double)y0) * g.dx2 + ((double)z1 - (double)z0) * g.dx3));
+        const int ip = a == P - 1 && b == Q - 1 ? i - (N - 1) : i + 1;
+        const Rf y[3] = {py[i], py[i + N], py[i + jw]};
+#pragma unroll
+        for (int l = 0; l < 2; ++l) {
+          const Rf x0 = px[i + l * N], x1 = px[ip + l * N], z0 = pz[i + l * N], z1 = pu[i + l * N];
+          T dq = ((T)x1 - (T)x0) * dx1 + ((T)y[l + 1] - (T)y[l]) * dx2 + ((T)z1 - (T)z0) * dx3;
+          z[l] = dq * usdtal;
+          if (div_slots)
+            dmax = fmax(dmax, fabs(((double)x1 - (double)x0) * g.dx1 + ((double)y[l + 1] - (double)y[l]) * g.dx2 + ((double)z1 - (double)z0) * g.dx3));
+        }
       }
+      v[a] = mkc<T>(z[0], z[1]);
     }
-    v[a] = mkc<T>(z[0], z[1]);
   }
   if (div_slots) block_max_to_slots(dmax, div_slots);
   __syncthreads();   // twiddles
-  reg_fft_fwd<T, P>(v, L, c, b, false);   // v[k2] = Z[b + P k2]
-  // mirror bins Z[N-m] of the line pair through LDS, one component at a time
-  T* zs = L.ex + c * N;
-  T zrx[P];
-  __syncthreads();   // the transpose tile is read
+  if (inA) stage_a<T, P, Q>(v, L.tw, b, false);
+  exchange_ab<T, P, Q, NPB>(v, u, L, c, b, inA, d, kb, inB);
+  if (inB) stage_b<T, P, Q>(u, L.tw, kb, false);   // u[k2] = Z[kb + P k2]
+  // mirror bins Z[N-m] of the line pair through LDS, one component at a time;
+  // a thread stores the bins kb + P k2 < n1hp, all but the last of them without
+  // a test (the bin counts follow from N)
+  constexpr int N1H = N / 2 + 1, N1HP = (N1H + 7) & ~7, KS = (N1HP + P - 1) / P;
+  T* zs = L.ex + (inB ? d : 0) * N;
+  T zrx[KS];
+  __syncthreads();   // the exchange tile is read
+  if (inB)
 #pragma unroll
-  for (int k2 = 0; k2 < P; ++k2) zs[b + P * k2] = v[k2].x;
+    for (int k2 = 0; k2 < Q; ++k2) zs[kb + P * k2] = u[k2].x;
   __syncthreads();
+  if (inB)
 #pragma unroll
-  for (int k2 = 0; k2 < P; ++k2) {
-    const int m = b + P * k2;
-    zrx[k2] = zs[m == 0 ? 0 : N - m];
-  }
+    for (int k2 = 0; k2 < KS; ++k2) zrx[k2] = zs[k2 == 0 && kb == 0 ? 0 : N - kb - P * k2];
   __syncthreads();
+  if (inB)
 #pragma unroll
-  for (int k2 = 0; k2 < P; ++k2) zs[b + P * k2] = v[k2].y;
+    for (int k2 = 0; k2 < Q; ++k2) zs[kb + P * k2] = u[k2].y;
   __syncthreads();
-  const size_t row = (size_t)S.n1hp * ((size_t)j + (size_t)g.n2 * k);
+  if (!inB) return;
+  cx<T>* out = S.spec + (size_t)N1HP * ((size_t)(jt * 2 * NPB) + (size_t)g.n2 * k);   // uniform; lanes at 32-bit offsets
+  const int o = N1HP * 2 * d + kb;
 #pragma unroll
-  for (int k2 = 0; k2 < P; ++k2) {
-    const int m = b + P * k2;
-    if (m >= S.n1hp) break;
-    cx<T> A = mkc<T>(0, 0), B = mkc<T>(0, 0);
-    if (m < S.n1h) {
-      const cx<T> z = v[k2], zr = mkc<T>(zrx[k2], zs[m == 0 ? 0 : N - m]);
-      // A = (Z[m] + conj Z[N-m]) / 2,  B = (Z[m] - conj Z[N-m]) / (2i)
-      A = mkc<T>((z.x + zr.x) * T(0.5), (z.y - zr.y) * T(0.5));
-      B = mkc<T>((z.y + zr.y) * T(0.5), (zr.x - z.x) * T(0.5));
-    }
-    S.spec[row + m] = A;
-    S.spec[row + S.n1hp + m] = B;
+  for (int k2 = 0; k2 < KS; ++k2) {
+    const int m = kb + P * k2;
+    if (P * k2 + P > N1HP && m >= N1HP) break;
+    const cx<T> z = u[k2], zr = mkc<T>(zrx[k2], zs[k2 == 0 && kb == 0 ? 0 : N - m]);
+    // A = (Z[m] + conj Z[N-m]) / 2,  B = (Z[m] - conj Z[N-m]) / (2i)
+    cx<T> A = mkc<T>((z.x + zr.x) * T(0.5), (z.y - zr.y) * T(0.5));
+    cx<T> B = mkc<T>((z.y + zr.y) * T(0.5), (zr.x - z.x) * T(0.5));
+    if (P * k2 + P > N1H && m >= N1H) A = B = mkc<T>(0, 0);
+    out[o + P * k2] = A;
+    out[o + N1HP + P * k2] = B;
   }
 }
 
-// x pass, backward, with register FFTs (FFTW c2r semantics as k_fft_x_bwd):
-// thread (c, b) packs Z = A + iB of line pair c for bins b + P k2 (the bins
-// above N/2 as conj(A) + i conj(B) of the mirror bin), transforms, and writes
-// line j from the real and line j+1 from the imaginary part.
-template <typename Rf, typename T, int P>
-__global__ __launch_bounds__(RF_XT) void k_fft_x_bwd_reg(SpecArgs<T> S, const cx<T>* __restrict__ tw, Rf* __restrict__ dst,
-                                                         const int* __restrict__ gate) {
+// Z = A + iB of a line pair at bin m (FFTW c2r semantics as k_fft_x_bwd), the
+// bins above N/2 as conj(A) + i conj(B) of the mirror bin; o: the pair's first
+// bin, row: bins per line.  lo <= m <= hi are known at compile time, so which
+// half a bin is in is only tested around N/2.
+template <typename T, int N>
+__device__ __forceinline__ cx<T> pair_bin(const cx<T>* __restrict__ in, int o, int row, int m, int lo, int hi) {
+  const bool lower = hi <= N / 2 || (lo <= N / 2 && m <= N / 2);
+  const int q = o + (lower ? m : N - m);
+  cx<T> A = in[q], B = in[q + row];
+  if (m == 0 || 2 * m == N) { A.y = T(0); B.y = T(0); }
+  return lower ? mkc<T>(A.x - B.y, A.y + B.x) : mkc<T>(A.x + B.y, B.x - A.y);
+}
+
+// x pass, backward, with register FFTs: the line pairs' bins are packed
+// (pair_bin) into the thread's order of the transform (in reverse from stage B
+// for the square lengths, else from stage A), and line j comes from the real,
+// line j+1 from the imaginary part.
+template <typename Rf, typename T, int P, int Q>
+__global__ __launch_bounds__(rf_threads(P, Q, x_pairs(P * Q))) void k_fft_x_bwd_reg(SpecArgs<T> S, const cx<T>* __restrict__ tw,
+                                                                                    Rf* __restrict__ dst, const int* __restrict__ gate) {
   if (gate && *gate == 0) return;
-  constexpr int N = P * P, NPB = RF_XT / P;
-  __shared__ RegFftLds<T, P, NPB> L;
+  constexpr int N = P * Q, NPB = x_pairs(N), NT = rf_threads(P, Q, NPB), TB = NT / NPB;
+  static_assert(N % (2 * NPB) == 0, "whole line pairs per block");
+  __shared__ RegFftLds<T, P, Q, NPB> L;
   const Grid& g = S.g;
-  const int t = threadIdx.x, b = t % P, c = t / P;
+  const int t = threadIdx.x, b = t % TB, c = t / TB, kb = t % P, d = t / P;
+  const bool inA = b < Q, inB = d < NPB;
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
   const int ntj = g.n2 / (2 * NPB);
-  const int j = (int)(blk % (unsigned)ntj) * 2 * NPB + 2 * c, k = (int)(blk / (unsigned)ntj);
-  for (int q = t; q < N; q += RF_XT) L.tw[q] = tw[q];
-  const size_t row = (size_t)S.n1hp * ((size_t)j + (size_t)g.n2 * k);
-  cx<T> v[P];
+  const int j0 = (int)(blk % (unsigned)ntj) * 2 * NPB, k = (int)(blk / (unsigned)ntj);
+  for (int q = t; q < N; q += NT) L.tw[q] = tw[q];
+  constexpr int N1HP = (N / 2 + 8) & ~7;
+  const cx<T>* in = S.spec + (size_t)N1HP * ((size_t)j0 + (size_t)g.n2 * k);   // uniform; lanes at 32-bit offsets
+  Rf* out = dst + (size_t)N * ((size_t)j0 + (size_t)g.n2 * k);
+  cx<T> v[P], u[Q];
+  if constexpr (P == Q) {
+    if (inB)
 #pragma unroll
-  for (int k2 = 0; k2 < P; ++k2) {
-    const int m = b + P * k2;
-    if (m < S.n1h) {
-      cx<T> A = S.spec[row + m], B = S.spec[row + S.n1hp + m];
-      if (m == 0 || 2 * m == N) { A.y = T(0); B.y = T(0); }
-      v[k2] = mkc<T>(A.x - B.y, A.y + B.x);   // A + iB
-    } else {
-      const cx<T> A = S.spec[row + (N - m)], B = S.spec[row + S.n1hp + (N - m)];
-      v[k2] = mkc<T>(A.x + B.y, B.x - A.y);   // conj(A) + i conj(B)
+      for (int k2 = 0; k2 < Q; ++k2) u[k2] = pair_bin<T, N>(in, N1HP * 2 * d, N1HP, kb + P * k2, P * k2, P * k2 + P - 1);
+    __syncthreads();   // twiddles
+    if (inB) dft_twiddle<T, Q>(u, L.tw, kb, true);   // over k2: u[n1] = W_N^-(k1 n1) Z[k1 = kb][n1]
+    exchange_ba<T, P, Q, NPB>(v, u, L, c, b, inA, d, kb, inB);
+    if (!inA) return;
+    dft_reg<T, P>(v, true);   // over k1: v[n2] = z[b + Q n2]
+    const int o = N * 2 * c + b;
+#pragma unroll
+    for (int n2 = 0; n2 < P; ++n2) {
+      out[o + Q * n2] = (Rf)v[n2].x;
+      out[o + N + Q * n2] = (Rf)v[n2].y;
     }
-  }
-  __syncthreads();   // twiddles
-  reg_fft_back<T, P>(v, L, c, b, true);   // v[n2] = z[b + P n2]
-  const size_t o0 = (size_t)N * ((size_t)j + (size_t)g.n2 * k);
+  } else {
+    if (inA)
 #pragma unroll
-  for (int n2 = 0; n2 < P; ++n2) {
-    const int i = b + P * n2;
-    dst[o0 + i] = (Rf)v[n2].x;
-    dst[o0 + N + i] = (Rf)v[n2].y;
+      for (int a = 0; a < P; ++a) v[a] = pair_bin<T, N>(in, N1HP * 2 * c, N1HP, b + Q * a, Q * a, Q * a + Q - 1);
+    __syncthreads();   // twiddles
+    if (inA) stage_a<T, P, Q>(v, L.tw, b, true);
+    exchange_ab<T, P, Q, NPB>(v, u, L, c, b, inA, d, kb, inB);
+    if (!inB) return;
+    stage_b<T, P, Q>(u, L.tw, kb, true);   // u[k2] = z[kb + P k2]
+    const int o = N * 2 * d + kb;
+#pragma unroll
+    for (int k2 = 0; k2 < Q; ++k2) {
+      out[o + P * k2] = (Rf)u[k2].x;
+      out[o + N + P * k2] = (Rf)u[k2].y;
+    }
   }
 }
 
-// P with P*P = n, or 0
-int reg_fft_p(int n) { return n == 256 ? 16 : n == 64 ? 8 : 0; }
+// Calls f(P, Q) (as integral constants) for a line length with a register FFT;
+// false otherwise: shorter lines are bound by their launches either way, and
+// 768 and 1024 points would hold 48 or more values a thread.
+template <class F>
+bool with_reg_fft(int n, F&& f) {
+#define RF(NN, PP, QQ) case NN: f(std::integral_constant<int, PP>{}, std::integral_constant<int, QQ>{}); return true;
+  switch (n) {
+    RF(32, 4, 8) RF(48, 4, 12) RF(64, 8, 8) RF(96, 16, 6) RF(128, 16, 8) RF(192, 16, 12) RF(256, 16, 16) RF(384, 16, 24) RF(512, 16, 32)
+    default: return false;
+  }
+#undef RF
+}
 
 bool make_plan(int N, FftPlan& P) {
   P.N = N;
@@ -702,19 +910,14 @@ int solve_t(melt_ctx* ctx, int fused_divg, const int* gate, unsigned long long* 
   size_t shx = sizeof(cx<T>) * (size_t)(nlx / 2) * (ctx->n1 + 1);
   T usdtal = T(1.0 / (ctx->dt * ctx->al));
   unsigned gx = (unsigned)((ctx->n2 / nlx) * ctx->n3);
-  // x lines of 64 or 256 points: register FFTs (RF_XT threads, RF_XT / P line pairs per block)
-  const int px = reg_fft_p(ctx->n1);
-  const unsigned grx = px ? (unsigned)((ctx->n2 / (2 * RF_XT / px)) * ctx->n3) : 0;
   const Rf* src = fused_divg ? nullptr : fld<Rf>(ctx, MELT_DPH);
   unsigned long long* dsl = fused_divg ? div_slots : nullptr;
   if (!gate) timing_begin(ctx, SLOT_DIVG_FFTX, &ev);
-  if (px == 16)
-    hipLaunchKernelGGL((k_fft_x_fwd_reg<Rf, T, 16>), dim3(grx), dim3(RF_XT), 0, ctx->stream, S, twx, fld<Rf>(ctx, MELT_VX), fld<Rf>(ctx, MELT_VY),
-                       fld<Rf>(ctx, MELT_VZ), src, usdtal, gate, dsl);
-  else if (px == 8)
-    hipLaunchKernelGGL((k_fft_x_fwd_reg<Rf, T, 8>), dim3(grx), dim3(RF_XT), 0, ctx->stream, S, twx, fld<Rf>(ctx, MELT_VX), fld<Rf>(ctx, MELT_VY),
-                       fld<Rf>(ctx, MELT_VZ), src, usdtal, gate, dsl);
-  else
+  if (!with_reg_fft(ctx->n1, [&](auto P, auto Q) {
+        constexpr int p = decltype(P)::value, q = decltype(Q)::value, npb = x_pairs(p * q);
+        hipLaunchKernelGGL((k_fft_x_fwd_reg<Rf, T, p, q>), dim3((unsigned)(ctx->n2 / (2 * npb) * ctx->n3)), dim3(rf_threads(p, q, npb)), 0,
+                           ctx->stream, S, twx, fld<Rf>(ctx, MELT_VX), fld<Rf>(ctx, MELT_VY), fld<Rf>(ctx, MELT_VZ), src, usdtal, gate, dsl);
+      }))
     hipLaunchKernelGGL((k_fft_x_fwd<Rf, T>), dim3(gx), dim3(FFT_NT), shx, ctx->stream, S, Px, twx, nlx, fld<Rf>(ctx, MELT_VX), fld<Rf>(ctx, MELT_VY),
                        fld<Rf>(ctx, MELT_VZ), src, usdtal, gate, dsl);
   MELT_HIP(hipGetLastError());
@@ -723,16 +926,16 @@ int solve_t(melt_ctx* ctx, int fused_divg, const int* gate, unsigned long long* 
   int nly = std::max(1, std::min(ctx->n1hp, (FFT_EPT * FFT_NT) / ctx->n2));
   size_t shy = sizeof(cx<T>) * (size_t)nly * ctx->n2;
   unsigned gy = (unsigned)(((ctx->n1hp + nly - 1) / nly) * ctx->n3);
-  // y and z lines of 64 or 256 points: register FFTs (RF_NC columns per block)
-  const int py = reg_fft_p(ctx->n2), pz = reg_fft_p(ctx->n3);
-  const unsigned gry = (unsigned)((ctx->n1hp / RF_NC) * ctx->n3), grz = (unsigned)(((ctx->n1hp + RF_NCZ - 1) / RF_NCZ) * ctx->n2);
-  auto fft_y = [&](int inv) {
-    if (py == 16) hipLaunchKernelGGL((k_fft_y_reg<T, 16>), dim3(gry), dim3(RF_NC * 16), 0, ctx->stream, S, twy, inv, gate);
-    else if (py == 8) hipLaunchKernelGGL((k_fft_y_reg<T, 8>), dim3(gry), dim3(RF_NC * 8), 0, ctx->stream, S, twy, inv, gate);
-    else hipLaunchKernelGGL((k_fft_y<T>), dim3(gy), dim3(FFT_NT), shy, ctx->stream, S, Py, twy, nly, inv, gate);
+  const unsigned gry = (unsigned)((ctx->n1hp / RF_NC) * ctx->n3), grz = (unsigned)((ctx->n1hp / RF_NC) * ctx->n2);
+  auto fft_y = [&](auto inv) {
+    if (!with_reg_fft(ctx->n2, [&](auto P, auto Q) {
+          constexpr int p = decltype(P)::value, q = decltype(Q)::value;
+          hipLaunchKernelGGL((k_fft_y_reg<T, p, q, decltype(inv)::value>), dim3(gry), dim3(rf_threads(p, q, RF_NC)), 0, ctx->stream, S, twy, gate);
+        }))
+      hipLaunchKernelGGL((k_fft_y<T>), dim3(gy), dim3(FFT_NT), shy, ctx->stream, S, Py, twy, nly, decltype(inv)::value ? 1 : 0, gate);
   };
   if (!gate) timing_begin(ctx, SLOT_FFTY, &ev);
-  fft_y(0);
+  fft_y(std::false_type{});
   MELT_HIP(hipGetLastError());
   if (!gate) timing_end(ctx, SLOT_FFTY, ev);
 
@@ -741,26 +944,26 @@ int solve_t(melt_ctx* ctx, int fused_divg, const int* gate, unsigned long long* 
   unsigned gz = (unsigned)(((ctx->n1hp + nlz - 1) / nlz) * ctx->n2);
   double nrm = (double)((long long)ctx->n1 * ctx->n2 * ctx->n3);
   if (!gate) timing_begin(ctx, SLOT_FFTZ_SOLVE, &ev);
-  if (pz == 16)
-    hipLaunchKernelGGL((k_fft_z_solve_reg<T, 16>), dim3(grz), dim3(RF_NCZ * 16), 0, ctx->stream, S, twz, ctx->ak1, ctx->ak2, ctx->ak3, nrm, gate);
-  else if (pz == 8)
-    hipLaunchKernelGGL((k_fft_z_solve_reg<T, 8>), dim3(grz), dim3(RF_NCZ * 8), 0, ctx->stream, S, twz, ctx->ak1, ctx->ak2, ctx->ak3, nrm, gate);
-  else
+  if (!with_reg_fft(ctx->n3, [&](auto P, auto Q) {
+        constexpr int p = decltype(P)::value, q = decltype(Q)::value;
+        hipLaunchKernelGGL((k_fft_z_solve_reg<T, p, q>), dim3(grz), dim3(rf_threads(p, q, RF_NC)), 0, ctx->stream, S, twz, ctx->ak1, ctx->ak2,
+                           ctx->ak3, nrm, gate);
+      }))
     hipLaunchKernelGGL((k_fft_z_solve<T>), dim3(gz), dim3(FFT_NT), shz, ctx->stream, S, Pz, twz, nlz, ctx->ak1, ctx->ak2, ctx->ak3, nrm, gate);
   MELT_HIP(hipGetLastError());
   if (!gate) timing_end(ctx, SLOT_FFTZ_SOLVE, ev);
 
   if (!gate) timing_begin(ctx, SLOT_IFFTY, &ev);
-  fft_y(1);
+  fft_y(std::true_type{});
   MELT_HIP(hipGetLastError());
   if (!gate) timing_end(ctx, SLOT_IFFTY, ev);
 
   if (!gate) timing_begin(ctx, SLOT_IFFTX, &ev);
-  if (px == 16)
-    hipLaunchKernelGGL((k_fft_x_bwd_reg<Rf, T, 16>), dim3(grx), dim3(RF_XT), 0, ctx->stream, S, twx, fld<Rf>(ctx, MELT_DPH), gate);
-  else if (px == 8)
-    hipLaunchKernelGGL((k_fft_x_bwd_reg<Rf, T, 8>), dim3(grx), dim3(RF_XT), 0, ctx->stream, S, twx, fld<Rf>(ctx, MELT_DPH), gate);
-  else
+  if (!with_reg_fft(ctx->n1, [&](auto P, auto Q) {
+        constexpr int p = decltype(P)::value, q = decltype(Q)::value, npb = x_pairs(p * q);
+        hipLaunchKernelGGL((k_fft_x_bwd_reg<Rf, T, p, q>), dim3((unsigned)(ctx->n2 / (2 * npb) * ctx->n3)), dim3(rf_threads(p, q, npb)), 0,
+                           ctx->stream, S, twx, fld<Rf>(ctx, MELT_DPH), gate);
+      }))
     hipLaunchKernelGGL((k_fft_x_bwd<Rf, T>), dim3(gx), dim3(FFT_NT), shx, ctx->stream, S, Px, twx, nlx, fld<Rf>(ctx, MELT_DPH), gate);
   MELT_HIP(hipGetLastError());
   if (!gate) timing_end(ctx, SLOT_IFFTX, ev);
@@ -768,6 +971,5 @@ int solve_t(melt_ctx* ctx, int fused_divg, const int* gate, unsigned long long* 
 }
 
 int poisson_solve(melt_ctx* ctx, int fused_divg, const int* gate, unsigned long long* div_slots) {
-  if (!ctx->fp32) return solve_t<double, double>(ctx, fused_divg, gate, div_slots);
-  return ctx->spec64 ? solve_t<float, double>(ctx, fused_divg, gate, div_slots) : solve_t<float, float>(ctx, fused_divg, gate, div_slots);
+  return ctx->fp32 ? solve_t<float, float>(ctx, fused_divg, gate, div_slots) : solve_t<double, double>(ctx, fused_divg, gate, div_slots);
 }
