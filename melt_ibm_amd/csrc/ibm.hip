@@ -291,25 +291,31 @@ struct Win3 { int e[3]; };
 // Face base indices floor(x*dx)+1 (unwrapped) bound every cell the MLS
 // supports (base-1..base+2) and the tagging band (base-2..base+2) touch.
 // Min / max of the face base indices over all live faces: one block per 256
-// faces, combined with integer atomics (order-independent).
+// faces, wave shuffles and then integer atomics (order-independent; shared
+// atomics of 256 threads on one address serialise, 15 -> 5 us for the tagging's
+// set-up).
 __device__ void window_box_block(const Grid& g, const double* __restrict__ bar, const unsigned char* __restrict__ gf, int nf, melt_window* win,
                                  int blk) {
-  __shared__ int mn[3], mx[3];
-  if (threadIdx.x < 3) { mn[threadIdx.x] = INT_MAX; mx[threadIdx.x] = INT_MIN; }
-  __syncthreads();
-  int f = blk * blockDim.x + threadIdx.x;
-  if (f < nf && !gf[f]) {
-    const double dx[3] = {g.dx1, g.dx2, g.dx3};
-    for (int d = 0; d < 3; ++d) {
-      int b = (int)floor(bar[3 * f + d] * dx[d]) + 1;
-      atomicMin(&mn[d], b);
-      atomicMax(&mx[d], b);
+  __shared__ int mn[3][4], mx[3][4];
+  const int f = blk * 256 + (int)threadIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const bool live = f < nf && !gf[f];
+  const double dx[3] = {g.dx1, g.dx2, g.dx3};
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const int b = live ? (int)floor(bar[3 * f + d] * dx[d]) + 1 : 0;
+    int lo = live ? b : INT_MAX, hi = live ? b : INT_MIN;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      lo = min(lo, __shfl_xor(lo, o, 64));
+      hi = max(hi, __shfl_xor(hi, o, 64));
     }
+    if (lane == 0) { mn[d][w] = lo; mx[d][w] = hi; }
   }
   __syncthreads();
   if (threadIdx.x < 3) {
-    atomicMin(&win->bmin[threadIdx.x], mn[threadIdx.x]);
-    atomicMax(&win->bmax[threadIdx.x], mx[threadIdx.x]);
+    const int d = threadIdx.x;
+    atomicMin(&win->bmin[d], min(min(mn[d][0], mn[d][1]), min(mn[d][2], mn[d][3])));
+    atomicMax(&win->bmax[d], max(max(mx[d][0], mx[d][1]), max(mx[d][2], mx[d][3])));
   }
 }
 __global__ __launch_bounds__(256) void k_window_box(Grid g, const double* __restrict__ bar, const unsigned char* __restrict__ gf, int nf,
@@ -330,11 +336,10 @@ __global__ void k_window_reset(melt_window* win, int n) {
 }
 
 // Place the forcing (which & 1: win[0]) and / or tagging (which & 2: win[1])
-// box from the face extent reduced into win[0].bmin/bmax, then reset the
-// extent for the next call.
-__global__ void k_window_final(melt_window* win, Win3 ef, Win3 et, int which, int* err) {
-  int mn[3], mx[3];
-  for (int d = 0; d < 3; ++d) { mn[d] = win[0].bmin[d]; mx[d] = win[0].bmax[d]; win[0].bmin[d] = INT_MAX; win[0].bmax[d] = INT_MIN; }
+// box from the face extent in win[0].bmin/bmax (one thread).
+__device__ void window_place(melt_window* win, const Win3& ef, const Win3& et, int which, int* err) {
+  const int* mn = win[0].bmin;
+  const int* mx = win[0].bmax;
   if (which & 1) {  // forcing window
     melt_window& w = win[0];
     for (int d = 0; d < 3; ++d) {
@@ -354,6 +359,14 @@ __global__ void k_window_final(melt_window* win, Win3 ef, Win3 et, int which, in
     }
     w.pad = 1;  // current box is valid from now on
   }
+}
+// Reset the extent for the next call.
+__device__ void window_reset_extent(melt_window* win) {
+  for (int d = 0; d < 3; ++d) { win[0].bmin[d] = INT_MAX; win[0].bmax[d] = INT_MIN; }
+}
+__global__ void k_window_final(melt_window* win, Win3 ef, Win3 et, int which, int* err) {
+  window_place(win, ef, et, which, err);
+  window_reset_extent(win);
 }
 
 // ------------------------------------------------------------ narrow band
@@ -412,10 +425,9 @@ __device__ double dist_point_tri(const double P[3], const double* V0, const doub
 // The tagging's set-up in one launch: blocks [0, nbox) reduce the face
 // extent (as k_window_box), the other 256 set sdf to 999 over the window the
 // previous tagging wrote (that tagging's cells are re-tagged from scratch)
-// and clear the per-cell keys.  This runs before k_window_final moves the
-// tagging window, so it takes the previous window from where
-// k_window_final's update leaves it (prev_org := org, prev_valid := pad,
-// while prev_valid >= 0).
+// and clear the per-cell keys.  This runs before window_place moves the
+// tagging window, so it takes the previous window from where its update leaves
+// it (prev_org := org, prev_valid := pad, while prev_valid >= 0).
 template <typename R>
 __global__ __launch_bounds__(256) void k_tag_prepare(Grid g, const double* __restrict__ bar, const unsigned char* __restrict__ gf, int nf,
                                                      int nbox, melt_window* win, R* __restrict__ sdf, Win3 et,
@@ -424,18 +436,19 @@ __global__ __launch_bounds__(256) void k_tag_prepare(Grid g, const double* __res
     window_box_block(g, bar, gf, nf, win, blockIdx.x);
     return;
   }
-  const size_t t0 = (size_t)(blockIdx.x - nbox) * blockDim.x + threadIdx.x, step = (size_t)(gridDim.x - nbox) * blockDim.x;
+  // (window cells are below 2^30: 32-bit indices)
+  const unsigned t0 = (blockIdx.x - (unsigned)nbox) * 256u + threadIdx.x, step = (gridDim.x - (unsigned)nbox) * 256u;
   const melt_window& w = win[1];
   const bool moved = w.prev_valid >= 0;
   if ((moved ? w.pad : w.prev_valid) > 0) {
     const int o0 = moved ? w.org[0] : w.prev_org[0], o1 = moved ? w.org[1] : w.prev_org[1], o2 = moved ? w.org[2] : w.prev_org[2];
-    const size_t n = (size_t)et.e[0] * et.e[1] * et.e[2];
-    for (size_t s = t0; s < n; s += step) {
-      int a = (int)(s % et.e[0]), b = (int)((s / et.e[0]) % et.e[1]), c = (int)(s / ((size_t)et.e[0] * et.e[1]));
-      sdf[widx(g, o0 + a, o1 + b, o2 + c)] = R(999.0);
+    const unsigned e0 = (unsigned)et.e[0], e1 = (unsigned)et.e[1], n = e0 * e1 * (unsigned)et.e[2];
+    for (unsigned s = t0; s < n; s += step) {
+      const unsigned r = s / e0, c = r / e1;
+      sdf[widx(g, o0 + (int)(s - r * e0), o1 + (int)(r - c * e1), o2 + (int)c)] = R(999.0);
     }
   }
-  for (size_t s = t0; s < ncell; s += step) {
+  for (unsigned s = t0; s < ncell; s += step) {
     key[s] = ~0ull;
     face[s] = INT_MAX;
   }
@@ -450,13 +463,19 @@ struct MeshArgs {
   int nf;
 };
 
-// mode 0: distance of every (face, band cell), kept in dist[], and the min
-// per cell; 1: lowest face among the minima; 2: write sdf and VOFp
-template <typename R>
-__global__ __launch_bounds__(256) void k_tag_pass(Grid g, MeshArgs M, const melt_window* __restrict__ win, Win3 et,
+// MODE 0: distance of every (face, band cell), kept in dist[], and the min
+// per cell; 1: lowest face among the minima; 2: write sdf and VOFp.  The window
+// follows from the extent k_tag_prepare reduced: modes 0 and 1 take its origin
+// straight from there, one thread of mode 1 places the windows (no thread of
+// modes 0 and 1 reads the placed origin), and one of mode 2 resets the extent
+// (mode 2 reads the placed origin), so no launch of its own does.
+template <int MODE, typename R>
+__global__ __launch_bounds__(256) void k_tag_pass(Grid g, MeshArgs M, melt_window* __restrict__ win, Win3 ef, Win3 et, int which,
                                                   unsigned long long* __restrict__ key, int* __restrict__ face, double* __restrict__ dst,
-                                                  R* __restrict__ sdf, R* __restrict__ vofp, int mode, double pi, int* err) {
-  size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+                                                  R* __restrict__ sdf, R* __restrict__ vofp, double pi, int* err) {
+  const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (MODE == 1 && id == 0) window_place(win, ef, et, which, err);
+  if (MODE == 2 && id == 0) window_reset_extent(win);
   if (id >= (size_t)M.nf * 125) return;
   int f = (int)(id / 125), q = (int)(id % 125);
   if (M.gf[f]) return;
@@ -464,9 +483,12 @@ __global__ __launch_bounds__(256) void k_tag_pass(Grid g, MeshArgs M, const melt
   int i = (int)floor(pos[0] * g.dx1) + 1 + (q % 5) - 2;
   int j = (int)floor(pos[1] * g.dx2) + 1 + (q / 5) % 5 - 2;
   int k = (int)floor(pos[2] * g.dx3) + 1 + q / 25 - 2;
-  long long s = win_slot(win[1].org, et.e, i, j, k);
+  int org[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) org[d] = MODE == 2 ? win[1].org[d] : win[0].bmin[d] - 2;
+  long long s = win_slot(org, et.e, i, j, k);
   if (s < 0) { raise_error(err, MELT_ERR_WINDOW); return; }
-  if (mode == 0) {
+  if constexpr (MODE == 0) {
     const double* V0 = &M.xyzv[3 * M.vof[3 * f + 0]];
     const double* V1 = &M.xyzv[3 * M.vof[3 * f + 1]];
     const double* V2 = &M.xyzv[3 * M.vof[3 * f + 2]];
@@ -474,24 +496,24 @@ __global__ __launch_bounds__(256) void k_tag_pass(Grid g, MeshArgs M, const melt
     double dist = dist_point_tri(P, V0, V1, V2);
     dst[id] = dist;
     atomicMin(&key[s], (unsigned long long)__double_as_longlong(dist));
-    return;
-  }
-  const double dist = dst[id];
-  if (mode == 1) {
-    if (key[s] == (unsigned long long)__double_as_longlong(dist)) atomicMin(&face[s], f);
-  } else if (face[s] == f) {
-    double P[3] = {gxm(g, i), gym(g, j), gzm(g, k)};
-    const double* n = &M.nor[3 * f];
-    double dot = n[0] * (pos[0] - P[0]) + n[1] * (pos[1] - P[1]) + n[2] * (pos[2] - P[2]);
-    double sgn = signbit(dot) ? -1.0 : 1.0;
-    double sg = dist * (-sgn);
-    size_t c = widx(g, i, j, k);
-    sdf[c] = (R)sg;
-    double eps = 1.0 / g.dx1, v;  // sdf_to_VOF genSDF.f90:237-255
-    if (sg <= -eps) v = 0.0;
-    else if (sg >= eps) v = 1.0;
-    else v = 0.5 * (1.0 + sg * g.dx1 + (1.0 / pi) * det_sin(pi * sg * g.dx1));
-    vofp[c] = (R)v;
+  } else {
+    const double dist = dst[id];
+    if constexpr (MODE == 1) {
+      if (key[s] == (unsigned long long)__double_as_longlong(dist)) atomicMin(&face[s], f);
+    } else if (face[s] == f) {
+      double P[3] = {gxm(g, i), gym(g, j), gzm(g, k)};
+      const double* n = &M.nor[3 * f];
+      double dot = n[0] * (pos[0] - P[0]) + n[1] * (pos[1] - P[1]) + n[2] * (pos[2] - P[2]);
+      double sgn = signbit(dot) ? -1.0 : 1.0;
+      double sg = dist * (-sgn);
+      size_t c = widx(g, i, j, k);
+      sdf[c] = (R)sg;
+      double eps = 1.0 / g.dx1, v;  // sdf_to_VOF genSDF.f90:237-255
+      if (sg <= -eps) v = 0.0;
+      else if (sg >= eps) v = 1.0;
+      else v = 0.5 * (1.0 + sg * g.dx1 + (1.0 / pi) * det_sin(pi * sg * g.dx1));
+      vofp[c] = (R)v;
+    }
   }
 }
 
@@ -1223,13 +1245,16 @@ static int ibm_tag_t(melt_ctx* ctx) {  // tagCells.f90:4-27 (tagType 1) + interp
                      ctx->d_win, fld<R>(ctx, MELT_SDF), et, ctx->d_tkey, ctx->d_tface, ctx->twin_cells);
   // the fused substep places the forcing window from the same extent (the
   // faces do not move between tagging and forcing)
-  hipLaunchKernelGGL(k_window_final, dim3(1), dim3(1), 0, ctx->stream, ctx->d_win, ef, et, ctx->force_window_from_tag ? 3 : 2,
-                     ctx->d_err);
+  const int which = ctx->force_window_from_tag ? 3 : 2;
   MeshArgs M = mesh_args(ctx);
   unsigned blocks = nb((size_t)ctx->nf * 125, 256);
-  for (int mode = 0; mode < 3; ++mode)
-    hipLaunchKernelGGL(k_tag_pass<R>, dim3(blocks), dim3(256), 0, ctx->stream, g, M, ctx->d_win, et, ctx->d_tkey, ctx->d_tface, ctx->d_tdist,
-                       fld<R>(ctx, MELT_SDF), fld<R>(ctx, MELT_VOFP), mode, ctx->pi, ctx->d_err);
+#define TAG_PASS(MODE)                                                                                                                 \
+  hipLaunchKernelGGL((k_tag_pass<MODE, R>), dim3(blocks), dim3(256), 0, ctx->stream, g, M, ctx->d_win, ef, et, which, ctx->d_tkey,      \
+                     ctx->d_tface, ctx->d_tdist, fld<R>(ctx, MELT_SDF), fld<R>(ctx, MELT_VOFP), ctx->pi, ctx->d_err)
+  TAG_PASS(0);
+  TAG_PASS(1);
+  TAG_PASS(2);
+#undef TAG_PASS
   MELT_HIP(hipGetLastError());
   return 0;
 }
