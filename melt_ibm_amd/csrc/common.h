@@ -46,8 +46,8 @@ struct melt_window {
 
 // Per-face probe results of the MLS gradient / interpolation evaluations.
 enum {
-  PRB_QO = 0, PRB_QI, PRB_P, PRB_GP, PRB_GU = PRB_GP + 3, PRB_GV = PRB_GU + 3, PRB_GW = PRB_GV + 3,
-  PRB_GT0 = PRB_GW + 3, PRB_GT1 = PRB_GT0 + 3,  // temperature gradients behind QO / QI
+  PRB_P = 0, PRB_GP, PRB_GU = PRB_GP + 3, PRB_GV = PRB_GU + 3, PRB_GW = PRB_GV + 3,
+  PRB_GT0 = PRB_GW + 3, PRB_GT1 = PRB_GT0 + 3,  // temperature gradients on the fluid and solid sides
   PRB_N = PRB_GT1 + 3
 };
 

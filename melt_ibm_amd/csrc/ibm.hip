@@ -992,10 +992,19 @@ __device__ inline double* probe_out(double* out, int f, int kind, int d) {
 // + d], and k_probes_apply later sums them against the field in the same
 // order; without it the lanes sum against the field directly.  Either way
 // the values round as in the single-thread formulation.
+// With ppw (and coef) the blocks from gradient block count nblk on store the pressure
+// interpolation's 27 shape functions of one face per thread at ppw[q nf + f].
 template <typename R>
 __global__ __launch_bounds__(256) void k_probes_grad(Grid g, ProbeArgs<R> P, double* __restrict__ out, int* __restrict__ pind, int klo,
-                                                     int nkinds, double* __restrict__ coef, int* err) {
+                                                     int nkinds, double* __restrict__ coef, double* __restrict__ ppw, int nblk, int* err) {
   __shared__ double shA[64][16];
+  if ((int)blockIdx.x >= nblk) {
+    const int f = ((int)blockIdx.x - nblk) * 256 + (int)threadIdx.x;
+    if (f >= P.nf || P.gf[f]) return;
+    int icent, jcent, kw;
+    if (pressure_phi(g, P, f, icent, jcent, kw, [&](int q, double phi) { ppw[(size_t)q * P.nf + f] = phi; })) raise_error(err, MELT_ERR_SINGULAR_MLS);
+    return;
+  }
   const int id = blockIdx.x * blockDim.x + threadIdx.x;
   const int item = id >> 2, lane = id & 3, slot = threadIdx.x >> 2;
   const int nitem = P.nf * nkinds;   // with coef: items over the coefficient slots
@@ -1022,16 +1031,31 @@ __global__ __launch_bounds__(256) void k_probes_grad(Grid g, ProbeArgs<R> P, dou
   if (!coef) *probe_out(out, f, kind, lane - 1) = gd;
 }
 
-// The field part of the gradient probes of the fused substep: one thread per
-// (item, component) sums the stored shape-function derivatives against the
-// field values in the reference's point order (and records the heat-flux
-// probes' cell indices, as the probes do).
+// The field part of the probes of the fused substep: one thread per (item,
+// component) sums the stored shape-function derivatives against the field
+// values in the reference's point order (and records the heat-flux probes'
+// cell indices, as the probes do); with ppw one more thread per face sums the
+// stored shape functions of the pressure probe, whose moment matrix and
+// inverse (11 us of latency) thereby leave the path to the forcing.
 template <typename R>
-__global__ __launch_bounds__(256) void k_probes_apply(Grid g, ProbeArgs<R> P, const double* __restrict__ coef, double* __restrict__ out,
-                                                      int* __restrict__ pind, int klo, int nkinds, int ncoef) {
+__global__ __launch_bounds__(256) void k_probes_apply(Grid g, ProbeArgs<R> P, const double* __restrict__ coef, const double* __restrict__ ppw,
+                                                      double* __restrict__ out, int* __restrict__ pind, int klo, int nkinds, int ncoef) {
   const int nitem = P.nf * nkinds;
   const int id = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (id >= 3 * nitem) return;
+  if (id >= 3 * nitem) {
+    const int f = id - 3 * nitem;
+    if (!ppw || f >= P.nf || P.gf[f]) return;
+    double pos[3];
+    probe_pos(P, f, 2, pos);
+    const int icent = (int)floor(pos[0] * g.dx1) + 1, jcent = (int)floor(pos[1] * g.dx2) + 1;
+    const int kw = pmod((int)floor(pos[2] * g.dx3), g.n3) + 1;
+    double pp = 0.0;
+#pragma unroll
+    for (int q = 0; q < 27; ++q)
+      pp = pp + P.pr[widx(g, icent - 1 + q % 3, jcent - 1 + (q / 3) % 3, kw - 1 + q / 9)] * ppw[(size_t)q * P.nf + f];
+    out[(size_t)PRB_N * f + PRB_P] = pp;
+    return;
+  }
   const int item = id / 3, d = id - 3 * item;
   const int f = item % P.nf, kind = grad_kind(klo + item / P.nf);
   if (P.gf[f]) return;
@@ -1056,36 +1080,33 @@ __global__ __launch_bounds__(256) void k_probes_apply(Grid g, ProbeArgs<R> P, co
   *probe_out(out, f, kind, d) = s;
 }
 
-// Pressure interpolation probe (kind 2) and the heat-flux dot products of
-// kinds 0/1 (q = n . grad T / Pe), one thread per face.
+// Shape functions of the pressure interpolation probe (kind 2, wght_press) of
+// face f: sink(q, phi) in the reference's point order.
+template <typename R, class Sink>
+__device__ __forceinline__ int pressure_phi(const Grid& g, const ProbeArgs<R>& P, int f, int& icent, int& jcent, int& kw, Sink sink) {
+  double pos[3];
+  probe_pos(P, f, 2, pos);
+  icent = (int)floor(pos[0] * g.dx1) + 1; jcent = (int)floor(pos[1] * g.dx2) + 1;
+  const int k1 = (int)floor(pos[2] * g.dx3) + 1;
+  kw = pmod(k1 - 1, g.n3) + 1;
+  const int cc[3] = {1, 1, 1};
+  return mls_phi(g, pos, icent - 1, jcent - 1, k1 - 1, cc, sink);
+}
+
+// Pressure interpolation probe (kind 2), one thread per face.
 template <typename R>
 __global__ __launch_bounds__(64) void k_probes_point(Grid g, ProbeArgs<R> P, double* __restrict__ out, int* err) {
   int f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= P.nf || P.gf[f]) return;
-  double* o = &out[(size_t)PRB_N * f];
-  if (P.heat) {
-    const double* nor = &P.nor[3 * f];
-    for (int kind = 0; kind < 2; ++kind) {
-      const double* gr = &o[kind == 0 ? PRB_GT0 : PRB_GT1];
-      double q = nor[0] * gr[0] + nor[1] * gr[1] + nor[2] * gr[2];
-      o[kind == 0 ? PRB_QO : PRB_QI] = q / P.pec;
-    }
-  }
-  if (!P.loads) return;
-  double pos[3];
-  probe_pos(P, f, 2, pos);
-  int icent = (int)floor(pos[0] * g.dx1) + 1, jcent = (int)floor(pos[1] * g.dx2) + 1;
-  int k1 = (int)floor(pos[2] * g.dx3) + 1;
-  int kw = pmod(k1 - 1, g.n3) + 1;
-  const int cc[3] = {1, 1, 1};
   double pp = 0.0;
   const R* pr = P.pr;
-  int info = mls_phi(g, pos, icent - 1, jcent - 1, k1 - 1, cc, [&](int q, double phi) {
+  int icent, jcent, kw;
+  int info = pressure_phi(g, P, f, icent, jcent, kw, [&](int q, double phi) {
     int kk = q / 9, j = jcent - 1 + (q / 3) % 3, i = icent - 1 + q % 3;
     pp = pp + pr[widx(g, i, j, kw - 1 + kk)] * phi;
   });
   if (info) { raise_error(err, MELT_ERR_SINGULAR_MLS); return; }
-  o[PRB_P] = pp;
+  out[(size_t)PRB_N * f + PRB_P] = pp;
 }
 
 inline unsigned nb(size_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -1368,18 +1389,25 @@ static ProbeArgs<R> probe_args(melt_ctx* ctx) {
 template <typename R>
 static int probe_coef_slots(const ProbeArgs<R>& P) { return P.heat && P.loads ? 5 : P.heat ? 2 : P.loads ? 4 : 0; }
 
-// The geometry part of the gradient probes (shape-function derivatives into
-// d_pcoef): reads only the faces and the grid, so the fused substep runs it
-// beside the explicit pass.
+// Where the pressure probe's shape functions sit in d_pcoef (27 x 18 doubles per
+// face): behind the gradient slots (27 x 15 at most).
+template <typename R>
+static double* probe_ppw(melt_ctx* ctx, const ProbeArgs<R>& P) {
+  return P.loads ? ctx->d_pcoef + (size_t)27 * 3 * probe_coef_slots(P) * ctx->nf : nullptr;
+}
+
+// The geometry part of the probes (shape-function derivatives and the pressure
+// probe's shape functions into d_pcoef): reads only the faces and the grid, so
+// the fused substep runs it beside the explicit pass.
 template <typename R>
 static int ibm_probe_coefs_t(melt_ctx* ctx) {
   ProbeArgs<R> P = probe_args<R>(ctx);
   int klo = P.heat ? 0 : 2, khi = P.loads ? 6 : 2;
   const int ncoef = probe_coef_slots(P);
   if (khi > klo) {
-    size_t threads = (size_t)ctx->nf * ncoef * 4;
-    hipLaunchKernelGGL(k_probes_grad<R>, dim3(nb(threads, 256)), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, ctx->d_pind,
-                       klo, ncoef, ctx->d_pcoef, ctx->d_err);
+    const int ngrad = (int)nb((size_t)ctx->nf * ncoef * 4, 256), npr = P.loads ? (int)nb(ctx->nf, 256) : 0;
+    hipLaunchKernelGGL(k_probes_grad<R>, dim3(ngrad + npr), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, ctx->d_pind,
+                       klo, ncoef, ctx->d_pcoef, probe_ppw(ctx, P), ngrad, ctx->d_err);
   }
   MELT_HIP(hipGetLastError());
   return 0;
@@ -1391,16 +1419,16 @@ static int ibm_probes_t(melt_ctx* ctx, int* pind_out, bool coefs_ready) {
   int klo = P.heat ? 0 : 2, khi = P.loads ? 6 : 2;
   int* pind = pind_out ? pind_out : ctx->d_pind;
   if (khi > klo && coefs_ready) {
-    size_t threads = (size_t)ctx->nf * (khi - klo) * 3;
-    hipLaunchKernelGGL(k_probes_apply<R>, dim3(nb(threads, 256)), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_pcoef, ctx->d_probe,
-                       pind, klo, khi - klo, probe_coef_slots(P));
+    size_t threads = (size_t)ctx->nf * (khi - klo) * 3 + (P.loads ? ctx->nf : 0);
+    hipLaunchKernelGGL(k_probes_apply<R>, dim3(nb(threads, 256)), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_pcoef, probe_ppw(ctx, P),
+                       ctx->d_probe, pind, klo, khi - klo, probe_coef_slots(P));
   } else if (khi > klo) {
-    size_t threads = (size_t)ctx->nf * (khi - klo) * 4;
-    hipLaunchKernelGGL(k_probes_grad<R>, dim3(nb(threads, 256)), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, pind, klo,
-                       khi - klo, nullptr, ctx->d_err);
+    const int ngrad = (int)nb((size_t)ctx->nf * (khi - klo) * 4, 256);
+    hipLaunchKernelGGL(k_probes_grad<R>, dim3(ngrad), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, pind, klo, khi - klo, nullptr,
+                       nullptr, ngrad, ctx->d_err);
+    if (P.loads)
+      hipLaunchKernelGGL(k_probes_point<R>, dim3(nb(ctx->nf, 64)), dim3(64), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, ctx->d_err);
   }
-  if (P.heat || P.loads)
-    hipLaunchKernelGGL(k_probes_point<R>, dim3(nb(ctx->nf, 64)), dim3(64), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, ctx->d_err);
   MELT_HIP(hipGetLastError());
   return 0;
 }

@@ -105,16 +105,25 @@ __device__ void rigid_finish(const double* s, double dens_ratio, double com[3], 
 enum { FIN_NONE = 0, FIN_FINAL = 4 };
 
 // The fixed-pattern sum of the nb <= 64 partials of quantity q into sm[q]
-// (one wave per quantity, butterfly over the lanes), for q < ns; ends with a
+// (one wave per quantity, butterfly over the lanes), for q < ns <= NS; ends with a
 // block barrier.
-__device__ void reduce_partials(const double* __restrict__ part, int nb, int ns, double* sm) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = RB / 64;
-  for (int q = wv; q < ns; q += nw) {
-    double v = lane < nb ? part[q * nb + lane] : 0.0;
+template <int NS>
+__device__ void reduce_partials(const double* __restrict__ part, int nb, double* sm, int ns = NS) {
+  constexpr int NW = RB / 64, NQ = (NS + NW - 1) / NW;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  double v[NQ];   // the wave's quantities, loaded together
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = v + __shfl_xor(v, off, 64);
-    if (lane == 0) sm[q] = v;
+  for (int i = 0; i < NQ; ++i) {
+    const int q = wv + i * NW;
+    v[i] = q < ns && lane < nb ? part[q * nb + lane] : 0.0;
   }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) v[i] = v[i] + __shfl_xor(v[i], off, 64);
+#pragma unroll
+  for (int i = 0; i < NQ; ++i)
+    if (lane == 0 && wv + i * NW < NS) sm[wv + i * NW] = v[i];
   __syncthreads();
 }
 
@@ -135,7 +144,7 @@ __device__ void loads_finish(melt_body* b, const double* s) {
 __global__ __launch_bounds__(RB) void k_sum_partials(const double* __restrict__ part, int nb, int ns, double* __restrict__ out, int fin,
                                                      melt_body* body, double dens_ratio, int* err) {
   __shared__ double sm[16];
-  reduce_partials(part, nb, ns, sm);
+  reduce_partials<12>(part, nb, sm, ns);
   if ((int)threadIdx.x < ns) out[threadIdx.x] = sm[threadIdx.x];
   if (threadIdx.x != 0 || fin != FIN_FINAL) return;
   melt_body* b = body;
@@ -185,17 +194,26 @@ __global__ void k_body_rigid(melt_body* b, const double* __restrict__ s, double 
 // small-volume abort (particle.f90:218-224)
 
 // ---------------------------------------------------------- heat / Stefan
-// With pind2, also commits the heat-flux probes' cell indices that the fused
-// substep staged there (the spreading had still read the old ones).
-__global__ __launch_bounds__(256) void k_face_post(LagArgs A, const double* __restrict__ probe, const melt_body* __restrict__ b,
-                                                   double* __restrict__ rxp, double* __restrict__ rxt, double ren, int heat, int loads,
-                                                   int* __restrict__ pind, const int* __restrict__ pind2) {
-  int f = blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= A.nf || A.gf[f]) return;
+// Heat flux through face f on the fluid (side 0) or solid (1) side, n . grad T /
+// Pe (mls_heatFlux.f90:33-60), from the probes' temperature gradients.
+__device__ __forceinline__ double face_flux(const LagArgs& A, const double* __restrict__ probe, int f, int side, double pec) {
+  const double* nor = &A.L[MELT_L_TRI_NOR][3 * f];
+  const double* gr = &probe[(size_t)PRB_N * f + (side ? PRB_GT1 : PRB_GT0)];
+  const double q = nor[0] * gr[0] + nor[1] * gr[1] + nor[2] * gr[2];
+  return q / pec;
+}
+
+// Face results of the probes.  With pind2, also commits the heat-flux probes'
+// cell indices that the fused substep staged there (the spreading had still
+// read the old ones).
+__device__ __forceinline__ void face_post(const LagArgs& A, int f, const double* __restrict__ probe, const melt_body* __restrict__ b,
+                                          double* __restrict__ rxp, double* __restrict__ rxt, double ren, double pec, int heat, int loads,
+                                          int* __restrict__ pind, const int* __restrict__ pind2) {
+  if (A.gf[f]) return;
   const double* pr = &probe[(size_t)PRB_N * f];
   if (pind2)
     for (int q = 0; q < 6; ++q) pind[6 * f + q] = pind2[6 * f + q];
-  if (heat) { A.L[MELT_L_QW_O][f] = pr[PRB_QO]; A.L[MELT_L_QW_I][f] = pr[PRB_QI]; }
+  if (heat) { A.L[MELT_L_QW_O][f] = face_flux(A, probe, f, 0, pec); A.L[MELT_L_QW_I][f] = face_flux(A, probe, f, 1, pec); }
   if (!loads) return;
   const double* nor = &A.L[MELT_L_TRI_NOR][3 * f];
   const double* bar = &A.L[MELT_L_TRI_BAR][3 * f];
@@ -224,20 +242,31 @@ __global__ __launch_bounds__(256) void k_face_post(LagArgs A, const double* __re
   }
 }
 
-__global__ __launch_bounds__(256) void k_vert_heat_stefan(LagArgs A, const melt_body* __restrict__ b, double cp_over_L, double dt, double ga,
-                                                          double ro, int stefan) {
-  int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= A.nv) return;
+// Vertex fluxes (mls_heatFlux.f90:302-319) and the Stefan update of the vertex
+// (stefanCondition.f90).  The faces of a vertex are taken four at a time, their
+// loads in flight together; the sum runs in face order.
+__device__ __forceinline__ void vert_stefan(const LagArgs& A, int v, const double* __restrict__ probe, double pec, double cp_over_L, double dt,
+                                            double ga, double ro) {
   double qo = 0.0, qi = 0.0, av = A.L[MELT_L_AVERT][v];
-  for (int p = A.v2f_ptr[v]; p < A.v2f_ptr[v + 1]; ++p) {
-    int f = A.v2f[p];
-    double w = A.L[MELT_L_SUR][f] / 3.0 / av;
-    qo = qo + A.L[MELT_L_QW_O][f] * w;
-    qi = qi + A.L[MELT_L_QW_I][f] * w;
+  const int p1 = A.v2f_ptr[v + 1];
+  for (int p = A.v2f_ptr[v]; p < p1; p += 4) {
+    double w[4], fo[4], fi[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int f = A.v2f[min(p + q, p1 - 1)];
+      w[q] = A.L[MELT_L_SUR][f] / 3.0 / av;
+      fo[q] = face_flux(A, probe, f, 0, pec);
+      fi[q] = face_flux(A, probe, f, 1, pec);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (p + q < p1) {
+        qo = qo + fo[q] * w[q];
+        qi = qi + fi[q] * w[q];
+      }
   }
   A.L[MELT_L_QW_OVERT][v] = qo;
   A.L[MELT_L_QW_IVERT][v] = qi;
-  if (!stefan) return;
   double* vm = &A.L[MELT_L_VMELT][3 * v];
   double* vm1 = &A.L[MELT_L_VMELT_M1][3 * v];
   for (int d = 0; d < 3; ++d) vm1[d] = vm[d];
@@ -246,6 +275,18 @@ __global__ __launch_bounds__(256) void k_vert_heat_stefan(LagArgs A, const melt_
   for (int d = 0; d < 3; ++d) vm[d] = cp_over_L * (qi - qo) * n[d];
   double* x = &A.L[MELT_L_XYZV][3 * v];
   for (int d = 0; d < 3; ++d) x[d] = x[d] + dt * (ga * vm[d] + ro * vm1[d]);
+}
+
+// Faces and, with heat, vertices in one launch: a vertex takes its faces'
+// fluxes from the probes itself (the same values), and moving it touches
+// nothing a face reads here (two launches 4.4 + 7.0 us at 1280 faces).
+__global__ __launch_bounds__(256) void k_face_post_stefan(LagArgs A, const double* __restrict__ probe, const melt_body* __restrict__ b,
+                                                          double* __restrict__ rxp, double* __restrict__ rxt, double ren, double pec, int heat,
+                                                          int loads, int* __restrict__ pind, const int* __restrict__ pind2, double cp_over_L,
+                                                          double dt, double ga, double ro) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < A.nf) face_post(A, t, probe, b, rxp, rxt, ren, pec, heat, loads, pind, pind2);
+  else if (heat && t - A.nf < A.nv) vert_stefan(A, t - A.nf, probe, pec, cp_over_L, dt, ga, ro);
 }
 
 // ---------------------------------------------------------- geometry
@@ -311,8 +352,9 @@ __global__ void k_clear_rm(melt_body* b) { b->rm_flag = 0; }
 // calculate_area (triaux.f90:82-119), calc_centroids_from_vert (:308-323) and
 // update_tri_normal of every live face in one pass (the same expressions as
 // k_face_area and k_face_centroid_normal); thread 0 also clears the remesh
-// flag that k_edge_len then sets.
-__global__ __launch_bounds__(256) void k_face_geom(LagArgs A, const double* __restrict__ x, melt_body* b) {
+// flag that k_edge_len then sets.  With vel, the face velocities too (as
+// k_face_vel, whose centroids are the same).
+__global__ __launch_bounds__(256) void k_face_geom(LagArgs A, const double* __restrict__ x, melt_body* b, int vel) {
   int f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f == 0) b->rm_flag = 0;
   if (f >= A.nf || A.gf[f]) return;
@@ -334,6 +376,11 @@ __global__ __launch_bounds__(256) void k_face_geom(LagArgs A, const double* __re
   n[2] = e1[0] * e2[1] - e1[1] * e2[0];
   double s = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
   for (int d = 0; d < 3; ++d) A.L[MELT_L_TRI_NOR][3 * f + d] = n[d] / s;
+  if (vel) {
+    double om[3];
+    dcross(om, b->omega_c, &A.L[MELT_L_DXYZ_S][3 * f]);
+    for (int d = 0; d < 3; ++d) A.L[MELT_L_VEL_TRI][3 * f + d] = b->vel_cm[d] + om[d];
+  }
 }
 
 __global__ __launch_bounds__(256) void k_skewness(LagArgs A) {  // calculate_skewness triaux.f90:325-358
@@ -381,11 +428,21 @@ __device__ inline void face_skewness(const LagArgs& A, int f, const double el[3]
 // area and normal of vertex v from its faces
 __device__ void vert_post_geom(const LagArgs& A, int v) {
   double av = 0.0, n[3] = {0.0, 0.0, 0.0};
-  for (int p = A.v2f_ptr[v]; p < A.v2f_ptr[v + 1]; ++p) {
-    int f = A.v2f[p];
-    double s = A.L[MELT_L_SUR][f];
-    av = av + s / 3.0;
-    for (int d = 0; d < 3; ++d) n[d] = n[d] + s * A.L[MELT_L_TRI_NOR][3 * f + d];
+  const int p1 = A.v2f_ptr[v + 1];
+  for (int p = A.v2f_ptr[v]; p < p1; p += 4) {   // four faces' loads in flight, summed in order
+    double s[4], m[4][3];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int f = A.v2f[min(p + q, p1 - 1)];
+      s[q] = A.L[MELT_L_SUR][f];
+      for (int d = 0; d < 3; ++d) m[q][d] = A.L[MELT_L_TRI_NOR][3 * f + d];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (p + q < p1) {
+        av = av + s[q] / 3.0;
+        for (int d = 0; d < 3; ++d) n[d] = n[d] + s[q] * m[q][d];
+      }
   }
   A.L[MELT_L_AVERT][v] = av;
   if (!A.gv[v]) {
@@ -584,7 +641,7 @@ __global__ __launch_bounds__(RB) void k_sum_motion(const double* __restrict__ pa
                                                    double zlen, double* __restrict__ aa_out, double* __restrict__ com_out, int* err) {
   constexpr int QV = L ? 12 : 0, QG = QV + (V ? 1 : 0), NS = QG + (L ? 10 : 0);
   __shared__ double sm[NS];
-  reduce_partials(part, nb, NS, sm);
+  reduce_partials<NS>(part, nb, sm);
   if ((int)threadIdx.x < NS) out[threadIdx.x] = sm[threadIdx.x];
   if (threadIdx.x != 0) return;
   melt_body* b = body;
@@ -664,10 +721,10 @@ LagArgs lag_args(melt_ctx* ctx) {
 }
 
 // geometry refresh of particle.f90:163-193
-int refresh_geometry(melt_ctx* ctx, LagArgs& A) {
+int refresh_geometry(melt_ctx* ctx, LagArgs& A, int vel = 0) {
   const double* x = ctx->d_lag[MELT_L_XYZV];
   hipStream_t s = ctx->stream;
-  hipLaunchKernelGGL(k_face_geom, dim3(nb(ctx->nf, 256)), dim3(256), 0, s, A, x, ctx->d_body);
+  hipLaunchKernelGGL(k_face_geom, dim3(nb(ctx->nf, 256)), dim3(256), 0, s, A, x, ctx->d_body, vel);
   // work that needs only the refreshed faces (the fused substep's next
   // tagging) forks here; the rest of the refresh does not touch what it reads
   if (const std::function<int()>* hook = ctx->after_faces) {
@@ -740,11 +797,10 @@ int lagr_after_force(melt_ctx* ctx, bool commit_pind) {
   hipStream_t s = ctx->stream;
   int heat = ctx->cfg.imelt == 1, loads = ctx->cfg.imlsstr == 1;
   if (heat || loads)
-    hipLaunchKernelGGL(k_face_post, dim3(nb(ctx->nf, 256)), dim3(256), 0, s, A, ctx->d_probe, ctx->d_body, ctx->d_rxp, ctx->d_rxt, ctx->cfg.ren,
-                       heat, loads, ctx->d_pind, commit_pind && heat ? ctx->d_pind2 : nullptr);
+    hipLaunchKernelGGL(k_face_post_stefan, dim3(nb((size_t)ctx->nf + (heat ? ctx->nv : 0), 256)), dim3(256), 0, s, A, ctx->d_probe, ctx->d_body,
+                       ctx->d_rxp, ctx->d_rxt, ctx->cfg.ren, ctx->cfg.ren * ctx->cfg.prandtl, heat, loads, ctx->d_pind,
+                       commit_pind && heat ? ctx->d_pind2 : nullptr, ctx->cfg.cpliquid / ctx->cfg.latheat, ctx->dt, ctx->ga, ctx->ro);
   if (heat) {
-    hipLaunchKernelGGL(k_vert_heat_stefan, dim3(nb(ctx->nv, 256)), dim3(256), 0, s, A, ctx->d_body, ctx->cfg.cpliquid / ctx->cfg.latheat, ctx->dt,
-                       ctx->ga, ctx->ro, 1);
     // the volume after melting is the one the remeshing restores (particle.f90:86-90)
     if (ctx->cfg.iremesh == 1)
       MELT_HIP(hipMemcpyAsync(ctx->d_xyz_melt, ctx->d_lag[MELT_L_XYZV], sizeof(double) * 3 * ctx->nv, hipMemcpyDeviceToDevice, s));
@@ -757,10 +813,10 @@ int lagr_after_force(melt_ctx* ctx, bool commit_pind) {
   else if (heat) motion_sums<false, true>(ctx, A);
   if (loads) {
     hipLaunchKernelGGL(k_rel_update, dim3(nb((size_t)ctx->nv + ctx->nf, 256)), dim3(256), 0, s, A, ctx->d_body, ctx->d_red + 48, ctx->d_red + 32);
-    hipLaunchKernelGGL(k_face_vel, dim3(nb(ctx->nf, 256)), dim3(256), 0, s, A, ctx->d_body);
+    if (ctx->cfg.iremesh == 1) hipLaunchKernelGGL(k_face_vel, dim3(nb(ctx->nf, 256)), dim3(256), 0, s, A, ctx->d_body);
   }
   MELT_HIP(hipGetLastError());
-  if (ctx->cfg.iremesh != 1) return refresh_geometry(ctx, A);
+  if (ctx->cfg.iremesh != 1) return refresh_geometry(ctx, A, loads);
   // calculate_eLengths (particle.f90:128): the short-edge flag goes to the host
   hipLaunchKernelGGL(k_clear_rm, dim3(1), dim3(1), 0, s, ctx->d_body);
   hipLaunchKernelGGL(k_edge_len, dim3(nb(ctx->ne, 256)), dim3(256), 0, s, A, ctx->d_lag[MELT_L_XYZV], ctx->d_body, ctx->h_body.e_thresh);
