@@ -640,7 +640,7 @@ static int particle_impl(melt_ctx* ctx, int defer) {
   if ((rc = ibm_weights(ctx))) return rc;
   if ((rc = ibm_force_scatter(ctx))) return rc;
   if ((rc = ibm_probes(ctx))) return rc;      // heat flux and loads read the pre-force fields
-  if ((rc = ibm_force_drain(ctx, 1))) return rc;
+  if ((rc = ibm_force_drain(ctx, 1)) || (rc = ibm_force_mean(ctx))) return rc;
   if (!defer && (rc = ibm_sub_mean(ctx))) return rc;
   return lagr_after_force(ctx);
 }
@@ -851,15 +851,23 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
   // probe geometry stage: only the next substep's probes read its output, and
   // they run on the side stream after it; the call's last substep joins it
   const bool coef_after_join = tag_next && coef_next && probes && !one_stream(ctx);
+  // within a tschem call the next substep's cell indices and shape functions
+  // (they read only the refreshed faces; this substep's spreading is done with
+  // them) are formed here too, off the path from its line solves to its forcing
+  // (9 us at 1280 faces).  Not across calls: the arrays a caller sees are those
+  // the last substep used.
+  const bool weights_next = tag_next && moving && !one_stream(ctx);
   auto queue_next = [&]() -> int {
     int r = 0;
     if (tag_next && moving && !ctx->tag_ahead) r = tag_now();
+    if (!r && weights_next && !(r = ibm_weights(ctx, true))) ctx->weights_ahead = 1;
     if (!r && coef_next && probes && !coef_after_join) r = queue_coef();
     return r;
   };
   if (ibm) {
     timing_begin(ctx, SLOT_IBM, &e);
-    if ((rc = ibm_weights(ctx, true))) return rc;   // cell indices and shape functions
+    if (!ctx->weights_ahead && (rc = ibm_weights(ctx, true))) return rc;   // cell indices and shape functions
+    ctx->weights_ahead = 0;
     // the gradient probes read the same pre-force fields as the spreading and
     // write only their own outputs (their cell indices into d_pind2, since the
     // spreading still reads d_pind): side stream, alongside the spreading
@@ -867,7 +875,6 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
     rc = ibm_force_scatter(ctx);
     ctx->force_window_from_tag = 0;
     if (rc || (rc = side_join(ctx)) || (rc = ibm_force_drain(ctx, 1))) return rc;
-    timing_end(ctx, SLOT_IBM, e);
     // The Lagrangian update after the forcing (loads, heat flux, Stefan
     // melting, Newton-Euler motion, remeshing, geometry refresh) reads only
     // the probe results and the body arrays, which the pressure phase does
@@ -878,6 +885,9 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
     // the device needs it (queued first, they left the main stream idle for
     // 0.1-0.23 ms per substep while the host submitted them).
     if ((rc = side_fork(ctx))) return rc;
+    // the mean force: only the projection reads it
+    if ((rc = ibm_force_mean(ctx))) return rc;
+    timing_end(ctx, SLOT_IBM, e);
   }
   timing_end(ctx, SLOT_PH_MLS, e_ph);
 
@@ -952,6 +962,7 @@ static int tschem_launch(melt_ctx* ctx) {
     if (rc) {
       ctx->tag_ahead = 0;
       ctx->coef_ahead = 0;
+      ctx->weights_ahead = 0;
       if (ctx->graph_uses_ahead) graph_drop(ctx);
       return rc;
     }

@@ -182,6 +182,7 @@ struct melt_ctx {
   int force_window_from_tag = 0;  // fused substep: tagging also places the forcing window
   int tag_ahead = 0;              // the next substep's tagging is already queued (side stream)
   int coef_ahead = 0;             // and the geometry part of its gradient probes
+  int weights_ahead = 0;          // and its MLS cell indices and shape functions (within a tschem call only)
   int graph_uses_ahead = 0;       // the captured step's first substep reads coefficients queued before it
 
   // timing
@@ -511,6 +512,7 @@ int ibm_find_centroid_indices(melt_ctx* ctx);
 int ibm_weights(melt_ctx* ctx, bool find = false);   // find: form the cell indices too
 int ibm_force_scatter(melt_ctx* ctx);
 int ibm_force_drain(melt_ctx* ctx, int apply_now);
+int ibm_force_mean(melt_ctx* ctx);   // of the forces the last ibm_force_drain(ctx, 1) applied, into d_fmean
 int ibm_sub_mean(melt_ctx* ctx);
 int ibm_velforce(melt_ctx* ctx, int defer);
 int ibm_tempforce(melt_ctx* ctx);

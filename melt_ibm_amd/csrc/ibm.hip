@@ -1316,21 +1316,30 @@ static int ibm_force_scatter_t(melt_ctx* ctx) {
   return 0;
 }
 
+static unsigned drain_blocks(const melt_ctx* ctx) { return (unsigned)std::min<size_t>(512, nb(ctx->fwin_cells, 256)); }
+
+// The exact mean of the velocity forces into d_fmean, for the projection
+// (velforce.f90:21-51 with the uniform shift deferred), from the block sums of
+// ibm_force_drain (d_red[64..3136), which the Lagrangian update's sums leave alone).
+int ibm_force_mean(melt_ctx* ctx) {
+  hipLaunchKernelGGL(k_fmean_final, dim3(1), dim3(256), 0, ctx->stream, reinterpret_cast<unsigned long long*>(ctx->d_red + 64),
+                     (int)drain_blocks(ctx), (double)((long long)ctx->n1 * ctx->n2 * ctx->n3), ctx->d_fmean);
+  MELT_HIP(hipGetLastError());
+  return 0;
+}
+
 // Drain the accumulators.  apply_now = 1 (fused substep): forces go straight
-// into u, v, w, T and the exact mean of the velocity forces lands in d_fmean
-// for the projection (velforce.f90:21-51 with the uniform shift deferred);
-// 0: the folded for_* fields are written (per-routine API, mlsForce output).
+// into u, v, w, T, and the block sums of the velocity forces are left for
+// ibm_force_mean; 0: the folded for_* fields are written (per-routine API, mlsForce output).
 template <typename R>
 static int ibm_force_drain_t(melt_ctx* ctx, int apply_now) {
   Grid g = make_grid(ctx);
   Win3 ef{{ctx->fwin[0], ctx->fwin[1], ctx->fwin[2]}};
-  unsigned blocks = (unsigned)std::min<size_t>(512, nb(ctx->fwin_cells, 256));
+  const unsigned blocks = drain_blocks(ctx);
   unsigned long long* part = reinterpret_cast<unsigned long long*>(ctx->d_red + 64);
   if (apply_now) {
     hipLaunchKernelGGL(k_force_apply<R>, dim3(blocks), dim3(256), 0, ctx->stream, g, ctx->d_win, ef, ctx->d_acc, ctx->fwin_cells, fld<R>(ctx, MELT_VX),
                        fld<R>(ctx, MELT_VY), fld<R>(ctx, MELT_TEMP), fld<R>(ctx, MELT_VZ), 0, part);
-    hipLaunchKernelGGL(k_fmean_final, dim3(1), dim3(256), 0, ctx->stream, part, (int)blocks, (double)((long long)ctx->n1 * ctx->n2 * ctx->n3),
-                       ctx->d_fmean);
   } else {
     for (int id = MELT_FOR_XC; id <= MELT_FOR_TEMP; ++id)
       hipLaunchKernelGGL(k_fill<R>, dim3(1024), dim3(256), 0, ctx->stream, fld<R>(ctx, id), 0.0, ctx->nc);
