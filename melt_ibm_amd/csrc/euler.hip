@@ -584,6 +584,12 @@ __global__ __launch_bounds__(256) void k_explicit_xsolve(EulerArgs<R> A, RhsCoef
 template <int...>
 constexpr bool no_stencil_value = false;
 
+// LDS of one x-line of the z-march: four padded lines of rhs and two sets of
+// eight exchange rows.
+__host__ __device__ constexpr size_t zmarch_lds(int n1, size_t bytes) {
+  return sizeof(double) * 4 * (size_t)(n1 + 2 * FIR_KMAX) + bytes * 16 * (size_t)n1;
+}
+
 // Stencil values of one cell of the z-marching pass: the centre column at
 // k-1, k, k+1 rolls in registers, the rows j-1 and j+1 are loaded per plane,
 // and the x-neighbours are read from the plane's rows published in LDS.
@@ -668,22 +674,27 @@ __device__ __forceinline__ void zcell(const EulerArgs<R>& A, const RhsCoef<R>& c
 // coming from LDS rows (two sets, alternating per plane, so one barrier
 // separates writing a set from reading it).  Each plane then runs the x-line
 // filter like k_explicit_xsolve.  Every value and expression is the same as
-// there, so the results are identical.  Off: 32-bit (fields < 4 GiB) or
-// 64-bit byte offsets.
-template <typename R, typename Off>
-__global__ __launch_bounds__(512) void k_explicit_zmarch(EulerArgs<R> A, RhsCoef<R> cf, R* __restrict__ ru1, R* __restrict__ ru2,
+// there, so the results are identical.  Fields are addressed by 32-bit
+// byte offsets (n1 = n2 <= 512 and n3 <= 1024: at most 2 GiB).  With ROWS = 2 a block holds two rows j (blockDim.y);
+// they share nothing but the barriers.
+template <typename R, int ROWS>
+__global__ __launch_bounds__(ROWS == 2 ? 768 : 512) void k_explicit_zmarch(EulerArgs<R> A, RhsCoef<R> cf, R* __restrict__ ru1, R* __restrict__ ru2,
                                                          R* __restrict__ ru3, R* __restrict__ rut, R* __restrict__ r_u, R* __restrict__ r_v,
                                                          R* __restrict__ r_w, R* __restrict__ r_t, double sc_u, double sc_t, int D, Green gu,
                                                          Green gt) {
-  extern __shared__ double lds[];
+  extern __shared__ double lds_all[];
   constexpr int H = FIR_KMAX;
   enum { XU, XUJM, XV, XVJP, XWP, XT, XP, XO, NX };   // exchange rows of one set
   const Grid& g = A.g;
   const int M = g.n1, i = threadIdx.x, ldx = M + 2 * H;
+  using Off = unsigned;
+  const int jr = ROWS > 1 ? (int)threadIdx.y : 0;
+  double* lds = ROWS > 1 ? lds_all + (size_t)jr * (zmarch_lds(M, sizeof(R)) / sizeof(double)) : lds_all;
   R* xr = reinterpret_cast<R*>(lds + 4 * ldx);
   auto row = [&](int set, int r) { return xr + (set * NX + r) * M; };
   const unsigned b = xcd_block(blockIdx.x, gridDim.x);
-  const int j = (int)(b % (unsigned)g.n2), k0 = (int)(b / (unsigned)g.n2) * D;
+  const unsigned nj = (unsigned)g.n2 / ROWS;
+  const int j = (int)(b % nj) * ROWS + jr, k0 = (int)(b / nj) * D;
   const int jm = j == 0 ? g.n2 - 1 : j - 1, jp = j == g.n2 - 1 ? 0 : j + 1;
   const int im = i == 0 ? M - 1 : i - 1, ip = i == M - 1 ? 0 : i + 1;
   auto off = [&](int jj, int kk) { return ((Off)i + (Off)M * ((Off)jj + (Off)g.n2 * (Off)kk)) * (Off)sizeof(R); };
@@ -762,12 +773,12 @@ __global__ __launch_bounds__(512) void k_explicit_zmarch(EulerArgs<R> A, RhsCoef
 // threads' pairs published in LDS as in the one-cell form.  Same values and
 // expressions per cell, so the results are identical to it.  Block: n1 / 2
 // threads.
-template <typename Off>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_explicit_zmarch_pair(EulerArgs<float> A, RhsCoef<float> cf, float* __restrict__ ru1,
                                                               float* __restrict__ ru2, float* __restrict__ ru3, float* __restrict__ rut,
                                                               float* __restrict__ r_u, float* __restrict__ r_v, float* __restrict__ r_w,
                                                               float* __restrict__ r_t, double sc_u, double sc_t, int D, Green gu, Green gt) {
   using R = float;
+  using Off = unsigned;
   typedef float f2 __attribute__((ext_vector_type(2)));
   typedef double d2 __attribute__((ext_vector_type(2)));
   extern __shared__ double lds[];
@@ -1324,50 +1335,64 @@ int launch_explicit_xsolve(melt_ctx* ctx, double bxu, double bxt) {
   R* r4[4] = {static_cast<R*>(ctx->rhs4[RHS_U]), static_cast<R*>(ctx->rhs4[RHS_V]), static_cast<R*>(ctx->rhs4[RHS_W]),
               static_cast<R*>(ctx->rhs4[RHS_T])};
   // z-march (one x-line per block, D planes) unless line-tile shapes are asked for
-  const size_t zshm = sizeof(double) * 4 * (ctx->n1 + 2 * FIR_KMAX) + sizeof(R) * 16 * (size_t)ctx->n1;
-  // (with geometric face fractions, tagType 0, the line tiles read them)
-  if (fir && ctx->tune[TUNE_XF_W] == 0 && ctx->tune[TUNE_XF_NT] == 0 && ctx->n1 % 64 == 0 && ctx->n1 <= 512 && zshm <= ctx->lds_max &&
-      ctx->cfg.tagtype != 0) {
-    int D = ctx->tune[TUNE_XF_Z];
+  // (with geometric face fractions, tagType 0, the line tiles read them).  Lines
+  // of 64 cells take the tiles below: a march of single waves exposes every
+  // plane's latency (64^3 FP64 32 us at 8 planes, 18 at 2, tiles 17; FP32 22 and 13;
+  // 128^3 FP64 87 marching, 100 in tiles).
+  const size_t zshm = zmarch_lds(ctx->n1, sizeof(R));
+  const int zd = ctx->tune[TUNE_XF_Z];
+  if (fir && ctx->tune[TUNE_XF_W] == 0 && ctx->tune[TUNE_XF_NT] == 0 && ctx->n1 % 64 == 0 && ctx->n1 <= 512 && (ctx->n1 >= 128 || zd > 0) &&
+      zshm <= ctx->lds_max && ctx->cfg.tagtype != 0) {
+    // two cells per thread (8-byte accesses) for 4-byte values where the half
+    // line is whole waves of enough of them: 256^3 333 us against 341, 384^3 1115
+    // against 1547, but 128^3 49 against 48 and 192^3 (one and a half waves) 178
+    // against 152
+    const bool pair = sizeof(R) == 4 && ctx->tune[TUNE_XF_ONE] == 0 && ctx->n1 % 128 == 0 && ctx->n1 >= 256;
+    const size_t lines = (size_t)ctx->n2 * ctx->n3 * (pair ? ctx->n1 / 128 : ctx->n1 / 64);   // waves at one plane each
+    int D = zd;
     if (D <= 0 || ctx->n3 % D) {
+      // planes per block: as many as leave 8192 waves, about 2.7 rounds of what the
+      // chip holds (128^3 FP64, 8 / 4 / 2 planes: 97 / 87 / 86 us; 256^3: 645 / 657 /
+      // 673); the two-cell form 8 from twice the work of 256^3 on, else 4 (384^3 1114 /
+      // 1157, 256^3 336 / 333)
       D = 1;
-      // 8 planes per block measured best for one cell per thread (FP32 1-2%,
-      // FP64 level or better), 4 for the two-cell form (1%)
-      const bool pair = sizeof(R) == 4 && ctx->tune[TUNE_XF_ONE] == 0;
       for (int d : {8, 4, 2})
-        if (!(pair && d == 8) && ctx->n3 % d == 0) { D = d; break; }
+        if (ctx->n3 % d == 0 && lines / d >= (pair && d == 8 ? 32768 : 8192)) { D = d; break; }
+      if (D == 1 && ctx->n3 % 2 == 0) D = 2;
     }
-    const unsigned blocks = (unsigned)((size_t)ctx->n2 * (ctx->n3 / D));
     if constexpr (std::is_same_v<R, float>) {
-      if (ctx->tune[TUNE_XF_ONE] == 0) {   // two cells per thread, 8-byte accesses
-        if (ctx->nc * sizeof(R) < (size_t(1) << 32))
-          hipLaunchKernelGGL((k_explicit_zmarch_pair<unsigned>), dim3(blocks), dim3(ctx->n1 / 2), zshm, ctx->stream, A, cf,
-                             fld<R>(ctx, MELT_RU1), fld<R>(ctx, MELT_RU2), fld<R>(ctx, MELT_RU3), fld<R>(ctx, MELT_RUT), r4[0], r4[1],
-                             r4[2], r4[3], sc_u, sc_t, D, gu, gt);
-        else
-          hipLaunchKernelGGL((k_explicit_zmarch_pair<size_t>), dim3(blocks), dim3(ctx->n1 / 2), zshm, ctx->stream, A, cf,
-                             fld<R>(ctx, MELT_RU1), fld<R>(ctx, MELT_RU2), fld<R>(ctx, MELT_RU3), fld<R>(ctx, MELT_RUT), r4[0], r4[1],
-                             r4[2], r4[3], sc_u, sc_t, D, gu, gt);
+      if (pair) {
+        const unsigned blocks = (unsigned)((size_t)ctx->n2 * (ctx->n3 / D));
+        hipLaunchKernelGGL(k_explicit_zmarch_pair, dim3(blocks), dim3(ctx->n1 / 2), zshm, ctx->stream, A, cf, fld<R>(ctx, MELT_RU1),
+                           fld<R>(ctx, MELT_RU2), fld<R>(ctx, MELT_RU3), fld<R>(ctx, MELT_RUT), r4[0], r4[1], r4[2], r4[3], sc_u, sc_t, D, gu,
+                           gt);
         MELT_HIP(hipGetLastError());
         return 0;
       }
     }
-    if (ctx->nc * sizeof(R) < (size_t(1) << 32))
-      hipLaunchKernelGGL((k_explicit_zmarch<R, unsigned>), dim3(blocks), dim3(ctx->n1), zshm, ctx->stream, A, cf, fld<R>(ctx, MELT_RU1),
-                         fld<R>(ctx, MELT_RU2), fld<R>(ctx, MELT_RU3), fld<R>(ctx, MELT_RUT), r4[0], r4[1], r4[2], r4[3], sc_u, sc_t, D, gu, gt);
-    else
-      hipLaunchKernelGGL((k_explicit_zmarch<R, size_t>), dim3(blocks), dim3(ctx->n1), zshm, ctx->stream, A, cf, fld<R>(ctx, MELT_RU1),
-                         fld<R>(ctx, MELT_RU2), fld<R>(ctx, MELT_RU3), fld<R>(ctx, MELT_RUT), r4[0], r4[1], r4[2], r4[3], sc_u, sc_t, D, gu, gt);
+    // A CU takes three waves of this kernel per SIMD, and a block only where every
+    // SIMD has room for its share rounded up: of six-wave blocks (384 cells) one,
+    // half the waves.  Two rows per block make twelve waves, three per SIMD
+    // (384^3 FP64 3197 -> 2637 us; 9.5 GB, 2000 us at the rate of a copy).
+    const int rows = (ctx->n1 / 64) % 4 == 2 && ctx->n1 > 256 && ctx->n2 % 2 == 0 && 2 * zshm <= ctx->lds_max ? 2 : 1;
+    const dim3 grid((unsigned)((size_t)(ctx->n2 / rows) * (ctx->n3 / D))), block(ctx->n1, rows);
+#define ZM_LAUNCH(ROWS)                                                                                                                    \
+  hipLaunchKernelGGL((k_explicit_zmarch<R, ROWS>), grid, block, rows * zshm, ctx->stream, A, cf, fld<R>(ctx, MELT_RU1),                     \
+                     fld<R>(ctx, MELT_RU2), fld<R>(ctx, MELT_RU3), fld<R>(ctx, MELT_RUT), r4[0], r4[1], r4[2], r4[3], sc_u, sc_t, D, gu, gt)
+    if (rows == 2) ZM_LAUNCH(2);
+    else ZM_LAUNCH(1);
+#undef ZM_LAUNCH
     MELT_HIP(hipGetLastError());
     return 0;
   }
-  // W x-lines per block: the fewest that give a 256-cell tile (one cell per
-  // thread); small tiles keep the LDS and register footprint low.
-  int W = 0;
+  // W x-lines per block: as many as make at most 256 cells, one per thread
+  // (96^3 FP64: 2 lines 45 us, 3 lines with two cells a thread 59; 48^3: 4 lines 14,
+  // 6 lines 18); small tiles keep the LDS and register footprint low.
+  int W = 1;
   if (ctx->tune[TUNE_XF_W] > 0 && ctx->n2 % ctx->tune[TUNE_XF_W] == 0) W = ctx->tune[TUNE_XF_W];
   else
-    for (int w = 1; w <= ctx->n2 && !W; ++w)
-      if (ctx->n2 % w == 0 && (w * ctx->n1 >= 256 || w == ctx->n2)) W = w;
+    for (int w = 2; w <= ctx->n2 && w * ctx->n1 <= 256; ++w)
+      if (ctx->n2 % w == 0) W = w;
   if (W * ctx->n1 > 2048) return melt_fail(ctx, MELT_ERR_ARG, "explicit_xsolve", "tile too large");
   int ncell = W * ctx->n1;
   int nt = pick_threads(ncell, 256, ctx->tune[TUNE_XF_NT]);
