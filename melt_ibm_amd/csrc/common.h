@@ -442,21 +442,30 @@ __device__ inline void raise_error(int* err, int code) {
 }
 
 // Max reductions of non-negative doubles: their bit patterns order like the
-// values, so partial maxima combine with integer atomicMax.  Each block folds
-// its maximum into slot blockIdx % REDUCE_SLOTS (few atomics per address);
-// euler_fold_slots turns the slots into one value and clears them.
+// values, so partial maxima combine as integers.  A launch of at most
+// REDUCE_SLOTS blocks stores each block's maximum in its own slot
+// (block_max_store); a larger one folds it into slot blockIdx % REDUCE_SLOTS
+// (block_max_to_slots: few atomics per address).  euler_fold_slots turns the
+// slots into one value and clears them.
 constexpr int REDUCE_SLOTS = 1024;
-__device__ inline void block_max_to_slots(double v, unsigned long long* slots) {
+__device__ inline double block_max(double v) {   // valid in thread 0
   __shared__ double wm[16];
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
   if (lane == 0) wm[w] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double m = wm[0];
+  double m = wm[0];
+  if (threadIdx.x == 0)
     for (int q = 1; q < nw; ++q) m = fmax(m, wm[q]);
-    atomicMax(&slots[blockIdx.x % REDUCE_SLOTS], (unsigned long long)__double_as_longlong(m));
-  }
+  return m;
+}
+__device__ inline void block_max_to_slots(double v, unsigned long long* slots) {
+  const double m = block_max(v);
+  if (threadIdx.x == 0) atomicMax(&slots[blockIdx.x % REDUCE_SLOTS], (unsigned long long)__double_as_longlong(m));
+}
+__device__ inline void block_max_store(double v, unsigned long long* slot) {
+  const double m = block_max(v);
+  if (threadIdx.x == 0) *slot = (unsigned long long)__double_as_longlong(m);
 }
 
 // XCD-aware block remap: consecutive logical blocks land on the same XCD (the
@@ -506,7 +515,7 @@ int poisson_init(melt_ctx* ctx);
 // div_slots != null: the forward x pass also folds max |div u| (FP64, as
 // divgck) into those REDUCE_SLOTS slots.
 int poisson_solve(melt_ctx* ctx, int fused_divg, const int* gate = nullptr, unsigned long long* div_slots = nullptr);
-int euler_fold_slots(melt_ctx* ctx, unsigned long long* slots, unsigned long long* out);
+int euler_fold_slots(melt_ctx* ctx, unsigned long long* slots, unsigned long long* out, int used = REDUCE_SLOTS);
 int ibm_tag(melt_ctx* ctx);
 int ibm_find_centroid_indices(melt_ctx* ctx);
 int ibm_weights(melt_ctx* ctx, bool find = false);   // find: form the cell indices too

@@ -1229,17 +1229,23 @@ __global__ __launch_bounds__(256) void k_interp_vof(Grid g, const R* __restrict_
 
 // Max reductions of cfl.f90:9-25 (what = 0), divgck divg.f90:36-50
 // (what = 1) and get_dt's advective measure cfl.f90:48-51 (what = 2, with dt),
-// in FP64 arithmetic whatever the storage type; the result (non-negative) is
-// combined by atomicMax on its bit pattern.
+// in FP64 arithmetic whatever the storage type.  At most REDUCE_SLOTS blocks
+// walk the tiles of REDUCE_THREADS * V cells and store one (non-negative)
+// maximum each, so no slot has to be cleared beforehand.
+constexpr int REDUCE_THREADS = 512;
+inline unsigned reduce_tiles(size_t nc, int V) { return (unsigned)((nc / V + REDUCE_THREADS - 1) / REDUCE_THREADS); }
+inline unsigned reduce_blocks(size_t nc, int V) { return std::min(reduce_tiles(nc, V), (unsigned)REDUCE_SLOTS); }
 template <typename R>
-__global__ __launch_bounds__(256) void k_reduce_max(Grid g, const R* __restrict__ vx, const R* __restrict__ vy, const R* __restrict__ vz,
-                                                    int what, double dt, int nc, unsigned long long* slots) {
+__global__ __launch_bounds__(REDUCE_THREADS) void k_reduce_max(Grid g, const R* __restrict__ vx, const R* __restrict__ vy, const R* __restrict__ vz,
+                                                    int what, double dt, int nc, unsigned tiles, unsigned long long* __restrict__ slots) {
   // V consecutive x cells per thread through 16-byte loads (n1 % V == 0)
   constexpr int V = 16 / sizeof(R);
   struct alignas(16) Vec { R v[V]; };
   double m = what == 0 ? 0.00000001 : 0.0;
-  const int c = (int)(xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x) * V;
-  if (c < nc) {
+  for (unsigned t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const unsigned at = (xcd_block(t, tiles) * blockDim.x + threadIdx.x) * V;
+    if (at >= (unsigned)nc) continue;
+    const int c = (int)at;
     const Cell s = make_cell(g, c);
     const Vec X = *reinterpret_cast<const Vec*>(vx + c), Y0 = *reinterpret_cast<const Vec*>(vy + c);
     const Vec Y1 = *reinterpret_cast<const Vec*>(vy + s.at(0, 1, 0)), Z0 = *reinterpret_cast<const Vec*>(vz + c);
@@ -1258,22 +1264,30 @@ __global__ __launch_bounds__(256) void k_reduce_max(Grid g, const R* __restrict_
       m = fmax(m, q);
     }
   }
-  block_max_to_slots(m, slots);
+  block_max_store(m, slots + blockIdx.x);
 }
 
-// The REDUCE_SLOTS partial maxima into *out; the slots are cleared for the
-// next reduction.  One block of REDUCE_SLOTS threads.
-__global__ __launch_bounds__(REDUCE_SLOTS) void k_fold_slots(unsigned long long* __restrict__ slots, unsigned long long* __restrict__ out) {
-  __shared__ unsigned long long sm[REDUCE_SLOTS];
+// The first `used` partial maxima into *out; all the slots are cleared for
+// the next reduction.  One block of FOLD_THREADS threads.
+constexpr int FOLD_THREADS = 256;
+__global__ __launch_bounds__(FOLD_THREADS) void k_fold_slots(unsigned long long* __restrict__ slots, int used, unsigned long long* __restrict__ out) {
+  __shared__ unsigned long long sm[FOLD_THREADS / 64];
   const int t = threadIdx.x;
-  sm[t] = slots[t];
-  slots[t] = 0ull;
-  __syncthreads();
-  for (int w = REDUCE_SLOTS / 2; w > 0; w >>= 1) {
-    if (t < w) sm[t] = sm[t] > sm[t + w] ? sm[t] : sm[t + w];
-    __syncthreads();
+  unsigned long long v[REDUCE_SLOTS / FOLD_THREADS], m = 0ull;
+#pragma unroll
+  for (int q = 0; q < REDUCE_SLOTS / FOLD_THREADS; ++q) v[q] = slots[t + q * FOLD_THREADS];
+#pragma unroll
+  for (int q = 0; q < REDUCE_SLOTS / FOLD_THREADS; ++q) {
+    slots[t + q * FOLD_THREADS] = 0ull;
+    if (t + q * FOLD_THREADS < used) m = max(m, v[q]);
   }
-  if (t == 0) *out = sm[0];
+  for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned long long)__shfl_xor((long long)m, o, 64));
+  if ((t & 63) == 0) sm[t >> 6] = m;
+  __syncthreads();
+  if (t == 0) {
+    for (int q = 1; q < FOLD_THREADS / 64; ++q) m = max(m, sm[q]);
+    *out = m;
+  }
 }
 
 // Refinement gate of the precision form: refine while the FP64 divergence of
@@ -1646,17 +1660,18 @@ int launch_interp_vof(melt_ctx* ctx) {
   return 0;
 }
 
-// Launch the max reduction into d: one cell per thread into the partial
+// Launch the max reduction into d: one maximum per block into the partial
 // slots, then one block folds them (kernels only, so the sequence may be
 // captured into a graph).
 template <typename R>
 int launch_reduce_max(melt_ctx* ctx, int what, unsigned long long* d, double dt) {
   constexpr int V = 16 / sizeof(R);
   if (ctx->n1 % V) return melt_fail(ctx, MELT_ERR_ARG, "reduce_max", "n1m is not a multiple of the vector width");
-  hipLaunchKernelGGL(k_reduce_max<R>, dim3(nblocks(ctx->nc / V, 256)), dim3(256), 0, ctx->stream, make_grid(ctx), fld<R>(ctx, MELT_VX),
-                     fld<R>(ctx, MELT_VY), fld<R>(ctx, MELT_VZ), what, dt, (int)ctx->nc, ctx->d_slots);
+  const unsigned nb = reduce_blocks(ctx->nc, V);
+  hipLaunchKernelGGL(k_reduce_max<R>, dim3(nb), dim3(REDUCE_THREADS), 0, ctx->stream, make_grid(ctx), fld<R>(ctx, MELT_VX),
+                     fld<R>(ctx, MELT_VY), fld<R>(ctx, MELT_VZ), what, dt, (int)ctx->nc, reduce_tiles(ctx->nc, V), ctx->d_slots);
   MELT_HIP(hipGetLastError());
-  return euler_fold_slots(ctx, ctx->d_slots, d);
+  return euler_fold_slots(ctx, ctx->d_slots, d, (int)nb);
 }
 
 template <typename R>
@@ -1699,8 +1714,8 @@ int euler_launch_interp_vof(melt_ctx* ctx) { return ctx->fp32 ? launch_interp_vo
 int euler_launch_reduce_max(melt_ctx* ctx, int what, unsigned long long* d, double dt) {
   return ctx->fp32 ? launch_reduce_max<float>(ctx, what, d, dt) : launch_reduce_max<double>(ctx, what, d, dt);
 }
-int euler_fold_slots(melt_ctx* ctx, unsigned long long* slots, unsigned long long* out) {
-  hipLaunchKernelGGL(k_fold_slots, dim3(1), dim3(REDUCE_SLOTS), 0, ctx->stream, slots, out);
+int euler_fold_slots(melt_ctx* ctx, unsigned long long* slots, unsigned long long* out, int used) {
+  hipLaunchKernelGGL(k_fold_slots, dim3(1), dim3(FOLD_THREADS), 0, ctx->stream, slots, used, out);
   MELT_HIP(hipGetLastError());
   return 0;
 }
@@ -1753,16 +1768,14 @@ int noalloc_scratch(unsigned long long** out) {
   return 0;
 }
 
-__global__ __launch_bounds__(REDUCE_SLOTS) void k_clear_slots(unsigned long long* __restrict__ slots) { slots[threadIdx.x] = 0ull; }
-
 template <typename R>
 int divgck_noalloc(const void* vx, const void* vy, const void* vz, const Grid& g, hipStream_t s, double* qmax, unsigned long long* slots) {
   constexpr int V = 16 / sizeof(R);
   const size_t nc = (size_t)g.n1 * g.n2 * g.n3;
-  hipLaunchKernelGGL(k_clear_slots, dim3(1), dim3(REDUCE_SLOTS), 0, s, slots);
-  hipLaunchKernelGGL(k_reduce_max<R>, dim3(nblocks(nc / V, 256)), dim3(256), 0, s, g, static_cast<const R*>(vx), static_cast<const R*>(vy),
-                     static_cast<const R*>(vz), 1, 0.0, (int)nc, slots);
-  hipLaunchKernelGGL(k_fold_slots, dim3(1), dim3(REDUCE_SLOTS), 0, s, slots, reinterpret_cast<unsigned long long*>(qmax));
+  const unsigned nb = reduce_blocks(nc, V);
+  hipLaunchKernelGGL(k_reduce_max<R>, dim3(nb), dim3(REDUCE_THREADS), 0, s, g, static_cast<const R*>(vx), static_cast<const R*>(vy),
+                     static_cast<const R*>(vz), 1, 0.0, (int)nc, reduce_tiles(nc, V), slots);
+  hipLaunchKernelGGL(k_fold_slots, dim3(1), dim3(FOLD_THREADS), 0, s, slots, (int)nb, reinterpret_cast<unsigned long long*>(qmax));
   return hipGetLastError() == hipSuccess ? 0 : MELT_ERR_HIP;
 }
 
