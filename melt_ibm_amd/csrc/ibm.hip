@@ -270,13 +270,16 @@ __device__ __forceinline__ int mls_grad_lanes(const Grid& g, const R* __restrict
 // high word changes only when the running sum crosses a multiple of 2^64
 // (for a small negative contribution its all-ones high word and the carry
 // cancel), so its atomic is issued only when hi + carry is not zero.
-__device__ inline void acc_add(unsigned long long* w /* [lo, hi] */, double v) {
-  unsigned long long lo, hi;
-  acc_split(v, lo, hi);
+__device__ inline void acc_add_split(unsigned long long* w /* [lo, hi] */, unsigned long long lo, unsigned long long hi) {
   if ((lo | hi) == 0) return;
   unsigned long long old = atomicAdd(&w[0], lo);
   unsigned long long carry = (old + lo < old) ? 1ull : 0ull;
   if (hi + carry) atomicAdd(&w[1], hi + carry);
+}
+__device__ inline void acc_add(unsigned long long* w, double v) {
+  unsigned long long lo, hi;
+  acc_split(v, lo, hi);
+  acc_add_split(w, lo, hi);
 }
 
 __device__ inline long long win_slot(const int org[3], const int E[3], int iu, int ju, int ku) {
@@ -741,6 +744,15 @@ __global__ __launch_bounds__(64) void k_mls_weights(Grid g, const double* __rest
   if (mls_phi(g, pos, i0, j0, k0, c, [&](int q, double v) { o[q] = v; })) raise_error(err, MELT_ERR_SINGULAR_MLS);
 }
 
+constexpr int FORCE_CELLS = 1024;   // table of k_mls_force: 20 KiB of LDS
+constexpr int FORCE_FACES = 64;     // faces per block, at most
+
+// Order the LDS accesses of one wave (its lanes run in step).
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 template <typename R>
 struct ForceArgs {
   const R* fld[4];        // vx, vy, temp, vz
@@ -750,47 +762,108 @@ struct ForceArgs {
   double tmelt;
 };
 
-// forc1/forc2/forctemp/forc3: Um = sum q phi; spread cfac (V - Um) phi
+// A block's open-addressing table of window cells in LDS: `slot` of a cell,
+// claimed on first use, or -1 once PROBES neighbours are taken by others (the
+// caller then works on the cell in memory).  Neighbouring faces share most of
+// their stencil cells, whatever the mesh's order makes of the group's extent,
+// so one update per cell and block leaves the CU instead of one per (face, cell).
+template <int N>
+struct CellTable {
+  static constexpr int PROBES = 8, RUN = 8;   // RUN neighbours of a line stay together: 128 bytes of accumulators
+  static_assert((N & (N - 1)) == 0, "a power of two");
+  int cell[N];   // -1: free
+  __device__ int slot(int s) {
+    unsigned h = ((unsigned)s / RUN * 2654435761u >> (32 - __builtin_ctz(N / RUN))) * RUN + (unsigned)s % RUN;
+#pragma unroll 1
+    for (int q = 0; q < PROBES; ++q) {
+      int have = cell[h];
+      if (have == -1) have = atomicCAS(&cell[h], -1, s);
+      if (have == -1 || have == s) return (int)h;
+      h = (h + RUN) & (N - 1);
+    }
+    return -1;
+  }
+};
+
 // forc1/forc2/forctemp/forc3 (forc1.f90:28-65): Um = sum q phi, spread
-// cfac (V - Um) phi.  32 lanes per (face, component): lane l < 27 loads stencil
-// point l and its weight, every lane forms Um from the 27 products in the
-// reference's point order (shuffles, so Um rounds exactly as the serial loop),
-// and lane l adds its contribution to the exact 64.64 accumulators.
-template <typename R>
-__global__ __launch_bounds__(256) void k_mls_force(Grid g, ForceArgs<R> F, const double* __restrict__ bar, const unsigned char* __restrict__ gf,
-                                                   int nf, const int* __restrict__ pind, const melt_window* __restrict__ win, Win3 ef,
+// cfac (V - Um) phi.  32 lanes per face: lane l < 27 loads stencil point l and
+// its weight, every lane forms Um from the 27 products in the reference's
+// point order (so Um rounds exactly as the serial loop), and lane l adds its
+// contribution to the exact 64.64 accumulators.  A block takes fpb faces of one
+// component and sums them per cell in LDS first (integer words: the sums do not
+// depend on the order).  Bound by updates of the accumulators in memory, whose
+// atomics no cache takes: 77 us for 20480 faces on 128^3 with an update per
+// face and cell, 38 with a table whose every cell hashes by itself (16 of them the
+// flush, each update a transaction of its own), 27 with eight cells of a line
+// kept together.
+template <typename R, int T>
+__global__ __launch_bounds__(T) void k_mls_force(Grid g, ForceArgs<R> F, const double* __restrict__ bar, const unsigned char* __restrict__ gf,
+                                                   int nf, int fpb, const int* __restrict__ pind, const melt_window* __restrict__ win, Win3 ef,
                                                    unsigned long long* __restrict__ acc, size_t cells, int* err) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int item = gid >> 5, l = threadIdx.x & 31, lbase = threadIdx.x & 32;
-  const int f = item >> 2, comp = item & 3;
-  // every lane takes part in the shuffles; dead items / lanes carry zeros
-  const bool live = f < nf && !gf[f];
-  int i0 = 0, j0 = 0, kw = 0, ku = 0;
-  if (live) {
-    const int* p = &pind[6 * f];
-    const double* pos = &bar[3 * f];
-    int k1u = (int)floor(pos[2] * g.dx3) + 1, kstu = fnint(pos[2] * g.dx3) + 1;
-    if (comp == 0) { i0 = p[3]; j0 = p[1]; kw = p[2]; ku = k1u; }
-    else if (comp == 1) { i0 = p[0]; j0 = p[4]; kw = p[2]; ku = k1u; }
-    else if (comp == 2) { i0 = p[0]; j0 = p[1]; kw = p[2]; ku = k1u; }
-    else { i0 = p[0]; j0 = p[1]; kw = p[5]; ku = kstu; }
+  __shared__ CellTable<FORCE_CELLS> tab;
+  __shared__ unsigned long long sum[FORCE_CELLS][2];
+  __shared__ __align__(16) double prods[T / 32][28];
+  __shared__ int site[FORCE_FACES][6];       // centre of the stencil: wrapped, 0-based; from the window's origin
+  __shared__ double face[FORCE_FACES][2];    // V, cfac
+  __shared__ bool alive[FORCE_FACES];
+  const int t = threadIdx.x, l = t & 31, comp = blockIdx.x & 3, f0 = (int)(blockIdx.x >> 2) * fpb;
+  if (t < fpb) {
+    const int f = f0 + t;
+    const bool live = f < nf && !gf[f];
+    alive[t] = live;
+    if (live) {
+      const int* p = &pind[6 * f];
+      const double z = bar[3 * f + 2] * g.dx3;
+      const int i0 = p[comp == 0 ? 3 : 0], j0 = p[comp == 1 ? 4 : 1], kw = p[comp == 3 ? 5 : 2];
+      const int ku = comp == 3 ? fnint(z) + 1 : (int)floor(z) + 1;
+      site[t][0] = pmod(i0 - 1, g.n1); site[t][1] = pmod(j0 - 1, g.n2); site[t][2] = pmod(kw - 1, g.n3);
+      site[t][3] = i0 - win[0].org[0]; site[t][4] = j0 - win[0].org[1]; site[t][5] = ku - win[0].org[2];
+      face[t][0] = comp == 2 ? F.tmelt : F.vel_tri[3 * f + (comp == 3 ? 2 : comp)];
+      face[t][1] = F.cfac[f];
+    }
   }
-  const bool act = live && l < 27;
+  for (int q = t; q < FORCE_CELLS; q += T) { tab.cell[q] = -1; sum[q][0] = 0ull; sum[q][1] = 0ull; }
+  __syncthreads();
+  unsigned long long* const out = acc + (size_t)comp * cells * 2;
+  const R* __restrict__ fld = F.fld[comp];
+  const double* __restrict__ phi = F.phi[comp];
   const int di = l % 3 - 1, dj = (l / 3) % 3 - 1, dk = l / 9 - 1;
-  double ph = 0.0, prod = 0.0;
-  if (act) {
-    ph = F.phi[comp][27 * (size_t)f + l];
-    prod = (double)F.fld[comp][widx(g, i0 + di, j0 + dj, kw + dk)] * ph;
-  }
-  double Um = 0.0;
+  double* const pr = prods[t >> 5];
+  auto wrap = [](int i, int n) { return i < 0 ? i + n : i >= n ? i - n : i; };
+  // the loads of the next face are in flight while this one is summed
+  auto load = [&](int r, double& ph, R& val) {
+    ph = 0.0;
+    val = R(0);
+    if (r >= fpb || l >= 27 || !alive[r]) return;
+    const int* st = site[r];
+    ph = phi[27 * (size_t)(f0 + r) + l];
+    val = fld[wrap(st[0] + di, g.n1) + g.n1 * (wrap(st[1] + dj, g.n2) + g.n2 * wrap(st[2] + dk, g.n3))];
+  };
+  double ph_next;
+  R val_next;
+  load(t >> 5, ph_next, val_next);
+  for (int r = t >> 5; r < fpb; r += T / 32) {
+    const double ph = ph_next;
+    const R val = val_next;
+    load(r + T / 32, ph_next, val_next);
+    if (!alive[r]) continue;   // all 32 lanes alike
+    if (l < 27) pr[l] = (double)val * ph;
+    wave_lds_fence();
+    double Um = 0.0;
 #pragma unroll
-  for (int q = 0; q < 27; ++q) Um = Um + __shfl(prod, lbase + q, 64);
-  if (!act) return;
-  double V = comp == 2 ? F.tmelt : F.vel_tri[3 * f + (comp == 0 ? 0 : comp == 1 ? 1 : 2)];
-  double v = F.cfac[f] * (V - Um) * ph;
-  long long sl = win_slot(win[0].org, ef.e, i0 + di, j0 + dj, ku + dk);
-  if (sl < 0) { raise_error(err, MELT_ERR_WINDOW); return; }
-  acc_add(&acc[((size_t)comp * cells + (size_t)sl) * 2], v);
+    for (int q = 0; q < 27; ++q) Um = Um + pr[q];
+    wave_lds_fence();
+    if (l >= 27) continue;
+    const double v = face[r][1] * (face[r][0] - Um) * ph;
+    const int a = site[r][3] + di, b = site[r][4] + dj, c = site[r][5] + dk;
+    if (a < 0 || b < 0 || c < 0 || a >= ef.e[0] || b >= ef.e[1] || c >= ef.e[2]) { raise_error(err, MELT_ERR_WINDOW); continue; }
+    const int sl = a + ef.e[0] * (b + ef.e[1] * c);   // window cells are below 2^30
+    const int h = tab.slot(sl);
+    acc_add(h >= 0 ? sum[h] : &out[(size_t)sl * 2], v);
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < FORCE_CELLS; q += T)
+    if (tab.cell[q] >= 0) acc_add_split(&out[(size_t)tab.cell[q] * 2], sum[q][0], sum[q][1]);
 }
 
 // Drain the accumulators: mode 0 adds the forces to the fields (velocity
@@ -1310,8 +1383,17 @@ static int ibm_force_scatter_t(melt_ctx* ctx) {
   F.phi[0] = ctx->d_lag[MELT_L_PTXAB_Q1]; F.phi[1] = ctx->d_lag[MELT_L_PTXAB_Q2];
   F.phi[2] = ctx->d_lag[MELT_L_PTXAB_TEMP]; F.phi[3] = ctx->d_lag[MELT_L_PTXAB_Q3];
   F.vel_tri = ctx->d_lag[MELT_L_VEL_TRI]; F.cfac = ctx->d_lag[MELT_L_CFAC]; F.tmelt = ctx->cfg.tmelt;
-  hipLaunchKernelGGL(k_mls_force<R>, dim3(nb((size_t)ctx->nf * 4 * 32, 256)), dim3(256), 0, ctx->stream, g, F, ctx->d_lag[MELT_L_TRI_BAR], ctx->d_gf,
-                     ctx->nf, ctx->d_pind, ctx->d_win, ef, ctx->d_acc, ctx->fwin_cells, ctx->d_err);
+#define MLS_FORCE(T, FPB)                                                                                                              \
+  hipLaunchKernelGGL((k_mls_force<R, T>), dim3(4 * nb(ctx->nf, FPB)), dim3(T), 0, ctx->stream, g, F, ctx->d_lag[MELT_L_TRI_BAR], ctx->d_gf, \
+                     ctx->nf, FPB, ctx->d_pind, ctx->d_win, ef, ctx->d_acc, ctx->fwin_cells, ctx->d_err)
+  // Many faces: as many per block as share their cells best (20480 faces: 64
+  // per block 27 us, 32 46, one update per face and cell 77).  Fewer faces: more
+  // blocks and more faces at a time (1280 faces: 16 by 512 threads 6.7 us,
+  // 8 by 256 8.1, 64 15.6; 5120 beside the probes: 32 by 512 15.7, 64 by 256 20.5).
+  if (ctx->nf > 8192) MLS_FORCE(256, 64);
+  else if (ctx->nf > 2560) MLS_FORCE(512, 32);
+  else MLS_FORCE(512, 16);
+#undef MLS_FORCE
   MELT_HIP(hipGetLastError());
   return 0;
 }

@@ -1,0 +1,45 @@
+"""The MLS forcing's groups of faces (16, 32 and 64 per block by the face
+count, with remainders) against the oracle, and the same body with its faces in
+random order, whose groups touch more cells than a block's table holds.  The
+spread forces are exact integer sums, so the order of the faces changes no bit.
+The oracle adds the same contributions in double precision, a few hundred per
+cell: below 1e-13 of the sum of their magnitudes, 1e-12 of the largest force."""
+import numpy as np
+import pytest
+
+import oracle
+from melt_ibm_amd import geometry
+from melt_ibm_amd.api import MeltContext
+from tests.helpers import load_state, make_cfg, random_state
+
+pytestmark = pytest.mark.gpu
+
+FORCES = ("for_xc", "for_yc", "for_zc", "for_temp")
+
+
+def _forces(cfg, st, mesh, order, lib=None):
+    c = MeltContext(cfg, lib=lib) if lib is not None else oracle.context(cfg)
+    c.set_geometry(mesh.xyz, mesh.vert_of_edge, np.ascontiguousarray(mesh.edge_of_face[order]), 1.1)
+    load_state(c, st)
+    c.set_dt(0.004)
+    c.findCentroidIndices()
+    c.mlsWeight()
+    c.mlsForce()
+    out = [c.download(f) for f in FORCES]
+    c.close()
+    return out
+
+
+@pytest.mark.parametrize("freq", [3, 11, 13, 22])   # 180, 2420, 3380, 9680 faces
+def test_forces_over_group_sizes_and_orders(gpu_lib, freq):
+    cfg = make_cfg(64)
+    st = random_state(cfg, 5)
+    mesh = geometry.icosphere(freq)
+    nf = mesh.edge_of_face.shape[0]
+    plain, mixed = np.arange(nf), np.random.default_rng(freq).permutation(nf)
+    want = _forces(cfg, st, mesh, plain)
+    print(f"# mlsForce {nf} faces, as built and shuffled", flush=True)
+    got, again = _forces(cfg, st, mesh, plain, gpu_lib), _forces(cfg, st, mesh, mixed, gpu_lib)
+    for name, a, b, w in zip(FORCES, got, again, want):
+        assert np.array_equal(a, b), (name, np.abs(a - b).max())
+        assert np.abs(w).max() > 0 and np.abs(a - w).max() <= 1e-12 * np.abs(w).max(), name
