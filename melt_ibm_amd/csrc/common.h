@@ -158,7 +158,7 @@ struct melt_ctx {
   size_t twin_cells = 0;
   unsigned long long* d_tkey = nullptr;
   int* d_tface = nullptr;
-  double* d_tdist = nullptr;   // the 125 band distances of every face (first tagging pass)
+  double* d_tdist = nullptr;   // 125 band distances (or records) and a record count per face (tagging)
   double* d_pcoef = nullptr;   // gradient probes' shape-function derivatives: 27 x 3 x 6 per face
   melt_window* d_win = nullptr;
   // ray tagging scratch (init only)

@@ -373,56 +373,59 @@ __global__ void k_window_final(melt_window* win, Win3 ef, Win3 et, int which, in
 }
 
 // ------------------------------------------------------------ narrow band
-// genSDF.f90:85-234, Eberly's point-triangle distance.
-__device__ double dist_point_tri(const double P[3], const double* V0, const double* V1, const double* V2) {
-  double E0[3], E1[3], DE[3];
-  for (int d = 0; d < 3; ++d) { E0[d] = V1[d] - V0[d]; E1[d] = V2[d] - V0[d]; DE[d] = V0[d] - P[d]; }
-  double a = E0[0] * E0[0] + E0[1] * E0[1] + E0[2] * E0[2];
-  double b = E0[0] * E1[0] + E0[1] * E1[1] + E0[2] * E1[2];
-  double c = E1[0] * E1[0] + E1[1] * E1[1] + E1[2] * E1[2];
-  double d = E0[0] * DE[0] + E0[1] * DE[1] + E0[2] * DE[2];
-  double e = E1[0] * DE[0] + E1[1] * DE[1] + E1[2] * DE[2];
-  double det = a * c - b * b, s = b * e - c * d, t = b * d - a * e;
-  if (s + t <= det) {
-    if (s < 0.0) {
-      if (t < 0.0) {
-        if (d < 0.0) { t = 0.0; s = (-d >= a) ? 1.0 : -d / a; }
-        else { s = 0.0; t = (e >= 0.0) ? 0.0 : ((-e >= c) ? 1.0 : -e / c); }
-      } else {
-        s = 0.0; t = (e >= 0.0) ? 0.0 : ((-e >= c) ? 1.0 : -e / c);
-      }
-    } else if (t < 0.0) {
-      t = 0.0; s = (d >= 0.0) ? 0.0 : ((-d >= a) ? 1.0 : -d / a);
-    } else {
-      double inv = 1.0 / det;
-      s = s * inv; t = t * inv;
-    }
+// genSDF.f90:85-234, Eberly's point-triangle distance.  The regions' cases
+// select one quotient, so a wave whose points lie in several regions divides
+// once (0/1 and 1/1 stand for the parameters 0 and 1).
+struct TriEdges {   // of one face, formed once
+  double V0[3], E0[3], E1[3], a, b, c, det;
+};
+__device__ inline TriEdges tri_edges(const double* V0, const double* V1, const double* V2) {
+  TriEdges T;
+  for (int d = 0; d < 3; ++d) { T.V0[d] = V0[d]; T.E0[d] = V1[d] - V0[d]; T.E1[d] = V2[d] - V0[d]; }
+  const double* E0 = T.E0;
+  const double* E1 = T.E1;
+  T.a = E0[0] * E0[0] + E0[1] * E0[1] + E0[2] * E0[2];
+  T.b = E0[0] * E1[0] + E0[1] * E1[1] + E0[2] * E1[2];
+  T.c = E1[0] * E1[0] + E1[1] * E1[1] + E1[2] * E1[2];
+  T.det = T.a * T.c - T.b * T.b;
+  return T;
+}
+__device__ double dist_point_tri(const double P[3], const TriEdges& T) {
+  const double a = T.a, b = T.b, c = T.c, det = T.det;
+  double DE[3];
+  for (int d = 0; d < 3; ++d) DE[d] = T.V0[d] - P[d];
+  const double d = T.E0[0] * DE[0] + T.E0[1] * DE[1] + T.E0[2] * DE[2];
+  const double e = T.E1[0] * DE[0] + T.E1[1] * DE[1] + T.E1[2] * DE[2];
+  double s = b * e - c * d, t = b * d - a * e;
+  const bool in = s + t <= det, sn = s < 0.0, tn = t < 0.0;
+  // past the edge opposite V0: the parameter t1 of the corner tested first
+  const double t0 = sn ? b + d : b + e, t1 = sn ? c + e : a + d;
+  const bool far = !in && (!(sn || tn) || t1 > t0);          // on that edge
+  const bool edge1 = in ? sn && !(tn && d < 0.0) : sn;       // else on E1 (s = 0) or E0 (t = 0)
+  const double g = edge1 ? e : d, h = edge1 ? c : a;
+  const bool inner = in && !sn && !tn;
+  double num, den;
+  if (inner) { num = 1.0; den = det; }
+  else if (far) {
+    num = sn || tn ? t1 - t0 : c + e - b - d;
+    den = a - 2.0 * b + c;
+    const bool zero = !(sn || tn) && num <= 0.0, one = num >= den;
+    if (zero || one) { num = zero ? 0.0 : 1.0; den = 1.0; }
   } else {
-    if (s < 0.0) {
-      double t0 = b + d, t1 = c + e;
-      if (t1 > t0) {
-        double num = t1 - t0, den = a - 2.0 * b + c;
-        if (num >= den) { s = 1.0; t = 0.0; } else { s = num / den; t = 1.0 - s; }
-      } else {
-        s = 0.0; t = (t1 <= 0.0) ? 1.0 : ((e >= 0.0) ? 0.0 : -e / c);
-      }
-    } else if (t < 0.0) {
-      double t0 = b + e, t1 = a + d;
-      if (t1 > t0) {
-        double num = t1 - t0, den = a - 2.0 * b + c;
-        if (num >= den) { t = 1.0; s = 0.0; } else { t = num / den; s = 1.0 - t; }
-      } else {
-        t = 0.0; s = (t1 <= 0.0) ? 1.0 : ((d >= 0.0) ? 0.0 : -d / a);
-      }
-    } else {
-      double num = c + e - b - d, den = a - 2.0 * b + c;
-      s = (num <= 0.0) ? 0.0 : ((num >= den) ? 1.0 : num / den);
-      t = 1.0 - s;
-    }
+    const bool one = in ? !(g >= 0.0) && -g >= h : t1 <= 0.0, zero = !one && g >= 0.0;
+    num = one ? 1.0 : zero ? 0.0 : -g;
+    den = one || zero ? 1.0 : h;
   }
-  double q[3];
-  for (int k = 0; k < 3; ++k) q[k] = (V0[k] + s * E0[k] + t * E1[k]) - P[k];
-  return sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
+  const double q = num / den;
+  if (inner) { s = s * q; t = t * q; }
+  else if (far) {
+    const bool on_t = !sn && tn;   // the quotient is t there, s elsewhere
+    s = on_t ? 1.0 - q : q;
+    t = on_t ? q : 1.0 - q;
+  } else { s = edge1 ? 0.0 : q; t = edge1 ? q : 0.0; }
+  double r[3];
+  for (int k = 0; k < 3; ++k) r[k] = (T.V0[k] + s * T.E0[k] + t * T.E1[k]) - P[k];
+  return sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
 }
 
 // The tagging's set-up in one launch: blocks [0, nbox) reduce the face
@@ -466,44 +469,199 @@ struct MeshArgs {
   int nf;
 };
 
-// MODE 0: distance of every (face, band cell), kept in dist[], and the min
-// per cell; 1: lowest face among the minima; 2: write sdf and VOFp.  The window
-// follows from the extent k_tag_prepare reduced: modes 0 and 1 take its origin
-// straight from there, one thread of mode 1 places the windows (no thread of
-// modes 0 and 1 reads the placed origin), and one of mode 2 resets the extent
-// (mode 2 reads the placed origin), so no launch of its own does.
-template <int MODE, typename R>
+// A block's open-addressing table of window cells in LDS: `slot` of a cell,
+// claimed on first use, or -1 once PROBES neighbours are taken by others (the
+// caller then works on the cell in memory).  Neighbouring faces share most of
+// their stencil cells, whatever the mesh's order makes of the group's extent,
+// so one update per cell and block leaves the CU instead of one per (face, cell).
+template <int N>
+struct CellTable {
+  static constexpr int PROBES = 8, RUN = 8;   // RUN neighbours of a line stay together: 128 bytes of accumulators
+  static_assert((N & (N - 1)) == 0, "a power of two");
+  int cell[N];   // -1: free
+  __device__ int slot(int s) {
+    unsigned h = ((unsigned)s / RUN * 2654435761u >> (32 - __builtin_ctz(N / RUN))) * RUN + (unsigned)s % RUN;
+#pragma unroll 1
+    for (int q = 0; q < PROBES; ++q) {
+      int have = cell[h];
+      if (have == -1) have = atomicCAS(&cell[h], -1, s);
+      if (have == -1 || have == s) return (int)h;
+      h = (h + RUN) & (N - 1);
+    }
+    return -1;
+  }
+};
+
+// Passes of the narrow-band tagging over groups of FPB faces.
+//
+// k_tag_band: distance of every (face, band cell) of a group, the min per cell
+// and the lowest face among the minima in LDS first, then one update of the
+// cell's key; the group's winners are left as records for the other two passes.
+// A group that touches more cells than its table or its records hold updates
+// the keys entry by entry and leaves its distances instead (count < 0).
+// k_tag_pass MODE 1: lowest face among the minima of all groups; 2: write sdf
+// and VOFp.
+// Neighbouring faces share most of their cells: a key update per entry (2.56 M
+// atomics for 20480 faces) and two more passes over all entries took 51 + 11 +
+// 20 us on 128^3; per group 28 + 5 + 9, the first bound by the distances'
+// arithmetic (36 before a wave's regions shared one division and the band's
+// coordinates were formed once per face).
+//
+// The window follows from the extent k_tag_prepare reduced: k_tag_band and mode
+// 1 take its origin straight from there, one thread of mode 1 places the
+// windows (no thread before mode 2 reads the placed origin), and one of mode 2
+// resets the extent (mode 2 reads the placed origin), so no launch of its own does.
+struct TagRecord {
+  unsigned long long key;   // the distance's bits
+  int cell, face;
+};
+
+// A group's share of the distances' memory: up to 125 distances a face, or
+// records, and behind the distances of all faces the groups' record counts.
+template <int FPB>
+struct TagGroup {
+  double* dist;
+  int* count;
+  int f0, nface;
+  __device__ TagGroup(double* dst, int nf, int group) {
+    f0 = group * FPB;
+    nface = min(FPB, nf - f0);
+    dist = dst + (size_t)f0 * 125;
+    count = reinterpret_cast<int*>(dst + (size_t)nf * 125) + group;
+  }
+  __device__ TagRecord* records() const { return reinterpret_cast<TagRecord*>(dist); }
+  __device__ int capacity() const { return nface * 125 / 2; }
+};
+
+template <int FPB, int T, int CELLS>
+__global__ __launch_bounds__(T) void k_tag_band(Grid g, MeshArgs M, const melt_window* __restrict__ win, Win3 et,
+                                                unsigned long long* __restrict__ key, double* __restrict__ dst, int* err) {
+  constexpr int E = (FPB * 125 + T - 1) / T;   // entries per thread
+  __shared__ CellTable<CELLS> tab;
+  __shared__ unsigned long long kmin[CELLS];
+  __shared__ int fmin[CELLS];
+  __shared__ TriEdges tri[FPB];
+  __shared__ double crd[FPB][15];   // the band's x, y and z (a division each)
+  __shared__ int base[FPB][3];
+  __shared__ bool alive[FPB];
+  __shared__ int used, full;
+  const TagGroup<FPB> G(dst, M.nf, blockIdx.x);
+  const int t = threadIdx.x, n = G.nface * 125;
+  if (t < FPB) {
+    const int f = G.f0 + t;
+    const bool live = t < G.nface && !M.gf[f];
+    alive[t] = live;
+    if (live) {
+      const int* v = &M.vof[3 * f];
+      tri[t] = tri_edges(&M.xyzv[3 * v[0]], &M.xyzv[3 * v[1]], &M.xyzv[3 * v[2]]);
+    }
+  }
+  for (int u = t; u < G.nface * 15; u += T) {
+    const int r = u / 15, m = u - 15 * r, d = m / 5, o = m - 5 * d;
+    const double x = M.bar[3 * (G.f0 + r) + d];
+    const int i0 = (int)floor(x * (d == 0 ? g.dx1 : d == 1 ? g.dx2 : g.dx3)) + 1, i = i0 + o - 2;
+    crd[r][m] = d == 0 ? gxm(g, i) : d == 1 ? gym(g, i) : gzm(g, i);
+    if (o == 0) base[r][d] = i0;
+  }
+  for (int q = t; q < CELLS; q += T) { tab.cell[q] = -1; kmin[q] = ~0ull; fmin[q] = INT_MAX; }
+  if (t == 0) { used = 0; full = 0; }
+  __syncthreads();
+  int org[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) org[d] = win[0].bmin[d] - 2;
+  unsigned long long dk[E];
+  int cell[E], slot[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int id = t + e * T, r = id / 125, q = id - 125 * r;
+    cell[e] = slot[e] = -1;
+    dk[e] = 0ull;
+    if (id >= n || !alive[r]) continue;
+    const int oi = q % 5, oj = (q / 5) % 5, ok = q / 25;
+    const long long s = win_slot(org, et.e, base[r][0] + oi - 2, base[r][1] + oj - 2, base[r][2] + ok - 2);
+    if (s < 0) { raise_error(err, MELT_ERR_WINDOW); continue; }
+    const double P[3] = {crd[r][oi], crd[r][5 + oj], crd[r][10 + ok]};
+    dk[e] = (unsigned long long)__double_as_longlong(dist_point_tri(P, tri[r]));
+    cell[e] = (int)s;   // window cells are below 2^30
+    slot[e] = tab.slot((int)s);
+    if (slot[e] >= 0) atomicMin(&kmin[slot[e]], dk[e]);
+    else full = 1;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (slot[e] >= 0 && kmin[slot[e]] == dk[e]) atomicMin(&fmin[slot[e]], G.f0 + (t + e * T) / 125);
+  for (int q0 = 0; q0 < CELLS; q0 += T) {
+    const unsigned long long m = __ballot(tab.cell[q0 + t] >= 0);
+    if ((t & 63) == 0 && m) atomicAdd(&used, (int)__popcll(m));
+  }
+  __syncthreads();
+  const int count = used;
+  if (full || count > G.capacity()) {
+    if (t == 0) *G.count = -1;
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (cell[e] >= 0) {
+        G.dist[t + e * T] = __longlong_as_double((long long)dk[e]);
+        atomicMin(&key[cell[e]], dk[e]);
+      }
+    return;
+  }
+  __syncthreads();
+  if (t == 0) { *G.count = count; used = 0; }
+  __syncthreads();
+  for (int q0 = 0; q0 < CELLS; q0 += T) {
+    const int q = q0 + t, c = tab.cell[q];
+    const unsigned long long m = __ballot(c >= 0);
+    int at = 0;
+    if ((t & 63) == 0 && m) at = atomicAdd(&used, (int)__popcll(m));
+    at = __shfl(at, 0, 64) + (int)__popcll(m & ((1ull << (t & 63)) - 1ull));
+    if (c >= 0) {
+      G.records()[at] = TagRecord{kmin[q], c, fmin[q]};
+      atomicMin(&key[c], kmin[q]);
+    }
+  }
+}
+
+template <int MODE, int FPB, typename R>
 __global__ __launch_bounds__(256) void k_tag_pass(Grid g, MeshArgs M, melt_window* __restrict__ win, Win3 ef, Win3 et, int which,
-                                                  unsigned long long* __restrict__ key, int* __restrict__ face, double* __restrict__ dst,
-                                                  R* __restrict__ sdf, R* __restrict__ vofp, double pi, int* err) {
-  const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (MODE == 1 && id == 0) window_place(win, ef, et, which, err);
-  if (MODE == 2 && id == 0) window_reset_extent(win);
-  if (id >= (size_t)M.nf * 125) return;
-  int f = (int)(id / 125), q = (int)(id % 125);
-  if (M.gf[f]) return;
-  const double* pos = &M.bar[3 * f];
-  int i = (int)floor(pos[0] * g.dx1) + 1 + (q % 5) - 2;
-  int j = (int)floor(pos[1] * g.dx2) + 1 + (q / 5) % 5 - 2;
-  int k = (int)floor(pos[2] * g.dx3) + 1 + q / 25 - 2;
+                                                  const unsigned long long* __restrict__ key, int* __restrict__ face,
+                                                  double* __restrict__ dst, R* __restrict__ sdf, R* __restrict__ vofp, double pi, int* err) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (MODE == 1) window_place(win, ef, et, which, err);
+    else window_reset_extent(win);
+  }
+  const TagGroup<FPB> G(dst, M.nf, blockIdx.x);
   int org[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) org[d] = MODE == 2 ? win[1].org[d] : win[0].bmin[d] - 2;
-  long long s = win_slot(org, et.e, i, j, k);
-  if (s < 0) { raise_error(err, MELT_ERR_WINDOW); return; }
-  if constexpr (MODE == 0) {
-    const double* V0 = &M.xyzv[3 * M.vof[3 * f + 0]];
-    const double* V1 = &M.xyzv[3 * M.vof[3 * f + 1]];
-    const double* V2 = &M.xyzv[3 * M.vof[3 * f + 2]];
-    double P[3] = {gxm(g, i), gym(g, j), gzm(g, k)};
-    double dist = dist_point_tri(P, V0, V1, V2);
-    dst[id] = dist;
-    atomicMin(&key[s], (unsigned long long)__double_as_longlong(dist));
-  } else {
-    const double dist = dst[id];
+  const int count = *G.count;
+  for (int id = threadIdx.x; id < (count >= 0 ? count : G.nface * 125); id += 256) {
+    int f, s, i, j, k;
+    unsigned long long dk;
+    if (count >= 0) {
+      const TagRecord rec = G.records()[id];
+      dk = rec.key; s = rec.cell; f = rec.face;
+      const int r = s / et.e[0], c = r / et.e[1];
+      i = org[0] + (s - r * et.e[0]); j = org[1] + (r - c * et.e[1]); k = org[2] + c;
+    } else {
+      const int q = id % 125;
+      f = G.f0 + id / 125;
+      if (M.gf[f]) continue;
+      const double* pos = &M.bar[3 * f];
+      i = (int)floor(pos[0] * g.dx1) + 1 + q % 5 - 2;
+      j = (int)floor(pos[1] * g.dx2) + 1 + (q / 5) % 5 - 2;
+      k = (int)floor(pos[2] * g.dx3) + 1 + q / 25 - 2;
+      const long long w = win_slot(org, et.e, i, j, k);
+      if (w < 0) continue;   // reported by k_tag_band
+      s = (int)w;
+      dk = (unsigned long long)__double_as_longlong(G.dist[id]);
+    }
     if constexpr (MODE == 1) {
-      if (key[s] == (unsigned long long)__double_as_longlong(dist)) atomicMin(&face[s], f);
+      if (key[s] == dk) atomicMin(&face[s], f);
     } else if (face[s] == f) {
+      const double dist = __longlong_as_double((long long)dk);
+      const double* pos = &M.bar[3 * f];
       double P[3] = {gxm(g, i), gym(g, j), gzm(g, k)};
       const double* n = &M.nor[3 * f];
       double dot = n[0] * (pos[0] - P[0]) + n[1] * (pos[1] - P[1]) + n[2] * (pos[2] - P[2]);
@@ -760,29 +918,6 @@ struct ForceArgs {
   const double* vel_tri;
   const double* cfac;
   double tmelt;
-};
-
-// A block's open-addressing table of window cells in LDS: `slot` of a cell,
-// claimed on first use, or -1 once PROBES neighbours are taken by others (the
-// caller then works on the cell in memory).  Neighbouring faces share most of
-// their stencil cells, whatever the mesh's order makes of the group's extent,
-// so one update per cell and block leaves the CU instead of one per (face, cell).
-template <int N>
-struct CellTable {
-  static constexpr int PROBES = 8, RUN = 8;   // RUN neighbours of a line stay together: 128 bytes of accumulators
-  static_assert((N & (N - 1)) == 0, "a power of two");
-  int cell[N];   // -1: free
-  __device__ int slot(int s) {
-    unsigned h = ((unsigned)s / RUN * 2654435761u >> (32 - __builtin_ctz(N / RUN))) * RUN + (unsigned)s % RUN;
-#pragma unroll 1
-    for (int q = 0; q < PROBES; ++q) {
-      int have = cell[h];
-      if (have == -1) have = atomicCAS(&cell[h], -1, s);
-      if (have == -1 || have == s) return (int)h;
-      h = (h + RUN) & (N - 1);
-    }
-    return -1;
-  }
 };
 
 // forc1/forc2/forctemp/forc3 (forc1.f90:28-65): Um = sum q phi, spread
@@ -1341,14 +1476,24 @@ static int ibm_tag_t(melt_ctx* ctx) {  // tagCells.f90:4-27 (tagType 1) + interp
   // faces do not move between tagging and forcing)
   const int which = ctx->force_window_from_tag ? 3 : 2;
   MeshArgs M = mesh_args(ctx);
-  unsigned blocks = nb((size_t)ctx->nf * 125, 256);
-#define TAG_PASS(MODE)                                                                                                                 \
-  hipLaunchKernelGGL((k_tag_pass<MODE, R>), dim3(blocks), dim3(256), 0, ctx->stream, g, M, ctx->d_win, ef, et, which, ctx->d_tkey,      \
-                     ctx->d_tface, ctx->d_tdist, fld<R>(ctx, MELT_SDF), fld<R>(ctx, MELT_VOFP), ctx->pi, ctx->d_err)
-  TAG_PASS(0);
-  TAG_PASS(1);
-  TAG_PASS(2);
-#undef TAG_PASS
+#define TAG_PASSES(FPB, T, CELLS)                                                                                                       \
+  do {                                                                                                                                  \
+    const dim3 groups(nb(ctx->nf, FPB));                                                                                                \
+    hipLaunchKernelGGL((k_tag_band<FPB, T, CELLS>), groups, dim3(T), 0, ctx->stream, g, M, ctx->d_win, et, ctx->d_tkey, ctx->d_tdist,    \
+                       ctx->d_err);                                                                                                     \
+    hipLaunchKernelGGL((k_tag_pass<1, FPB, R>), groups, dim3(256), 0, ctx->stream, g, M, ctx->d_win, ef, et, which, ctx->d_tkey,         \
+                       ctx->d_tface, ctx->d_tdist, fld<R>(ctx, MELT_SDF), fld<R>(ctx, MELT_VOFP), ctx->pi, ctx->d_err);                  \
+    hipLaunchKernelGGL((k_tag_pass<2, FPB, R>), groups, dim3(256), 0, ctx->stream, g, M, ctx->d_win, ef, et, which, ctx->d_tkey,         \
+                       ctx->d_tface, ctx->d_tdist, fld<R>(ctx, MELT_SDF), fld<R>(ctx, MELT_VOFP), ctx->pi, ctx->d_err);                  \
+  } while (0)
+  // As many faces a group as keep the chip's blocks busy (20480 faces on 128^3:
+  // 16 a group 42 us for the three passes, 8 50; 5120 faces: 8 22, 16 27; 1280: 4
+  // 16, 8 17), with twice the cells a group of neighbours touches in its table
+  // (16 faces with 1024 cells often leave their distances: 62).
+  if (ctx->nf > 8192) TAG_PASSES(16, 512, 2048);
+  else if (ctx->nf > 2560) TAG_PASSES(8, 512, 1024);
+  else TAG_PASSES(4, 512, 512);
+#undef TAG_PASSES
   MELT_HIP(hipGetLastError());
   return 0;
 }

@@ -940,7 +940,7 @@ int lagr_alloc(melt_ctx* ctx, const double* xyz0, const int* voe, const int* eof
   rc |= dalloc((void**)&ctx->d_acc, sizeof(unsigned long long) * 8 * ctx->fwin_cells);
   rc |= dalloc((void**)&ctx->d_tkey, sizeof(unsigned long long) * ctx->twin_cells);
   rc |= dalloc((void**)&ctx->d_tface, sizeof(int) * ctx->twin_cells);
-  rc |= dalloc((void**)&ctx->d_tdist, sizeof(double) * 125 * nf);
+  rc |= dalloc((void**)&ctx->d_tdist, (sizeof(double) * 125 + sizeof(int)) * nf);
   rc |= dalloc((void**)&ctx->d_pcoef, sizeof(double) * 27 * 3 * 6 * nf);
   rc |= dalloc((void**)&ctx->d_foe, sizeof(int) * 2 * ne);
   if (ctx->cfg.iremesh == 1) rc |= dalloc((void**)&ctx->d_xyz_melt, sizeof(double) * 3 * nv);

@@ -79,7 +79,7 @@ def request_bytes(m: Member, precision: int) -> int:
     nf = 20 * f * f
     nv = nf // 2 + 2
     win = min(n, int(np.ceil(2.0 * m.rad * max(1.0, m.aspect) * n / (2 * np.pi))) + 10) ** 3
-    b = esz * n ** 3 * 33 + 2 * esz * n1hp * n * n + 8 * (nf * (4 * 27 + 40 + 125 + 486) + nv * 24) + win * (4 * 16 + 12)
+    b = esz * n ** 3 * 33 + 2 * esz * n1hp * n * n + 8 * (nf * (4 * 27 + 40 + 126 + 486) + nv * 24) + win * (4 * 16 + 12)
     return int(b * 1.10) + 10 * 8 * n ** 3 + (64 << 20)
 
 

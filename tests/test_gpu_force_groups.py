@@ -1,9 +1,11 @@
-"""The MLS forcing's groups of faces (16, 32 and 64 per block by the face
-count, with remainders) against the oracle, and the same body with its faces in
+"""The tagging's and the MLS forcing's groups of faces (their size by
+the face count, with remainders) against the oracle, and the same body with its faces in
 random order, whose groups touch more cells than a block's table holds.  The
 spread forces are exact integer sums, so the order of the faces changes no bit.
 The oracle adds the same contributions in double precision, a few hundred per
-cell: below 1e-13 of the sum of their magnitudes, 1e-12 of the largest force."""
+cell: below 1e-13 of the sum of their magnitudes, 1e-12 of the largest force.
+The distances and volume fractions are the oracle's bit for bit, the lowest
+face among equals included."""
 import numpy as np
 import pytest
 
@@ -43,3 +45,22 @@ def test_forces_over_group_sizes_and_orders(gpu_lib, freq):
     for name, a, b, w in zip(FORCES, got, again, want):
         assert np.array_equal(a, b), (name, np.abs(a - b).max())
         assert np.abs(w).max() > 0 and np.abs(a - w).max() <= 1e-12 * np.abs(w).max(), name
+
+
+@pytest.mark.parametrize("freq", [3, 11, 13, 22])
+@pytest.mark.parametrize("order", ["as built", "shuffled"])
+def test_tags_over_group_sizes_and_orders(gpu_lib, freq, order):
+    cfg = make_cfg(96)
+    mesh = geometry.icosphere(freq)
+    nf = mesh.edge_of_face.shape[0]
+    perm = np.arange(nf) if order == "as built" else np.random.default_rng(freq).permutation(nf)
+    print(f"# tagCells {nf} faces, {order}", flush=True)
+    out = []
+    for c in (MeltContext(cfg, lib=gpu_lib), oracle.context(cfg)):
+        c.set_geometry(mesh.xyz, mesh.vert_of_edge, np.ascontiguousarray(mesh.edge_of_face[perm]), 1.9)
+        for _ in range(2):   # the second call resets what the first one tagged
+            c.tagCells()
+        out.append([c.download(f) for f in ("sdf", "VOFp")])
+        c.close()
+    for name, a, b in zip(("sdf", "VOFp"), *out):
+        assert np.array_equal(a, b), (name, int((a != b).sum()))
