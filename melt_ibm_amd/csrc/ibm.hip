@@ -108,117 +108,147 @@ __device__ int mls_phi(const Grid& g, const double pos[3], int i0, int j0, int k
   return 0;
 }
 
-__device__ inline double dweight(double pc, double gcrd, double nrm, double scale) {
+// The weight derivative of one axis; inv = 1 / scale.
+__device__ inline double dweight(double dist, double nrm, double inv) {
   if (nrm < 2.220446049250313e-16) return 0.0;  // EPSILON(1.0d0)
-  double d = mls_gauss_deriv(nrm);
-  return d * ((pc - gcrd) / fabs(pc - gcrd) / scale);
+  return mls_gauss_deriv(nrm) * copysign(inv, dist);   // dist / |dist| / scale
 }
+
+// Order the LDS accesses of one wave (its lanes run in step).
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Exchange area of the 64 probes of a k_probes_grad block.
+struct GradShared {
+  double crd[9][64], w[9][64], dw[9][64];   // coordinate, weight and its derivative of (axis, point) pair 3 axis + point
+  double A[16][64];                         // moment matrix, then its inverse
+  double pg[4][64];                         // probe position, then gamma
+  int info[64];                             // -1: no probe
+};
 
 // MLS gradient at a probe (wght_gradT mls_heatFlux.f90:85-300 and
 // wght_gradP/U/V/W mls_structLoads.f90:380-1297), computed by the 4 lanes of
 // one probe: lane 0 accumulates the moment matrix A, lane 1+d the derivative
-// matrix dA/dx_d; after A is shared through shA (16 doubles, block barrier),
-// lanes 1..3 each invert A and form gradient component d in the reference's
-// point order, so every value rounds as in the single-thread formulation.
+// matrix dA/dx_d; one wave inverts the block's 64 matrices, a lane each (a
+// different wave from block to block, for the SIMDs' sake); lanes 1..3 form
+// gradient component d in the reference's point order, so every value rounds
+// as in the single-thread formulation.
 // kz: grid indices used for the z coordinate (the reference uses k1-1, k1,
 // k1); ke: field planes (1-based, ghost-plane semantics) k1-1, k1, k1+1.
-// Must be reached by every thread of the block (it contains a barrier);
-// active = 0 lanes only take part in the barrier.  Returns the LU info of A
-// on lanes 1..3 (0 elsewhere); *grad_d receives component lane-1.
-template <typename R>
-__device__ __forceinline__ int mls_grad_lanes(const Grid& g, const R* __restrict__ fld, const double pos[3], int ic, int jc, const int kz[3],
-                              const int ke[3], const int c[3], int lane, bool active, double* shA, double* grad_d,
-                              double* coef = nullptr, size_t cstride = 0) {
-  const double sx = WSCL / g.dx1, sy = WSCL / g.dx2, sz = WSCL / g.dx3;
-  // the field planes, read once: a per-plane pick from ke[] inside the rolled
-  // loop is folded into one load at a selected offset, which keeps the
-  // caller's probe-site record in scratch memory
-  const int ke0 = ke[0], ke1 = ke[1], ke2 = ke[2];
-  double xs[3], ys[3], zs[3], w1[3], w2[3], w3[3], dw1[3], dw2[3], dw3[3];
-  double M[16];
-#pragma unroll
-  for (int q = 0; q < 16; ++q) M[q] = 0.0;
+// Must be reached by every thread of the block (it contains barriers);
+// active = 0 lanes only take part in the barriers.  Returns the LU info of A
+// on lanes 1..3 (0 elsewhere); with COEF the 27 shape-function derivatives of
+// component lane-1 go to coef[q cstride], otherwise *grad_d receives their sum
+// against the field.
+//
+// Bound by its FP64 instructions: 4350 a wave and 88 us for six probes of 20480
+// faces on 128^3 with every lane forming all nine coordinates and the inverse,
+// a branch per point for the lane's weight and a wrap per point of the field; 2970
+// and 60 us this way (with COEF, 5120 faces beside the explicit pass: 25 -> 18).
+template <bool COEF, typename R>
+__device__ __forceinline__ int mls_grad_lanes(const Grid& g, GradShared& sh, const R* __restrict__ fld, const double pos[3], int ic, int jc,
+                                              const int kz[3], const int ke[3], const int c[3], int lane, bool active, double* grad_d,
+                                              double* coef, size_t cstride) {
+  const int slot = threadIdx.x >> 2;
+  double M[16];   // column 0 only stands for row 0 too: (w 1) p_i and (w p_i) 1 round alike
   if (active) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      xs[q] = gco(g, 0, c[0], ic - 1 + q);
-      ys[q] = gco(g, 1, c[1], jc - 1 + q);
-      zs[q] = gco(g, 2, c[2], kz[q]);
-    }
-    // separable Gaussian factors and derivatives of the nine (axis, point)
-    // pairs: pair p = 3 axis + point is evaluated on lane p % 4 of the
-    // probe's 4-lane group only (one exponential per pair instead of one per
-    // pair and lane) and read by the others from there
-    double mw[3], md[3];
+    // pair p = 3 axis + point is evaluated on lane p % 4 of the probe's lanes
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
       const int pp = lane + 4 * r, ax = pp / 3, q = pp - 3 * ax;
+      if (pp >= 9) continue;
       // selects, not an indexed pick (which would put the arrays in scratch)
-      const double cx = q == 0 ? xs[0] : q == 1 ? xs[1] : xs[2], cy = q == 0 ? ys[0] : q == 1 ? ys[1] : ys[2];
-      const double cz = q == 0 ? zs[0] : q == 1 ? zs[1] : zs[2];
-      const double crd = ax == 0 ? cx : ax == 1 ? cy : cz;
+      const int i = ax == 0 ? ic - 1 + q : ax == 1 ? jc - 1 + q : q == 0 ? kz[0] : q == 1 ? kz[1] : kz[2];
+      const double n = ax == 0 ? (double)g.n1 : ax == 1 ? (double)g.n2 : (double)g.n3;
+      const double len = ax == 0 ? g.xlen : ax == 1 ? g.ylen : g.zlen;
       const double pc = ax == 0 ? pos[0] : ax == 1 ? pos[1] : pos[2];
-      const double sc = ax == 0 ? sx : ax == 1 ? sy : sz;
-      const double n = fabs(pc - crd) / sc;
-      mw[r] = pp < 9 ? mls_gaussian(n) : 0.0;
-      md[r] = pp < 9 ? dweight(pc, crd, n, sc) : 0.0;
+      const double sc = WSCL / (ax == 0 ? g.dx1 : ax == 1 ? g.dx2 : g.dx3);
+      const bool centre = (ax == 0 ? c[0] : ax == 1 ? c[1] : c[2]) != 0;
+      double x = len * ((double)(i - 1) / n);          // gco(g, ax, centre, i)
+      if (centre) x = (x + len * ((double)i / n)) * 0.5;
+      const double nrm = fabs(pc - x) / sc;
+      sh.crd[pp][slot] = x;
+      sh.w[pp][slot] = mls_gaussian(nrm);
+      sh.dw[pp][slot] = dweight(pc - x, nrm, 1.0 / sc);
     }
-    double wv[9], dv[9];
-#pragma unroll
-    for (int pp = 0; pp < 9; ++pp) {
-      wv[pp] = __shfl(mw[pp / 4], pp % 4, 4);
-      dv[pp] = __shfl(md[pp / 4], pp % 4, 4);
-    }
+    wave_lds_fence();
+    // this lane's factors: the derivative's on its own axis
+    const double(*fx)[64] = lane == 1 ? sh.dw : sh.w;
+    const double(*fy)[64] = lane == 2 ? sh.dw : sh.w;
+    const double(*fz)[64] = lane == 3 ? sh.dw : sh.w;
+    double xs[3], ys[3], f1[3], f2[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      w1[q] = wv[q]; dw1[q] = dv[q];
-      w2[q] = wv[3 + q]; dw2[q] = dv[3 + q];
-      w3[q] = wv[6 + q]; dw3[q] = dv[6 + q];
+      xs[q] = sh.crd[q][slot]; ys[q] = sh.crd[3 + q][slot];
+      f1[q] = fx[q][slot]; f2[q] = fy[3 + q][slot];
     }
+#pragma unroll
+    for (int q = 0; q < 16; ++q) M[q] = 0.0;
 #pragma unroll 1
     for (int nk = 0; nk < 3; ++nk) {
-      // the z loop stays rolled (code size); selecting its plane's values
-      // keeps the arrays in registers (an index by nk would put them in scratch)
-      const double zk = nk == 0 ? zs[0] : nk == 1 ? zs[1] : zs[2];
-      const double w3k = nk == 0 ? w3[0] : nk == 1 ? w3[1] : w3[2];
-      const double dw3k = nk == 0 ? dw3[0] : nk == 1 ? dw3[1] : dw3[2];
+      const double zk = sh.crd[6 + nk][slot], f3 = fz[6 + nk][slot];
+      // lane 0: w1 (w2 w3); the others: (f1 f2) f3
+      double G[3], H[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) { G[q] = lane == 0 ? f3 : f1[q]; H[q] = lane == 0 ? f1[q] : f3; }
 #pragma unroll
       for (int jq = 0; jq < 3; ++jq)
 #pragma unroll
         for (int iq = 0; iq < 3; ++iq) {
-          double p[4] = {1.0, xs[iq], ys[jq], zk};
-          double wgt;
-          if (lane == 0) wgt = w1[iq] * (w2[jq] * w3k);
-          else if (lane == 1) wgt = dw1[iq] * w2[jq] * w3k;
-          else if (lane == 2) wgt = w1[iq] * dw2[jq] * w3k;
-          else wgt = w1[iq] * w2[jq] * dw3k;
-          rank1(M, wgt, p);
+          const double wgt = (f2[jq] * G[iq]) * H[iq];
+          const double p[3] = {xs[iq], ys[jq], zk};
+          M[0] = M[0] + wgt;
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            const double temp = wgt * p[j];
+            M[j + 1] = M[j + 1] + temp;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) M[i + 1 + 4 * (j + 1)] = M[i + 1 + 4 * (j + 1)] + temp * p[i];
+          }
         }
     }
-    if (lane == 0)
 #pragma unroll
-      for (int q = 0; q < 16; ++q) shA[q] = M[q];
+    for (int j = 1; j < 4; ++j) M[4 * j] = M[j];
+  }
+  if (lane == 0) {
+    sh.info[slot] = active ? 0 : -1;
+    if (active) {
+#pragma unroll
+      for (int q = 0; q < 16; ++q) sh.A[q][slot] = M[q];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) sh.pg[q][slot] = pos[q];
+    }
+  }
+  __syncthreads();
+  if ((threadIdx.x >> 6) == (blockIdx.x & 3)) {
+    const int t = threadIdx.x & 63;
+    if (sh.info[t] == 0) {
+      double A[16], gam[4];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) A[q] = sh.A[q][t];
+      sh.info[t] = lu_inverse<4>(A);
+      const double ptx[4] = {1.0, sh.pg[0][t], sh.pg[1][t], sh.pg[2][t]};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) gam[i] = 0.0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gam[i] = gam[i] + ptx[j] * A[i + 4 * j];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) sh.A[q][t] = A[q];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sh.pg[q][t] = gam[q];
+    }
   }
   __syncthreads();
   if (!active || lane == 0) return 0;
-  double A[16];
-#pragma unroll
-  for (int q = 0; q < 16; ++q) A[q] = shA[q];
-  int info = lu_inverse<4>(A);
-  if (info) return info;
-  double ptx[4] = {1.0, pos[0], pos[1], pos[2]}, gam[4], dg[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) gam[i] = 0.0;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    double t = 1.0 * ptx[j];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) gam[i] = gam[i] + t * A[i + 4 * j];
-  }
+  if (const int info = sh.info[slot]) return info;
   const int d = lane - 1;
-  double pv[4];
+  double gam[4], pv[4], dg[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) pv[i] = i == d + 1 ? 1.0 : 0.0;   // unit vector e_(d+1), in registers
+  for (int i = 0; i < 4; ++i) { gam[i] = sh.pg[i][slot]; pv[i] = i == d + 1 ? 1.0 : 0.0; }   // unit vector e_(d+1), in registers
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     double t = -1.0 * gam[j];
@@ -228,37 +258,43 @@ __device__ __forceinline__ int mls_grad_lanes(const Grid& g, const R* __restrict
 #pragma unroll
   for (int i = 0; i < 4; ++i) dg[i] = 0.0;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    double t = 1.0 * pv[j];
+  for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dg[i] = dg[i] + t * A[i + 4 * j];
+    for (int i = 0; i < 4; ++i) dg[i] = dg[i] + pv[j] * sh.A[i + 4 * j][slot];
+  const double(*fx)[64] = lane == 1 ? sh.dw : sh.w;
+  const double(*fy)[64] = lane == 2 ? sh.dw : sh.w;
+  const double(*fz)[64] = lane == 3 ? sh.dw : sh.w;
+  double xs[3], ys[3], w1[3], w2[3], f1[3], f2[3];
+  int ci[3] = {0, 0, 0}, cj[3] = {0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    xs[q] = sh.crd[q][slot]; ys[q] = sh.crd[3 + q][slot];
+    w1[q] = sh.w[q][slot]; w2[q] = sh.w[3 + q][slot];
+    f1[q] = fx[q][slot]; f2[q] = fy[3 + q][slot];
+    if (!COEF) { ci[q] = pmod(ic - 2 + q, g.n1); cj[q] = pmod(jc - 2 + q, g.n2); }
   }
   double s = 0.0;
 #pragma unroll 1
   for (int nk = 0; nk < 3; ++nk) {
-    const double zk = nk == 0 ? zs[0] : nk == 1 ? zs[1] : zs[2];
-    const double w3k = nk == 0 ? w3[0] : nk == 1 ? w3[1] : w3[2];
-    const double dw3k = nk == 0 ? dw3[0] : nk == 1 ? dw3[1] : dw3[2];
-    const int kk = nk == 0 ? ke0 : nk == 1 ? ke1 : ke2;
+    const double zk = sh.crd[6 + nk][slot], w3k = sh.w[6 + nk][slot], f3 = fz[6 + nk][slot];
+    const int kk = COEF ? 0 : pmod((nk == 0 ? ke[0] : nk == 1 ? ke[1] : ke[2]) - 1, g.n3);
 #pragma unroll
-    for (int jq = 0; jq < 3; ++jq)
+    for (int jq = 0; jq < 3; ++jq) {
+      const R* line = COEF ? nullptr : fld + cidx(g, 0, cj[jq], kk);
 #pragma unroll
       for (int iq = 0; iq < 3; ++iq) {
         double wtx = w1[iq] * (w2[jq] * w3k);
         double p[4] = {1.0, xs[iq], ys[jq], zk};
-        double dw = d == 0 ? dw1[iq] * w2[jq] * w3k : d == 1 ? w1[iq] * dw2[jq] * w3k : w1[iq] * w2[jq] * dw3k;
+        double dw = f1[iq] * f2[jq] * f3;
         double acc = 0.0;
 #pragma unroll
-        for (int l = 0; l < 4; ++l) acc = acc + (1.0 * (wtx * p[l])) * dg[l];
+        for (int l = 0; l < 4; ++l) acc = acc + (wtx * p[l]) * dg[l];
 #pragma unroll
-        for (int l = 0; l < 4; ++l) acc = acc + (1.0 * (dw * p[l])) * gam[l];
-        if (coef) {   // geometry only: the point's shape-function derivative
-          coef[(size_t)(9 * nk + 3 * jq + iq) * cstride] = acc;
-        } else {
-          double val = fld[widx(g, ic - 1 + iq, jc - 1 + jq, kk)];
-          s = s + acc * val;
-        }
+        for (int l = 0; l < 4; ++l) acc = acc + (dw * p[l]) * gam[l];
+        if constexpr (COEF) coef[(size_t)(9 * nk + 3 * jq + iq) * cstride] = acc;   // geometry only
+        else s = s + acc * (double)line[ci[iq]];
       }
+    }
   }
   *grad_d = s;
   return 0;
@@ -905,12 +941,6 @@ __global__ __launch_bounds__(64) void k_mls_weights(Grid g, const double* __rest
 constexpr int FORCE_CELLS = 1024;   // table of k_mls_force: 20 KiB of LDS
 constexpr int FORCE_FACES = 64;     // faces per block, at most
 
-// Order the LDS accesses of one wave (its lanes run in step).
-__device__ inline void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 template <typename R>
 struct ForceArgs {
   const R* fld[4];        // vx, vy, temp, vz
@@ -1195,18 +1225,18 @@ __device__ inline double* probe_out(double* out, int f, int kind, int d) {
 
 // Gradient probes: kinds 0/1 (temperature, fluid/solid side), 3 (pressure),
 // 4/5/6 (u, v, w); item = kind slot x nf + face, 4 lanes per item.  With
-// coef (the fused substep) only the geometry part runs: lane 1+d stores the
+// COEF (the fused substep) only the geometry part runs: lane 1+d stores the
 // 27 shape-function derivatives of component d at coef[q * 3 nitems + 3 item
 // + d], and k_probes_apply later sums them against the field in the same
 // order; without it the lanes sum against the field directly.  Either way
 // the values round as in the single-thread formulation.
-// With ppw (and coef) the blocks from gradient block count nblk on store the pressure
+// With ppw (and COEF) the blocks from gradient block count nblk on store the pressure
 // interpolation's 27 shape functions of one face per thread at ppw[q nf + f].
-template <typename R>
+template <bool COEF, typename R>
 __global__ __launch_bounds__(256) void k_probes_grad(Grid g, ProbeArgs<R> P, double* __restrict__ out, int* __restrict__ pind, int klo,
                                                      int nkinds, double* __restrict__ coef, double* __restrict__ ppw, int nblk, int* err) {
-  __shared__ double shA[64][16];
-  if ((int)blockIdx.x >= nblk) {
+  __shared__ GradShared sh;
+  if (COEF && (int)blockIdx.x >= nblk) {
     const int f = ((int)blockIdx.x - nblk) * 256 + (int)threadIdx.x;
     if (f >= P.nf || P.gf[f]) return;
     int icent, jcent, kw;
@@ -1214,12 +1244,12 @@ __global__ __launch_bounds__(256) void k_probes_grad(Grid g, ProbeArgs<R> P, dou
     return;
   }
   const int id = blockIdx.x * blockDim.x + threadIdx.x;
-  const int item = id >> 2, lane = id & 3, slot = threadIdx.x >> 2;
+  const int item = id >> 2, lane = id & 3;
   const int nitem = P.nf * nkinds;   // with coef: items over the coefficient slots
   const bool inrange = item < nitem;
   const int f = inrange ? item % P.nf : 0;
   const int q = inrange ? item / P.nf : 0;
-  const int kind = coef ? coef_kind(q, P.heat, P.loads) : grad_kind(klo + q);
+  const int kind = COEF ? coef_kind(q, P.heat, P.loads) : grad_kind(klo + q);
   const bool active = inrange && !P.gf[f];
   ProbeSite<R> S;
   S.pos[0] = S.pos[1] = S.pos[2] = 0.0;
@@ -1228,15 +1258,15 @@ __global__ __launch_bounds__(256) void k_probes_grad(Grid g, ProbeArgs<R> P, dou
   S.fld = P.temp;
   if (active) {
     probe_site(g, P, f, kind, S);
-    if (!coef && kind <= 1 && lane == 0) { int* pi = &pind[6 * f + 3 * kind]; pi[0] = S.icent; pi[1] = S.jcent; pi[2] = S.kw; }
+    if (!COEF && kind <= 1 && lane == 0) { int* pi = &pind[6 * f + 3 * kind]; pi[0] = S.icent; pi[1] = S.jcent; pi[2] = S.kw; }
   }
   double gd = 0.0;
   const size_t cs = (size_t)3 * nitem;
-  double* cf = coef && lane > 0 ? coef + (size_t)3 * item + (lane - 1) : nullptr;
-  int info = mls_grad_lanes(g, S.fld, S.pos, S.ic, S.jc, S.kz, S.ke, S.cc, lane, active, shA[slot], &gd, cf, cs);
+  double* cf = COEF && lane > 0 ? coef + (size_t)3 * item + (lane - 1) : nullptr;
+  int info = mls_grad_lanes<COEF>(g, sh, S.fld, S.pos, S.ic, S.jc, S.kz, S.ke, S.cc, lane, active, &gd, cf, cs);
   if (!active || lane == 0) return;
   if (info) { raise_error(err, MELT_ERR_SINGULAR_MLS); return; }
-  if (!coef) *probe_out(out, f, kind, lane - 1) = gd;
+  if (!COEF) *probe_out(out, f, kind, lane - 1) = gd;
 }
 
 // The field part of the probes of the fused substep: one thread per (item,
@@ -1642,7 +1672,7 @@ static int ibm_probe_coefs_t(melt_ctx* ctx) {
   const int ncoef = probe_coef_slots(P);
   if (khi > klo) {
     const int ngrad = (int)nb((size_t)ctx->nf * ncoef * 4, 256), npr = P.loads ? (int)nb(ctx->nf, 256) : 0;
-    hipLaunchKernelGGL(k_probes_grad<R>, dim3(ngrad + npr), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, ctx->d_pind,
+    hipLaunchKernelGGL((k_probes_grad<true, R>), dim3(ngrad + npr), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, ctx->d_pind,
                        klo, ncoef, ctx->d_pcoef, probe_ppw(ctx, P), ngrad, ctx->d_err);
   }
   MELT_HIP(hipGetLastError());
@@ -1660,7 +1690,7 @@ static int ibm_probes_t(melt_ctx* ctx, int* pind_out, bool coefs_ready) {
                        ctx->d_probe, pind, klo, khi - klo, probe_coef_slots(P));
   } else if (khi > klo) {
     const int ngrad = (int)nb((size_t)ctx->nf * (khi - klo) * 4, 256);
-    hipLaunchKernelGGL(k_probes_grad<R>, dim3(ngrad), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, pind, klo, khi - klo, nullptr,
+    hipLaunchKernelGGL((k_probes_grad<false, R>), dim3(ngrad), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, pind, klo, khi - klo, nullptr,
                        nullptr, ngrad, ctx->d_err);
     if (P.loads)
       hipLaunchKernelGGL(k_probes_point<R>, dim3(nb(ctx->nf, 64)), dim3(64), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, ctx->d_err);

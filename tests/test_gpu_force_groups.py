@@ -12,7 +12,7 @@ import pytest
 import oracle
 from melt_ibm_amd import geometry
 from melt_ibm_amd.api import MeltContext
-from tests.helpers import load_state, make_cfg, random_state
+from tests.helpers import load_state, make_cfg, random_state, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +64,30 @@ def test_tags_over_group_sizes_and_orders(gpu_lib, freq, order):
         c.close()
     for name, a, b in zip(("sdf", "VOFp"), *out):
         assert np.array_equal(a, b), (name, int((a != b).sum()))
+
+
+def test_probes_of_a_body_across_the_corner(gpu_lib):
+    """180 faces (a last, incomplete group of 64 probes) around the corner of the
+    periodic box, where the stencils wrap in all three directions: heat fluxes
+    and loads of one particle call.  The probes keep the oracle's order of
+    operations on fields whose forces were added in another order (1e-16); a
+    gradient over cells and a cancelling sum over faces take that to 1e-13 or
+    so: 1e-10, as for the whole particle step."""
+    cfg = make_cfg(32)
+    st = random_state(cfg, 8)
+    mesh = geometry.icosphere(3)
+    out = []
+    for c in (MeltContext(cfg, lib=gpu_lib), oracle.context(cfg)):
+        c.set_geometry(mesh.xyz, mesh.vert_of_edge, mesh.edge_of_face, 1.2)
+        centre = np.array(c.body().pos_cm[:])
+        for q in ("xyzv", "tri_bar"):
+            c.set_lag(q, c.lag(q) - centre)
+        load_state(c, st)
+        c.set_dt(0.002)
+        c.set_stage(1)
+        c.particle()
+        b = c.body().as_dict()
+        out.append({**{q: c.lag(q) for q in ("qw_oVert", "qw_iVert")}, **{q: np.atleast_1d(b[q]) for q in ("int_prn_dA", "int_tau_dA")}})
+        c.close()
+    for q, w in out[1].items():
+        assert np.abs(w).max() > 0 and rel_err(out[0][q], w) <= 1e-10, q
