@@ -658,9 +658,18 @@ extern "C" int melt_particle(melt_ctx* ctx) {
 // queued on the main stream so far; side_join makes the main stream wait for
 // it.  Fork and join are stream events, so a captured step keeps them as
 // graph dependencies.
-// Tuning key streams = 1 keeps all work on the main stream (many contexts
-// sharing one GPU get their concurrency from each other).
-static bool one_stream(const melt_ctx* ctx) { return ctx->tune[TUNE_STREAMS] == 1; }
+// Tuning key streams: 1 keeps all work on the main stream (many contexts
+// sharing one GPU get their concurrency from each other), 2 uses the side
+// streams, 0 (built in) the main stream alone up to 64^3 cells unless the step is
+// replayed as a graph.  There the substep's 26 launches take no longer than the
+// events of its forks and joins (eager, one against several streams, 10 steps:
+// 32^3 4.4 / 5.0 ms in FP64, 4.5 / 5.9 in FP32, 64^3 with 1280 faces 5.5 / 5.9 and
+// 5.3 / 5.6, with 5120 6.1 / 6.1; 96^3 8.4 / 8.2 and 7.4 / 7.2); a graph's edges
+// cost less (64^3 5.6 / 5.2).
+static bool one_stream(const melt_ctx* ctx) {
+  const int t = ctx->tune[TUNE_STREAMS];
+  return t == 1 || (t == 0 && !ctx->use_graph && ctx->nc <= (size_t)64 * 64 * 64);
+}
 // Where the geometry stage of the gradient probes runs: 1 = queued on the side
 // stream after the previous substep's Lagrangian update and next tagging
 // (beside the pressure solve), 2 = on the side stream at the start of the
