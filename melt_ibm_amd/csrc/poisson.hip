@@ -648,8 +648,15 @@ __global__ __launch_bounds__(rf_threads(P, Q, RF_NC), P * Q == 512 ? 2 : 1) void
 }
 
 // Line pairs per block of the x passes: about 128 threads, and 2 NPB lines that
-// divide N (the passes have n1 = n2).
-constexpr int x_pairs(int N) { return N == 64 ? 16 : N == 512 ? 4 : 8; }
+// divide N (the passes have n1 = n2).  256 points take 16 pairs, whose rows j+1
+// the divergence reads once more per 32 lines instead of 16 (forward, FP64 125 ->
+// 107 us, FP32 84 -> 70; at 192 16 pairs are slower, 40 -> 44 in FP32, at 128 and 384
+// the same).
+constexpr int x_pairs(int N) { return N == 64 || N == 256 ? 16 : N == 512 ? 4 : 8; }
+// Waves per SIMD the forward x pass asks for: 384 points in FP64 take 172 registers
+// by themselves, four above what three waves leave (486 -> 400 us).
+template <typename T>
+constexpr int x_fwd_waves(int N) { return sizeof(T) == 8 && N == 384 ? 3 : 1; }
 
 // x pass, forward, with register FFTs (N1 = P*Q): thread (c, b) of stage A owns
 // line pair c of the block (lines j, j+1 packed as real and imaginary part,
@@ -657,7 +664,7 @@ constexpr int x_pairs(int N) { return N == 64 ? 16 : N == 512 ? 4 : 8; }
 // transform the two half spectra are separated with the mirror bins N-m,
 // exchanged through LDS.
 template <typename Rf, typename T, int P, int Q>
-__global__ __launch_bounds__(rf_threads(P, Q, x_pairs(P * Q))) void k_fft_x_fwd_reg(
+__global__ __launch_bounds__(rf_threads(P, Q, x_pairs(P * Q)), x_fwd_waves<T>(P * Q)) void k_fft_x_fwd_reg(
     SpecArgs<T> S, const cx<T>* __restrict__ tw, const Rf* __restrict__ vx, const Rf* __restrict__ vy, const Rf* __restrict__ vz,
     const Rf* __restrict__ src, T usdtal, const int* __restrict__ gate, unsigned long long* __restrict__ div_slots) {
   if (gate && *gate == 0) return;
