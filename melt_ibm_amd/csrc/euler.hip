@@ -1362,16 +1362,25 @@ int launch_explicit_xsolve(melt_ctx* ctx, double bxu, double bxt) {
     // against 1547, but 128^3 49 against 48 and 192^3 (one and a half waves) 178
     // against 152
     const bool pair = sizeof(R) == 4 && ctx->tune[TUNE_XF_ONE] == 0 && ctx->n1 % 128 == 0 && ctx->n1 >= 256;
+    // A CU takes three waves of this kernel per SIMD, and a block only where every
+    // SIMD has room for its share rounded up: of six-wave blocks (384 cells) one,
+    // half the waves.  Two rows per block make twelve waves, three per SIMD
+    // (384^3 FP64 3197 -> 2637 us; 9.5 GB, 2000 us at the rate of a copy).
+    const int rows = (ctx->n1 / 64) % 4 == 2 && ctx->n1 > 256 && ctx->n2 % 2 == 0 && 2 * zshm <= ctx->lds_max && !pair ? 2 : 1;
     const size_t lines = (size_t)ctx->n2 * ctx->n3 * (pair ? ctx->n1 / 128 : ctx->n1 / 64);   // waves at one plane each
     int D = zd;
     if (D <= 0 || ctx->n3 % D) {
       // planes per block: as many as leave 8192 waves, about 2.7 rounds of what the
       // chip holds (128^3 FP64, 8 / 4 / 2 planes: 97 / 87 / 86 us; 256^3: 645 / 657 /
       // 673); the two-cell form 8 from twice the work of 256^3 on, else 4 (384^3 1114 /
-      // 1157, 256^3 336 / 333)
+      // 1157, 256^3 336 / 333); blocks of two rows, one to a CU, as many as leave six
+      // rounds (384^3 FP64, 8 / 24 / 48 / 64 planes: 2613 / 2543 / 2522 / 2703)
       D = 1;
+      if (rows == 2)
+        for (int d : {48, 32, 24, 16, 12})
+          if (D == 1 && ctx->n3 % d == 0 && (size_t)(ctx->n2 / 2) * (ctx->n3 / d) >= 6 * 256) D = d;
       for (int d : {8, 4, 2})
-        if (ctx->n3 % d == 0 && lines / d >= (pair && d == 8 ? 32768 : 8192)) { D = d; break; }
+        if (D == 1 && ctx->n3 % d == 0 && lines / d >= (pair && d == 8 ? 32768 : 8192)) D = d;
       if (D == 1 && ctx->n3 % 2 == 0) D = 2;
     }
     if constexpr (std::is_same_v<R, float>) {
@@ -1384,11 +1393,6 @@ int launch_explicit_xsolve(melt_ctx* ctx, double bxu, double bxt) {
         return 0;
       }
     }
-    // A CU takes three waves of this kernel per SIMD, and a block only where every
-    // SIMD has room for its share rounded up: of six-wave blocks (384 cells) one,
-    // half the waves.  Two rows per block make twelve waves, three per SIMD
-    // (384^3 FP64 3197 -> 2637 us; 9.5 GB, 2000 us at the rate of a copy).
-    const int rows = (ctx->n1 / 64) % 4 == 2 && ctx->n1 > 256 && ctx->n2 % 2 == 0 && 2 * zshm <= ctx->lds_max ? 2 : 1;
     const dim3 grid((unsigned)((size_t)(ctx->n2 / rows) * (ctx->n3 / D))), block(ctx->n1, rows);
 #define ZM_LAUNCH(ROWS)                                                                                                                    \
   hipLaunchKernelGGL((k_explicit_zmarch<R, ROWS>), grid, block, rows * zshm, ctx->stream, A, cf, fld<R>(ctx, MELT_RU1),                     \
