@@ -336,8 +336,8 @@ int melt_graph_enable(melt_ctx* ctx, int32_t on);
  * block (8 or 16) of the pass that does the y and z solves together, 1 there
  * = two separate passes, 6 = streams: 1 keeps all of the context's work on its
  * one stream (for many contexts sharing a GPU), 2 runs the Lagrangian update,
- * probes and next tagging on two more (default: 1 up to 64^3 cells unless
- * steps are replayed as graphs, else 2), 7 = where the geometry
+ * probes and next tagging on two more (default: 1 up to 64^3 cells, else
+ * 2), 7 = where the geometry
  * stage of the gradient probes runs: 1 after the previous substep's Lagrangian
  * update (beside the pressure solve), 2 at the start of its own substep
  * (beside the explicit pass), 8 = faces a ray-tagging pencil may hold

@@ -660,15 +660,15 @@ extern "C" int melt_particle(melt_ctx* ctx) {
 // graph dependencies.
 // Tuning key streams: 1 keeps all work on the main stream (many contexts
 // sharing one GPU get their concurrency from each other), 2 uses the side
-// streams, 0 (built in) the main stream alone up to 64^3 cells unless the step is
-// replayed as a graph.  There the substep's 26 launches take no longer than the
-// events of its forks and joins (eager, one against several streams, 10 steps:
-// 32^3 4.4 / 5.0 ms in FP64, 4.5 / 5.9 in FP32, 64^3 with 1280 faces 5.5 / 5.9 and
-// 5.3 / 5.6, with 5120 6.1 / 6.1; 96^3 8.4 / 8.2 and 7.4 / 7.2); a graph's edges
-// cost less (64^3 5.6 / 5.2).
+// streams, 0 (built in) the main stream alone up to 64^3 cells.  There a substep's
+// launches take no longer than the events (or a graph's edges) of its forks and
+// joins add (10 steps, one against several streams, eager / as a graph: 32^3 FP64 4.0
+// / 3.7 ms against 5.6 / 4.4; 64^3 with 1280 faces 5.0 / 5.1 against 6.0 / 5.3, with
+// 5120 5.7 / 5.8 against 6.2 / 5.8; 96^3 with 2880 8.1 / 8.2 against 8.2 / 7.9, with
+// 11520 9.4 / 9.4 against 9.2 / 9.2; FP32 alike).
 static bool one_stream(const melt_ctx* ctx) {
   const int t = ctx->tune[TUNE_STREAMS];
-  return t == 1 || (t == 0 && !ctx->use_graph && ctx->nc <= (size_t)64 * 64 * 64);
+  return t == 1 || (t == 0 && ctx->nc <= (size_t)64 * 64 * 64);
 }
 // Where the geometry stage of the gradient probes runs: 1 = queued on the side
 // stream after the previous substep's Lagrangian update and next tagging
@@ -788,10 +788,15 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
   if (moving && ctx->tag_ahead) {
     ctx->force_window_from_tag = 1;   // placed by the tagging queued last substep
   } else if (moving) {
+    // the shape functions share the tagging's launch; so does, on one stream, the
+    // probes' geometry part (else it runs beside the explicit pass)
+    const bool wgt = c.tagtype != 0 && !ctx->weights_ahead, coef = wgt && one_stream(ctx) && !ctx->coef_ahead;
     timing_begin(ctx, SLOT_TAG, &e);
     ctx->force_window_from_tag = 1;
-    rc = ibm_tag(ctx);
+    rc = ibm_tag(ctx, wgt, coef);
     if (rc) { ctx->force_window_from_tag = 0; return rc; }
+    if (wgt) ctx->weights_ahead = 1;
+    if (coef) ctx->coef_ahead = 1;
     timing_end(ctx, SLOT_TAG, e);
   }
   ctx->tag_ahead = 0;
@@ -958,7 +963,9 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
 extern "C" int melt_substep(melt_ctx* ctx, int32_t ns) {
   if (check_ctx(ctx)) return MELT_ERR_ARG;
   if (ctx->graph_uses_ahead) graph_drop(ctx);
-  return substep_impl(ctx, ns, false, false);
+  const int rc = substep_impl(ctx, ns, false, false);
+  if (rc) ctx->coef_ahead = ctx->weights_ahead = 0;
+  return rc;
 }
 
 static int tschem_launch(melt_ctx* ctx) {

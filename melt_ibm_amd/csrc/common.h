@@ -516,7 +516,9 @@ int poisson_init(melt_ctx* ctx);
 // divgck) into those REDUCE_SLOTS slots.
 int poisson_solve(melt_ctx* ctx, int fused_divg, const int* gate = nullptr, unsigned long long* div_slots = nullptr);
 int euler_fold_slots(melt_ctx* ctx, unsigned long long* slots, unsigned long long* out, int used = REDUCE_SLOTS);
-int ibm_tag(melt_ctx* ctx);
+// Not with tagType 0: wgt also does ibm_weights(ctx, true), and coef with it
+// ibm_probe_coefs, in one launch with the band's distances.
+int ibm_tag(melt_ctx* ctx, bool wgt = false, bool coef = false);
 int ibm_find_centroid_indices(melt_ctx* ctx);
 int ibm_weights(melt_ctx* ctx, bool find = false);   // find: form the cell indices too
 int ibm_force_scatter(melt_ctx* ctx);

@@ -569,42 +569,51 @@ struct TagGroup {
   __device__ int capacity() const { return nface * 125 / 2; }
 };
 
+template <int FPB, int CELLS>
+struct BandShared {
+  CellTable<CELLS> tab;
+  unsigned long long kmin[CELLS];
+  int fmin[CELLS];
+  TriEdges tri[FPB];
+  double crd[FPB][15];   // the band's x, y and z (a division each)
+  int base[FPB][3];
+  bool alive[FPB];
+  int used, full;
+};
+struct BandArgs {
+  const melt_window* __restrict__ win;
+  Win3 et;
+  unsigned long long* __restrict__ key;
+  double* __restrict__ dst;
+};
+
 template <int FPB, int T, int CELLS>
-__global__ __launch_bounds__(T) void k_tag_band(Grid g, MeshArgs M, const melt_window* __restrict__ win, Win3 et,
-                                                unsigned long long* __restrict__ key, double* __restrict__ dst, int* err) {
+__device__ void tag_band_block(const Grid& g, const MeshArgs& M, const BandArgs& B, BandShared<FPB, CELLS>& sh, int group, int* err) {
   constexpr int E = (FPB * 125 + T - 1) / T;   // entries per thread
-  __shared__ CellTable<CELLS> tab;
-  __shared__ unsigned long long kmin[CELLS];
-  __shared__ int fmin[CELLS];
-  __shared__ TriEdges tri[FPB];
-  __shared__ double crd[FPB][15];   // the band's x, y and z (a division each)
-  __shared__ int base[FPB][3];
-  __shared__ bool alive[FPB];
-  __shared__ int used, full;
-  const TagGroup<FPB> G(dst, M.nf, blockIdx.x);
+  const TagGroup<FPB> G(B.dst, M.nf, group);
   const int t = threadIdx.x, n = G.nface * 125;
   if (t < FPB) {
     const int f = G.f0 + t;
     const bool live = t < G.nface && !M.gf[f];
-    alive[t] = live;
+    sh.alive[t] = live;
     if (live) {
       const int* v = &M.vof[3 * f];
-      tri[t] = tri_edges(&M.xyzv[3 * v[0]], &M.xyzv[3 * v[1]], &M.xyzv[3 * v[2]]);
+      sh.tri[t] = tri_edges(&M.xyzv[3 * v[0]], &M.xyzv[3 * v[1]], &M.xyzv[3 * v[2]]);
     }
   }
   for (int u = t; u < G.nface * 15; u += T) {
     const int r = u / 15, m = u - 15 * r, d = m / 5, o = m - 5 * d;
     const double x = M.bar[3 * (G.f0 + r) + d];
     const int i0 = (int)floor(x * (d == 0 ? g.dx1 : d == 1 ? g.dx2 : g.dx3)) + 1, i = i0 + o - 2;
-    crd[r][m] = d == 0 ? gxm(g, i) : d == 1 ? gym(g, i) : gzm(g, i);
-    if (o == 0) base[r][d] = i0;
+    sh.crd[r][m] = d == 0 ? gxm(g, i) : d == 1 ? gym(g, i) : gzm(g, i);
+    if (o == 0) sh.base[r][d] = i0;
   }
-  for (int q = t; q < CELLS; q += T) { tab.cell[q] = -1; kmin[q] = ~0ull; fmin[q] = INT_MAX; }
-  if (t == 0) { used = 0; full = 0; }
+  for (int q = t; q < CELLS; q += T) { sh.tab.cell[q] = -1; sh.kmin[q] = ~0ull; sh.fmin[q] = INT_MAX; }
+  if (t == 0) { sh.used = 0; sh.full = 0; }
   __syncthreads();
   int org[3];
 #pragma unroll
-  for (int d = 0; d < 3; ++d) org[d] = win[0].bmin[d] - 2;
+  for (int d = 0; d < 3; ++d) org[d] = B.win[0].bmin[d] - 2;
   unsigned long long dk[E];
   int cell[E], slot[E];
 #pragma unroll
@@ -612,51 +621,57 @@ __global__ __launch_bounds__(T) void k_tag_band(Grid g, MeshArgs M, const melt_w
     const int id = t + e * T, r = id / 125, q = id - 125 * r;
     cell[e] = slot[e] = -1;
     dk[e] = 0ull;
-    if (id >= n || !alive[r]) continue;
+    if (id >= n || !sh.alive[r]) continue;
     const int oi = q % 5, oj = (q / 5) % 5, ok = q / 25;
-    const long long s = win_slot(org, et.e, base[r][0] + oi - 2, base[r][1] + oj - 2, base[r][2] + ok - 2);
+    const long long s = win_slot(org, B.et.e, sh.base[r][0] + oi - 2, sh.base[r][1] + oj - 2, sh.base[r][2] + ok - 2);
     if (s < 0) { raise_error(err, MELT_ERR_WINDOW); continue; }
-    const double P[3] = {crd[r][oi], crd[r][5 + oj], crd[r][10 + ok]};
-    dk[e] = (unsigned long long)__double_as_longlong(dist_point_tri(P, tri[r]));
+    const double P[3] = {sh.crd[r][oi], sh.crd[r][5 + oj], sh.crd[r][10 + ok]};
+    dk[e] = (unsigned long long)__double_as_longlong(dist_point_tri(P, sh.tri[r]));
     cell[e] = (int)s;   // window cells are below 2^30
-    slot[e] = tab.slot((int)s);
-    if (slot[e] >= 0) atomicMin(&kmin[slot[e]], dk[e]);
-    else full = 1;
+    slot[e] = sh.tab.slot((int)s);
+    if (slot[e] >= 0) atomicMin(&sh.kmin[slot[e]], dk[e]);
+    else sh.full = 1;
   }
   __syncthreads();
 #pragma unroll
   for (int e = 0; e < E; ++e)
-    if (slot[e] >= 0 && kmin[slot[e]] == dk[e]) atomicMin(&fmin[slot[e]], G.f0 + (t + e * T) / 125);
+    if (slot[e] >= 0 && sh.kmin[slot[e]] == dk[e]) atomicMin(&sh.fmin[slot[e]], G.f0 + (t + e * T) / 125);
   for (int q0 = 0; q0 < CELLS; q0 += T) {
-    const unsigned long long m = __ballot(tab.cell[q0 + t] >= 0);
-    if ((t & 63) == 0 && m) atomicAdd(&used, (int)__popcll(m));
+    const unsigned long long m = __ballot(sh.tab.cell[q0 + t] >= 0);
+    if ((t & 63) == 0 && m) atomicAdd(&sh.used, (int)__popcll(m));
   }
   __syncthreads();
-  const int count = used;
-  if (full || count > G.capacity()) {
+  const int count = sh.used;
+  if (sh.full || count > G.capacity()) {
     if (t == 0) *G.count = -1;
 #pragma unroll
     for (int e = 0; e < E; ++e)
       if (cell[e] >= 0) {
         G.dist[t + e * T] = __longlong_as_double((long long)dk[e]);
-        atomicMin(&key[cell[e]], dk[e]);
+        atomicMin(&B.key[cell[e]], dk[e]);
       }
     return;
   }
   __syncthreads();
-  if (t == 0) { *G.count = count; used = 0; }
+  if (t == 0) { *G.count = count; sh.used = 0; }
   __syncthreads();
   for (int q0 = 0; q0 < CELLS; q0 += T) {
-    const int q = q0 + t, c = tab.cell[q];
+    const int q = q0 + t, c = sh.tab.cell[q];
     const unsigned long long m = __ballot(c >= 0);
     int at = 0;
-    if ((t & 63) == 0 && m) at = atomicAdd(&used, (int)__popcll(m));
+    if ((t & 63) == 0 && m) at = atomicAdd(&sh.used, (int)__popcll(m));
     at = __shfl(at, 0, 64) + (int)__popcll(m & ((1ull << (t & 63)) - 1ull));
     if (c >= 0) {
-      G.records()[at] = TagRecord{kmin[q], c, fmin[q]};
-      atomicMin(&key[c], kmin[q]);
+      G.records()[at] = TagRecord{sh.kmin[q], c, sh.fmin[q]};
+      atomicMin(&B.key[c], sh.kmin[q]);
     }
   }
+}
+
+template <int FPB, int T, int CELLS>
+__global__ __launch_bounds__(T) void k_tag_band(Grid g, MeshArgs M, BandArgs B, int* err) {
+  __shared__ BandShared<FPB, CELLS> sh;
+  tag_band_block<FPB, T, CELLS>(g, M, B, sh, blockIdx.x, err);
 }
 
 template <int MODE, int FPB, typename R>
@@ -911,9 +926,8 @@ struct PhiOut { double* q[4]; };  // ptxAB_q1, ptxAB_q2, ptxAB_temp, ptxAB_q3
 // With find, the face's cell indices are formed here as k_centroid_idx
 // forms them (findCentroidIndices.f90:16-48) and component 0 stores them;
 // otherwise they are read from pind.
-__global__ __launch_bounds__(64) void k_mls_weights(Grid g, const double* __restrict__ bar, const unsigned char* __restrict__ gf, int nf,
-                                                    int* __restrict__ pind, int find, PhiOut out, int* err) {
-  int id = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void mls_weights_item(const Grid& g, const double* __restrict__ bar, const unsigned char* __restrict__ gf, int nf,
+                                                 int* __restrict__ pind, int find, const PhiOut& out, int id, int* err) {
   if (id >= nf * 4) return;
   int f = id >> 2, comp = id & 3;
   if (gf[f]) return;
@@ -936,6 +950,11 @@ __global__ __launch_bounds__(64) void k_mls_weights(Grid g, const double* __rest
   else { i0 = p[0] - 1; j0 = p[1] - 1; k0 = kst - 1; c[0] = 1; c[1] = 1; c[2] = 0; }
   double* o = &out.q[comp][27 * (size_t)f];
   if (mls_phi(g, pos, i0, j0, k0, c, [&](int q, double v) { o[q] = v; })) raise_error(err, MELT_ERR_SINGULAR_MLS);
+}
+
+__global__ __launch_bounds__(64) void k_mls_weights(Grid g, const double* __restrict__ bar, const unsigned char* __restrict__ gf, int nf,
+                                                    int* __restrict__ pind, int find, PhiOut out, int* err) {
+  mls_weights_item(g, bar, gf, nf, pind, find, out, blockIdx.x * blockDim.x + threadIdx.x, err);
 }
 
 constexpr int FORCE_CELLS = 1024;   // table of k_mls_force: 20 KiB of LDS
@@ -1232,18 +1251,32 @@ __device__ inline double* probe_out(double* out, int f, int kind, int d) {
 // the values round as in the single-thread formulation.
 // With ppw (and COEF) the blocks from gradient block count nblk on store the pressure
 // interpolation's 27 shape functions of one face per thread at ppw[q nf + f].
+template <typename R>
+struct GradArgs {
+  ProbeArgs<R> P;
+  double* __restrict__ out;
+  int* __restrict__ pind;
+  int klo, nkinds;
+  double* __restrict__ coef;
+  double* __restrict__ ppw;
+  int nblk;
+};
 template <bool COEF, typename R>
-__global__ __launch_bounds__(256) void k_probes_grad(Grid g, ProbeArgs<R> P, double* __restrict__ out, int* __restrict__ pind, int klo,
-                                                     int nkinds, double* __restrict__ coef, double* __restrict__ ppw, int nblk, int* err) {
-  __shared__ GradShared sh;
-  if (COEF && (int)blockIdx.x >= nblk) {
-    const int f = ((int)blockIdx.x - nblk) * 256 + (int)threadIdx.x;
+__device__ __forceinline__ void probes_grad_block(const Grid& g, const GradArgs<R>& Q, GradShared& sh, int block, int* err) {
+  const ProbeArgs<R>& P = Q.P;
+  double* __restrict__ out = Q.out;
+  int* __restrict__ pind = Q.pind;
+  double* __restrict__ coef = Q.coef;
+  double* __restrict__ ppw = Q.ppw;
+  const int klo = Q.klo, nkinds = Q.nkinds, nblk = Q.nblk;
+  if (COEF && block >= nblk) {
+    const int f = (block - nblk) * 256 + (int)threadIdx.x;
     if (f >= P.nf || P.gf[f]) return;
     int icent, jcent, kw;
     if (pressure_phi(g, P, f, icent, jcent, kw, [&](int q, double phi) { ppw[(size_t)q * P.nf + f] = phi; })) raise_error(err, MELT_ERR_SINGULAR_MLS);
     return;
   }
-  const int id = blockIdx.x * blockDim.x + threadIdx.x;
+  const int id = block * 256 + (int)threadIdx.x;
   const int item = id >> 2, lane = id & 3;
   const int nitem = P.nf * nkinds;   // with coef: items over the coefficient slots
   const bool inrange = item < nitem;
@@ -1267,6 +1300,27 @@ __global__ __launch_bounds__(256) void k_probes_grad(Grid g, ProbeArgs<R> P, dou
   if (!active || lane == 0) return;
   if (info) { raise_error(err, MELT_ERR_SINGULAR_MLS); return; }
   if (!COEF) *probe_out(out, f, kind, lane - 1) = gd;
+}
+template <bool COEF, typename R>
+__global__ __launch_bounds__(256) void k_probes_grad(Grid g, GradArgs<R> Q, int* err) {
+  __shared__ GradShared sh;
+  probes_grad_block<COEF, R>(g, Q, sh, blockIdx.x, err);
+}
+
+// What the coming substep needs of the moved faces, in one launch: the band
+// distances of the tagging (as k_tag_band), the forcing's cell indices and
+// shape functions (k_mls_weights) and the probes' geometry part
+// (k_probes_grad).  On one stream each of the three would leave most of a small
+// mesh's chip idle for its own latency: 1280 faces 7 + 10 + 13 us apart, 15 together.
+template <int FPB, int CELLS, typename R>
+__global__ __launch_bounds__(256) void k_faces_next(Grid g, MeshArgs M, BandArgs B, GradArgs<R> Q, int ngrad, int nwgt, int* __restrict__ pind,
+                                                    PhiOut phi, int* err) {
+  constexpr size_t bytes = sizeof(GradShared) > sizeof(BandShared<FPB, CELLS>) ? sizeof(GradShared) : sizeof(BandShared<FPB, CELLS>);
+  __shared__ __align__(16) unsigned char mem[bytes];
+  const int b = blockIdx.x;
+  if (b < ngrad) probes_grad_block<true, R>(g, Q, *reinterpret_cast<GradShared*>(mem), b, err);
+  else if (b < ngrad + nwgt) mls_weights_item(g, M.bar, M.gf, M.nf, pind, 1, phi, (b - ngrad) * 256 + (int)threadIdx.x, err);
+  else tag_band_block<FPB, 256, CELLS>(g, M, B, *reinterpret_cast<BandShared<FPB, CELLS>*>(mem), b - ngrad - nwgt, err);
 }
 
 // The field part of the probes of the fused substep: one thread per (item,
@@ -1487,7 +1541,42 @@ static int ray_tag_init_t(melt_ctx* ctx) {
 }
 
 template <typename R>
-static int ibm_tag_t(melt_ctx* ctx) {  // tagCells.f90:4-27 (tagType 1) + interp_vof when not fused
+static ProbeArgs<R> probe_args(melt_ctx* ctx) {
+  ProbeArgs<R> P;
+  P.temp = fld<R>(ctx, MELT_TEMP); P.pr = fld<R>(ctx, MELT_PR); P.vx = fld<R>(ctx, MELT_VX); P.vy = fld<R>(ctx, MELT_VY); P.vz = fld<R>(ctx, MELT_VZ);
+  P.bar = ctx->d_lag[MELT_L_TRI_BAR]; P.nor = ctx->d_lag[MELT_L_TRI_NOR]; P.gf = ctx->d_gf; P.nf = ctx->nf;
+  P.h = ctx->h_body.h_eulerian; P.pec = ctx->cfg.ren * ctx->cfg.prandtl;
+  P.heat = ctx->cfg.imelt == 1;
+  P.loads = ctx->cfg.imlsstr == 1;
+  return P;
+}
+
+template <typename R>
+static int probe_coef_slots(const ProbeArgs<R>& P) { return P.heat && P.loads ? 5 : P.heat ? 2 : P.loads ? 4 : 0; }
+
+// Where the pressure probe's shape functions sit in d_pcoef (27 x 18 doubles per
+// face): behind the gradient slots (27 x 15 at most).
+template <typename R>
+static double* probe_ppw(melt_ctx* ctx, const ProbeArgs<R>& P) {
+  return P.loads ? ctx->d_pcoef + (size_t)27 * 3 * probe_coef_slots(P) * ctx->nf : nullptr;
+}
+
+// The geometry part of the probes: its arguments, and its blocks (0: no probes).
+template <typename R>
+static GradArgs<R> coef_args(melt_ctx* ctx, int* blocks) {
+  const ProbeArgs<R> P = probe_args<R>(ctx);
+  const int klo = P.heat ? 0 : 2, khi = P.loads ? 6 : 2, ncoef = probe_coef_slots(P);
+  const int ngrad = (int)nb((size_t)ctx->nf * ncoef * 4, 256), npr = P.loads ? (int)nb(ctx->nf, 256) : 0;
+  *blocks = khi > klo ? ngrad + npr : 0;
+  return {P, ctx->d_probe, ctx->d_pind, klo, ncoef, ctx->d_pcoef, probe_ppw(ctx, P), ngrad};
+}
+
+static PhiOut phi_out(melt_ctx* ctx) {
+  return {{ctx->d_lag[MELT_L_PTXAB_Q1], ctx->d_lag[MELT_L_PTXAB_Q2], ctx->d_lag[MELT_L_PTXAB_TEMP], ctx->d_lag[MELT_L_PTXAB_Q3]}};
+}
+
+template <typename R>
+static int ibm_tag_t(melt_ctx* ctx, bool wgt, bool coef) {  // tagCells.f90:4-27 (tagType 1) + interp_vof when not fused
   if (!ctx->has_geom) return melt_fail(ctx, MELT_ERR_NO_GEOMETRY, "tagCells", "no geometry");
   if (ctx->cfg.tagtype == 0) return sphere_tag_t<R>(ctx);
   Grid g = make_grid(ctx);
@@ -1506,14 +1595,22 @@ static int ibm_tag_t(melt_ctx* ctx) {  // tagCells.f90:4-27 (tagType 1) + interp
   // faces do not move between tagging and forcing)
   const int which = ctx->force_window_from_tag ? 3 : 2;
   MeshArgs M = mesh_args(ctx);
+  const BandArgs B{ctx->d_win, et, ctx->d_tkey, ctx->d_tdist};
+  int ngrad = 0;
+  const GradArgs<R> Q = coef_args<R>(ctx, &ngrad);
+  const int nwgt = (int)nb((size_t)ctx->nf * 4, 256);
+  if (!coef) ngrad = 0;
 #define TAG_PASSES(FPB, T, CELLS)                                                                                                       \
   do {                                                                                                                                  \
-    const dim3 groups(nb(ctx->nf, FPB));                                                                                                \
-    hipLaunchKernelGGL((k_tag_band<FPB, T, CELLS>), groups, dim3(T), 0, ctx->stream, g, M, ctx->d_win, et, ctx->d_tkey, ctx->d_tdist,    \
-                       ctx->d_err);                                                                                                     \
-    hipLaunchKernelGGL((k_tag_pass<1, FPB, R>), groups, dim3(256), 0, ctx->stream, g, M, ctx->d_win, ef, et, which, ctx->d_tkey,         \
+    const unsigned groups = nb(ctx->nf, FPB);                                                                                           \
+    if (wgt)                                                                                                                            \
+      hipLaunchKernelGGL((k_faces_next<FPB, CELLS, R>), dim3(ngrad + nwgt + groups), dim3(256), 0, ctx->stream, g, M, B, Q, ngrad, nwgt, \
+                         ctx->d_pind, phi_out(ctx), ctx->d_err);                                                                        \
+    else                                                                                                                                \
+      hipLaunchKernelGGL((k_tag_band<FPB, T, CELLS>), dim3(groups), dim3(T), 0, ctx->stream, g, M, B, ctx->d_err);                       \
+    hipLaunchKernelGGL((k_tag_pass<1, FPB, R>), dim3(groups), dim3(256), 0, ctx->stream, g, M, ctx->d_win, ef, et, which, ctx->d_tkey,   \
                        ctx->d_tface, ctx->d_tdist, fld<R>(ctx, MELT_SDF), fld<R>(ctx, MELT_VOFP), ctx->pi, ctx->d_err);                  \
-    hipLaunchKernelGGL((k_tag_pass<2, FPB, R>), groups, dim3(256), 0, ctx->stream, g, M, ctx->d_win, ef, et, which, ctx->d_tkey,         \
+    hipLaunchKernelGGL((k_tag_pass<2, FPB, R>), dim3(groups), dim3(256), 0, ctx->stream, g, M, ctx->d_win, ef, et, which, ctx->d_tkey,   \
                        ctx->d_tface, ctx->d_tdist, fld<R>(ctx, MELT_SDF), fld<R>(ctx, MELT_VOFP), ctx->pi, ctx->d_err);                  \
   } while (0)
   // As many faces a group as keep the chip's blocks busy (20480 faces on 128^3:
@@ -1536,7 +1633,7 @@ int ibm_find_centroid_indices(melt_ctx* ctx) {
 }
 
 int ibm_weights(melt_ctx* ctx, bool find) {
-  PhiOut o{{ctx->d_lag[MELT_L_PTXAB_Q1], ctx->d_lag[MELT_L_PTXAB_Q2], ctx->d_lag[MELT_L_PTXAB_TEMP], ctx->d_lag[MELT_L_PTXAB_Q3]}};
+  const PhiOut o = phi_out(ctx);
   hipLaunchKernelGGL(k_mls_weights, dim3(nb((size_t)ctx->nf * 4, 64)), dim3(64), 0, ctx->stream, make_grid(ctx), ctx->d_lag[MELT_L_TRI_BAR],
                      ctx->d_gf, ctx->nf, ctx->d_pind, find ? 1 : 0, o, ctx->d_err);
   MELT_HIP(hipGetLastError());
@@ -1641,40 +1738,14 @@ static int ibm_tempforce_t(melt_ctx* ctx) {  // tempforce.f90
   return 0;
 }
 
-template <typename R>
-static ProbeArgs<R> probe_args(melt_ctx* ctx) {
-  ProbeArgs<R> P;
-  P.temp = fld<R>(ctx, MELT_TEMP); P.pr = fld<R>(ctx, MELT_PR); P.vx = fld<R>(ctx, MELT_VX); P.vy = fld<R>(ctx, MELT_VY); P.vz = fld<R>(ctx, MELT_VZ);
-  P.bar = ctx->d_lag[MELT_L_TRI_BAR]; P.nor = ctx->d_lag[MELT_L_TRI_NOR]; P.gf = ctx->d_gf; P.nf = ctx->nf;
-  P.h = ctx->h_body.h_eulerian; P.pec = ctx->cfg.ren * ctx->cfg.prandtl;
-  P.heat = ctx->cfg.imelt == 1;
-  P.loads = ctx->cfg.imlsstr == 1;
-  return P;
-}
-
-template <typename R>
-static int probe_coef_slots(const ProbeArgs<R>& P) { return P.heat && P.loads ? 5 : P.heat ? 2 : P.loads ? 4 : 0; }
-
-// Where the pressure probe's shape functions sit in d_pcoef (27 x 18 doubles per
-// face): behind the gradient slots (27 x 15 at most).
-template <typename R>
-static double* probe_ppw(melt_ctx* ctx, const ProbeArgs<R>& P) {
-  return P.loads ? ctx->d_pcoef + (size_t)27 * 3 * probe_coef_slots(P) * ctx->nf : nullptr;
-}
-
 // The geometry part of the probes (shape-function derivatives and the pressure
 // probe's shape functions into d_pcoef): reads only the faces and the grid, so
 // the fused substep runs it beside the explicit pass.
 template <typename R>
 static int ibm_probe_coefs_t(melt_ctx* ctx) {
-  ProbeArgs<R> P = probe_args<R>(ctx);
-  int klo = P.heat ? 0 : 2, khi = P.loads ? 6 : 2;
-  const int ncoef = probe_coef_slots(P);
-  if (khi > klo) {
-    const int ngrad = (int)nb((size_t)ctx->nf * ncoef * 4, 256), npr = P.loads ? (int)nb(ctx->nf, 256) : 0;
-    hipLaunchKernelGGL((k_probes_grad<true, R>), dim3(ngrad + npr), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, ctx->d_pind,
-                       klo, ncoef, ctx->d_pcoef, probe_ppw(ctx, P), ngrad, ctx->d_err);
-  }
+  int blocks = 0;
+  const GradArgs<R> Q = coef_args<R>(ctx, &blocks);
+  if (blocks) hipLaunchKernelGGL((k_probes_grad<true, R>), dim3(blocks), dim3(256), 0, ctx->stream, make_grid(ctx), Q, ctx->d_err);
   MELT_HIP(hipGetLastError());
   return 0;
 }
@@ -1690,8 +1761,8 @@ static int ibm_probes_t(melt_ctx* ctx, int* pind_out, bool coefs_ready) {
                        ctx->d_probe, pind, klo, khi - klo, probe_coef_slots(P));
   } else if (khi > klo) {
     const int ngrad = (int)nb((size_t)ctx->nf * (khi - klo) * 4, 256);
-    hipLaunchKernelGGL((k_probes_grad<false, R>), dim3(ngrad), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, pind, klo, khi - klo, nullptr,
-                       nullptr, ngrad, ctx->d_err);
+    const GradArgs<R> Q{P, ctx->d_probe, pind, klo, khi - klo, nullptr, nullptr, ngrad};
+    hipLaunchKernelGGL((k_probes_grad<false, R>), dim3(ngrad), dim3(256), 0, ctx->stream, make_grid(ctx), Q, ctx->d_err);
     if (P.loads)
       hipLaunchKernelGGL(k_probes_point<R>, dim3(nb(ctx->nf, 64)), dim3(64), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, ctx->d_err);
   }
@@ -1706,7 +1777,7 @@ int ibm_window_reset(melt_ctx* ctx) {
 }
 
 // ------------------------------------------------- precision dispatch
-int ibm_tag(melt_ctx* ctx) { return ctx->fp32 ? ibm_tag_t<float>(ctx) : ibm_tag_t<double>(ctx); }
+int ibm_tag(melt_ctx* ctx, bool wgt, bool coef) { return ctx->fp32 ? ibm_tag_t<float>(ctx, wgt, coef) : ibm_tag_t<double>(ctx, wgt, coef); }
 int ibm_force_scatter(melt_ctx* ctx) { return ctx->fp32 ? ibm_force_scatter_t<float>(ctx) : ibm_force_scatter_t<double>(ctx); }
 int ibm_force_drain(melt_ctx* ctx, int apply_now) { return ctx->fp32 ? ibm_force_drain_t<float>(ctx, apply_now) : ibm_force_drain_t<double>(ctx, apply_now); }
 int ibm_sub_mean(melt_ctx* ctx) { return ctx->fp32 ? ibm_sub_mean_t<float>(ctx) : ibm_sub_mean_t<double>(ctx); }

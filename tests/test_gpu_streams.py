@@ -1,6 +1,6 @@
 """One stream or several: a step's results do not depend on it.  A small grid
-takes one stream by itself unless its step is replayed as a graph; switching
-between the two mid-run (graph on and off) keeps the bits as well."""
+takes one by itself; replaying some of the steps as graphs keeps the bits as
+well."""
 import numpy as np
 import pytest
 
