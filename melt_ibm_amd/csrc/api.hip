@@ -152,7 +152,7 @@ extern "C" void melt_ctx_destroy(melt_ctx* ctx) {
   for (auto e : ctx->ev_pool) hipEventDestroy(e);
   if (ctx->side) hipStreamSynchronize(ctx->side);
   if (ctx->side2) hipStreamSynchronize(ctx->side2);
-  for (hipEvent_t e : {ctx->ev_fork, ctx->ev_join, ctx->ev_fork2, ctx->ev_join2, ctx->ev_forc, ctx->ev_hit}) if (e) hipEventDestroy(e);
+  for (hipEvent_t e : {ctx->ev_fork, ctx->ev_join, ctx->ev_fork2, ctx->ev_join2, ctx->ev_forc, ctx->ev_hit, ctx->ev_coef}) if (e) hipEventDestroy(e);
   if (ctx->side) hipStreamDestroy(ctx->side);
   if (ctx->side2) hipStreamDestroy(ctx->side2);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
@@ -215,7 +215,8 @@ extern "C" int melt_ctx_create(const melt_config* cfg, melt_ctx** out) {
         hipEventCreateWithFlags(&ctx->ev_fork2, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&ctx->ev_join2, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&ctx->ev_forc, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&ctx->ev_hit, hipEventDisableTiming) != hipSuccess) {
+        hipEventCreateWithFlags(&ctx->ev_hit, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&ctx->ev_coef, hipEventDisableTiming) != hipSuccess) {
       rc = MELT_ERR_HIP;
       break;
     }
@@ -805,7 +806,15 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
   // since the last Lagrangian update) and the grid: queued with the tagging
   // ahead of time, else on the side stream beside the explicit pass
   const bool probes = ibm && (c.imelt == 1 || c.imlsstr == 1);
-  if (probes && !ctx->coef_ahead && (rc = side_run(ctx, [&] { return ibm_probe_coefs(ctx); }))) return rc;
+  // queued on the side stream, the coefficients are waited for by what reads them
+  auto side_coefs = [&]() -> int {
+    int r = ibm_probe_coefs(ctx);
+    if (r || one_stream(ctx)) return r;
+    MELT_HIP(hipEventRecord(ctx->ev_coef, ctx->stream));
+    ctx->coef_pending = 1;
+    return 0;
+  };
+  if (probes && !ctx->coef_ahead && (rc = side_run(ctx, side_coefs))) return rc;
   ctx->coef_ahead = 0;
 
   timing_begin(ctx, SLOT_PH_EULER, &e_ph);
@@ -856,15 +865,15 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
     return r;
   };
   const std::function<int()> tag_fork = [&]() -> int { return side2_run(ctx, tag_now); };
-  auto queue_coef = [&]() -> int {
-    int r = ibm_probe_coefs(ctx);
-    if (!r) ctx->coef_ahead = 1;
-    return r;
-  };
   // within a tschem call (tag_next) the main stream does not wait for the
   // probe geometry stage: only the next substep's probes read its output, and
   // they run on the side stream after it; the call's last substep joins it
   const bool coef_after_join = tag_next && coef_next && probes && !one_stream(ctx);
+  auto queue_coef = [&]() -> int {
+    int r = coef_after_join ? side_coefs() : ibm_probe_coefs(ctx);
+    if (!r) ctx->coef_ahead = 1;
+    return r;
+  };
   // within a tschem call the next substep's cell indices and shape functions
   // (they read only the refreshed faces; this substep's spreading is done with
   // them) are formed here too, off the path from its line solves to its forcing
@@ -882,13 +891,14 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
     timing_begin(ctx, SLOT_IBM, &e);
     if (!ctx->weights_ahead && (rc = ibm_weights(ctx, true))) return rc;   // cell indices and shape functions
     ctx->weights_ahead = 0;
-    // the gradient probes read the same pre-force fields as the spreading and
-    // write only their own outputs (their cell indices into d_pind2, since the
-    // spreading still reads d_pind): side stream, alongside the spreading
-    if ((rc = side_run(ctx, [&] { return ibm_probes(ctx, ctx->d_pind2, probes); }))) return rc;
-    rc = ibm_force_scatter(ctx);
+    // the field part of the probes reads the same pre-force fields as the spreading
+    // and writes only its own outputs (the cell indices into d_pind2, since the
+    // spreading still reads d_pind): one launch
+    if (ctx->coef_pending) MELT_HIP(hipStreamWaitEvent(ctx->stream, ctx->ev_coef, 0));
+    ctx->coef_pending = 0;
+    rc = ibm_force_scatter(ctx, probes);
     ctx->force_window_from_tag = 0;
-    if (rc || (rc = side_join(ctx)) || (rc = ibm_force_drain(ctx, 1))) return rc;
+    if (rc || (rc = ibm_force_drain(ctx, 1))) return rc;
     // The Lagrangian update after the forcing (loads, heat flux, Stefan
     // melting, Newton-Euler motion, remeshing, geometry refresh) reads only
     // the probe results and the body arrays, which the pressure phase does
@@ -964,7 +974,7 @@ extern "C" int melt_substep(melt_ctx* ctx, int32_t ns) {
   if (check_ctx(ctx)) return MELT_ERR_ARG;
   if (ctx->graph_uses_ahead) graph_drop(ctx);
   const int rc = substep_impl(ctx, ns, false, false);
-  if (rc) ctx->coef_ahead = ctx->weights_ahead = 0;
+  if (rc) ctx->coef_ahead = ctx->weights_ahead = ctx->coef_pending = 0;
   return rc;
 }
 
@@ -979,6 +989,7 @@ static int tschem_launch(melt_ctx* ctx) {
       ctx->tag_ahead = 0;
       ctx->coef_ahead = 0;
       ctx->weights_ahead = 0;
+      ctx->coef_pending = 0;
       if (ctx->graph_uses_ahead) graph_drop(ctx);
       return rc;
     }

@@ -85,6 +85,8 @@ struct melt_ctx {
   // after it touches the forcing, so melt_hit_force may run on side2 from
   // ev_forc on (the main stream then waits for ev_hit)
   hipEvent_t ev_forc = nullptr, ev_hit = nullptr;
+  hipEvent_t ev_coef = nullptr;   // behind the probe coefficients on the side stream, while coef_pending
+  int coef_pending = 0;
   int forc_free = 0;
   // graph replay of one RK3 step (melt_graph_enable): captured on first use,
   // dropped whenever a host-side launch parameter (dt, refinement) changes
@@ -521,7 +523,7 @@ int euler_fold_slots(melt_ctx* ctx, unsigned long long* slots, unsigned long lon
 int ibm_tag(melt_ctx* ctx, bool wgt = false, bool coef = false);
 int ibm_find_centroid_indices(melt_ctx* ctx);
 int ibm_weights(melt_ctx* ctx, bool find = false);   // find: form the cell indices too
-int ibm_force_scatter(melt_ctx* ctx);
+int ibm_force_scatter(melt_ctx* ctx, bool with_probes = false);
 int ibm_force_drain(melt_ctx* ctx, int apply_now);
 int ibm_force_mean(melt_ctx* ctx);   // of the forces the last ibm_force_drain(ctx, 1) applied, into d_fmean
 int ibm_sub_mean(melt_ctx* ctx);
@@ -529,8 +531,8 @@ int ibm_velforce(melt_ctx* ctx, int defer);
 int ibm_tempforce(melt_ctx* ctx);
 // pind_out: where the heat-flux probes' cell indices go (null: d_pind, as
 // mls_heatFlux does); lagr_after_force(ctx, true) copies d_pind2 into d_pind.
-int ibm_probes(melt_ctx* ctx, int* pind_out = nullptr, bool coefs_ready = false);
-// geometry part of the gradient probes into d_pcoef (then ibm_probes(..., true))
+int ibm_probes(melt_ctx* ctx);
+// geometry part of the gradient probes into d_pcoef (then ibm_force_scatter(ctx, true))
 int ibm_probe_coefs(melt_ctx* ctx);
 int ibm_window_reset(melt_ctx* ctx);
 // with commit_pind (the fused substep) it also commits the staged heat-flux probe indices.

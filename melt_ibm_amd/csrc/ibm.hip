@@ -967,6 +967,14 @@ struct ForceArgs {
   const double* vel_tri;
   const double* cfac;
   double tmelt;
+  const double* bar;
+  const unsigned char* gf;
+  int nf, fpb;   // fpb: faces per block
+  const int* pind;
+  const melt_window* win;
+  Win3 ef;
+  unsigned long long* acc;
+  size_t cells;
 };
 
 // forc1/forc2/forctemp/forc3 (forc1.f90:28-65): Um = sum q phi, spread
@@ -980,57 +988,58 @@ struct ForceArgs {
 // face and cell, 38 with a table whose every cell hashes by itself (16 of them the
 // flush, each update a transaction of its own), 27 with eight cells of a line
 // kept together.
+template <int T>
+struct ForceShared {
+  CellTable<FORCE_CELLS> tab;
+  unsigned long long sum[FORCE_CELLS][2];
+  alignas(16) double prods[T / 32][28];
+  int site[FORCE_FACES][6];       // centre of the stencil: wrapped, 0-based; from the window's origin
+  double face[FORCE_FACES][2];    // V, cfac
+  bool alive[FORCE_FACES];
+};
 template <typename R, int T>
-__global__ __launch_bounds__(T) void k_mls_force(Grid g, ForceArgs<R> F, const double* __restrict__ bar, const unsigned char* __restrict__ gf,
-                                                   int nf, int fpb, const int* __restrict__ pind, const melt_window* __restrict__ win, Win3 ef,
-                                                   unsigned long long* __restrict__ acc, size_t cells, int* err) {
-  __shared__ CellTable<FORCE_CELLS> tab;
-  __shared__ unsigned long long sum[FORCE_CELLS][2];
-  __shared__ __align__(16) double prods[T / 32][28];
-  __shared__ int site[FORCE_FACES][6];       // centre of the stencil: wrapped, 0-based; from the window's origin
-  __shared__ double face[FORCE_FACES][2];    // V, cfac
-  __shared__ bool alive[FORCE_FACES];
-  const int t = threadIdx.x, l = t & 31, comp = blockIdx.x & 3, f0 = (int)(blockIdx.x >> 2) * fpb;
-  if (t < fpb) {
+__device__ __forceinline__ void mls_force_block(const Grid& g, const ForceArgs<R>& F, ForceShared<T>& sh, int block, int* err) {
+  const int t = threadIdx.x, l = t & 31, comp = block & 3, f0 = (int)(block >> 2) * F.fpb;
+  if (t < F.fpb) {
     const int f = f0 + t;
-    const bool live = f < nf && !gf[f];
-    alive[t] = live;
+    const bool live = f < F.nf && !F.gf[f];
+    sh.alive[t] = live;
     if (live) {
-      const int* p = &pind[6 * f];
-      const double z = bar[3 * f + 2] * g.dx3;
+      const int* p = &F.pind[6 * f];
+      const double z = F.bar[3 * f + 2] * g.dx3;
       const int i0 = p[comp == 0 ? 3 : 0], j0 = p[comp == 1 ? 4 : 1], kw = p[comp == 3 ? 5 : 2];
       const int ku = comp == 3 ? fnint(z) + 1 : (int)floor(z) + 1;
-      site[t][0] = pmod(i0 - 1, g.n1); site[t][1] = pmod(j0 - 1, g.n2); site[t][2] = pmod(kw - 1, g.n3);
-      site[t][3] = i0 - win[0].org[0]; site[t][4] = j0 - win[0].org[1]; site[t][5] = ku - win[0].org[2];
-      face[t][0] = comp == 2 ? F.tmelt : F.vel_tri[3 * f + (comp == 3 ? 2 : comp)];
-      face[t][1] = F.cfac[f];
+      sh.site[t][0] = pmod(i0 - 1, g.n1); sh.site[t][1] = pmod(j0 - 1, g.n2); sh.site[t][2] = pmod(kw - 1, g.n3);
+      sh.site[t][3] = i0 - F.win[0].org[0]; sh.site[t][4] = j0 - F.win[0].org[1]; sh.site[t][5] = ku - F.win[0].org[2];
+      sh.face[t][0] = comp == 2 ? F.tmelt : F.vel_tri[3 * f + (comp == 3 ? 2 : comp)];
+      sh.face[t][1] = F.cfac[f];
     }
   }
-  for (int q = t; q < FORCE_CELLS; q += T) { tab.cell[q] = -1; sum[q][0] = 0ull; sum[q][1] = 0ull; }
+  for (int q = t; q < FORCE_CELLS; q += T) { sh.tab.cell[q] = -1; sh.sum[q][0] = 0ull; sh.sum[q][1] = 0ull; }
   __syncthreads();
-  unsigned long long* const out = acc + (size_t)comp * cells * 2;
+  unsigned long long* const out = F.acc + (size_t)comp * F.cells * 2;
   const R* __restrict__ fld = F.fld[comp];
   const double* __restrict__ phi = F.phi[comp];
   const int di = l % 3 - 1, dj = (l / 3) % 3 - 1, dk = l / 9 - 1;
-  double* const pr = prods[t >> 5];
+  double* const pr = sh.prods[t >> 5];
   auto wrap = [](int i, int n) { return i < 0 ? i + n : i >= n ? i - n : i; };
   // the loads of the next face are in flight while this one is summed
   auto load = [&](int r, double& ph, R& val) {
     ph = 0.0;
     val = R(0);
-    if (r >= fpb || l >= 27 || !alive[r]) return;
-    const int* st = site[r];
+    if (r >= F.fpb || l >= 27 || !sh.alive[r]) return;
+    const int* st = sh.site[r];
     ph = phi[27 * (size_t)(f0 + r) + l];
     val = fld[wrap(st[0] + di, g.n1) + g.n1 * (wrap(st[1] + dj, g.n2) + g.n2 * wrap(st[2] + dk, g.n3))];
   };
   double ph_next;
   R val_next;
   load(t >> 5, ph_next, val_next);
-  for (int r = t >> 5; r < fpb; r += T / 32) {
+  for (int r = t >> 5; r < F.fpb; r += T / 32) {
     const double ph = ph_next;
     const R val = val_next;
     load(r + T / 32, ph_next, val_next);
-    if (!alive[r]) continue;   // all 32 lanes alike
+    if (!sh.alive[r]) continue;   // all 32 lanes alike
     if (l < 27) pr[l] = (double)val * ph;
     wave_lds_fence();
     double Um = 0.0;
@@ -1038,16 +1047,21 @@ __global__ __launch_bounds__(T) void k_mls_force(Grid g, ForceArgs<R> F, const d
     for (int q = 0; q < 27; ++q) Um = Um + pr[q];
     wave_lds_fence();
     if (l >= 27) continue;
-    const double v = face[r][1] * (face[r][0] - Um) * ph;
-    const int a = site[r][3] + di, b = site[r][4] + dj, c = site[r][5] + dk;
-    if (a < 0 || b < 0 || c < 0 || a >= ef.e[0] || b >= ef.e[1] || c >= ef.e[2]) { raise_error(err, MELT_ERR_WINDOW); continue; }
-    const int sl = a + ef.e[0] * (b + ef.e[1] * c);   // window cells are below 2^30
-    const int h = tab.slot(sl);
-    acc_add(h >= 0 ? sum[h] : &out[(size_t)sl * 2], v);
+    const double v = sh.face[r][1] * (sh.face[r][0] - Um) * ph;
+    const int a = sh.site[r][3] + di, b = sh.site[r][4] + dj, c = sh.site[r][5] + dk;
+    if (a < 0 || b < 0 || c < 0 || a >= F.ef.e[0] || b >= F.ef.e[1] || c >= F.ef.e[2]) { raise_error(err, MELT_ERR_WINDOW); continue; }
+    const int sl = a + F.ef.e[0] * (b + F.ef.e[1] * c);   // window cells are below 2^30
+    const int h = sh.tab.slot(sl);
+    acc_add(h >= 0 ? sh.sum[h] : &out[(size_t)sl * 2], v);
   }
   __syncthreads();
   for (int q = threadIdx.x; q < FORCE_CELLS; q += T)
-    if (tab.cell[q] >= 0) acc_add_split(&out[(size_t)tab.cell[q] * 2], sum[q][0], sum[q][1]);
+    if (sh.tab.cell[q] >= 0) acc_add_split(&out[(size_t)sh.tab.cell[q] * 2], sh.sum[q][0], sh.sum[q][1]);
+}
+template <typename R, int T>
+__global__ __launch_bounds__(T) void k_mls_force(Grid g, ForceArgs<R> F, int* err) {
+  __shared__ ForceShared<T> sh;
+  mls_force_block<R, T>(g, F, sh, blockIdx.x, err);
 }
 
 // Drain the accumulators: mode 0 adds the forces to the fields (velocity
@@ -1246,7 +1260,7 @@ __device__ inline double* probe_out(double* out, int f, int kind, int d) {
 // 4/5/6 (u, v, w); item = kind slot x nf + face, 4 lanes per item.  With
 // COEF (the fused substep) only the geometry part runs: lane 1+d stores the
 // 27 shape-function derivatives of component d at coef[q * 3 nitems + 3 item
-// + d], and k_probes_apply later sums them against the field in the same
+// + d], and k_force_probes later sums them against the field in the same
 // order; without it the lanes sum against the field directly.  Either way
 // the values round as in the single-thread formulation.
 // With ppw (and COEF) the blocks from gradient block count nblk on store the pressure
@@ -1330,10 +1344,23 @@ __global__ __launch_bounds__(256) void k_faces_next(Grid g, MeshArgs M, BandArgs
 // stored shape functions of the pressure probe, whose moment matrix and
 // inverse (11 us of latency) thereby leave the path to the forcing.
 template <typename R>
-__global__ __launch_bounds__(256) void k_probes_apply(Grid g, ProbeArgs<R> P, const double* __restrict__ coef, const double* __restrict__ ppw,
-                                                      double* __restrict__ out, int* __restrict__ pind, int klo, int nkinds, int ncoef) {
+struct ApplyArgs {
+  ProbeArgs<R> P;
+  const double* __restrict__ coef;
+  const double* __restrict__ ppw;
+  double* __restrict__ out;
+  int* __restrict__ pind;
+  int klo, nkinds, ncoef;
+};
+template <typename R>
+__device__ __forceinline__ void probes_apply_item(const Grid& g, const ApplyArgs<R>& Q, int id) {
+  const ProbeArgs<R>& P = Q.P;
+  const double* __restrict__ coef = Q.coef;
+  const double* __restrict__ ppw = Q.ppw;
+  double* __restrict__ out = Q.out;
+  int* __restrict__ pind = Q.pind;
+  const int klo = Q.klo, nkinds = Q.nkinds, ncoef = Q.ncoef;
   const int nitem = P.nf * nkinds;
-  const int id = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (id >= 3 * nitem) {
     const int f = id - 3 * nitem;
     if (!ppw || f >= P.nf || P.gf[f]) return;
@@ -1370,6 +1397,16 @@ __global__ __launch_bounds__(256) void k_probes_apply(Grid g, ProbeArgs<R> P, co
       }
   }
   *probe_out(out, f, kind, d) = s;
+}
+
+// The forcing's spreading and the field part of the probes read the same
+// provisional fields and nothing of each other: blocks of one launch.
+template <typename R, int T>
+__global__ __launch_bounds__(T) void k_force_probes(Grid g, ForceArgs<R> F, ApplyArgs<R> Q, int nforce, int* err) {
+  __shared__ ForceShared<T> sh;
+  const int b = blockIdx.x;
+  if (b < nforce) mls_force_block<R, T>(g, F, sh, b, err);
+  else probes_apply_item<R>(g, Q, (b - nforce) * T + (int)threadIdx.x);
 }
 
 // Shape functions of the pressure interpolation probe (kind 2, wght_press) of
@@ -1571,6 +1608,18 @@ static GradArgs<R> coef_args(melt_ctx* ctx, int* blocks) {
   return {P, ctx->d_probe, ctx->d_pind, klo, ncoef, ctx->d_pcoef, probe_ppw(ctx, P), ngrad};
 }
 
+// The field part of the probes of the fused substep: its arguments and its threads.
+template <typename R>
+static ApplyArgs<R> apply_args(melt_ctx* ctx, int* pind) {
+  const ProbeArgs<R> P = probe_args<R>(ctx);
+  const int klo = P.heat ? 0 : 2, khi = P.loads ? 6 : 2;
+  return {P, ctx->d_pcoef, probe_ppw(ctx, P), ctx->d_probe, pind, klo, std::max(0, khi - klo), probe_coef_slots(P)};
+}
+template <typename R>
+static size_t apply_items(const ApplyArgs<R>& Q) {
+  return Q.nkinds ? (size_t)Q.P.nf * Q.nkinds * 3 + (Q.P.loads ? Q.P.nf : 0) : 0;
+}
+
 static PhiOut phi_out(melt_ctx* ctx) {
   return {{ctx->d_lag[MELT_L_PTXAB_Q1], ctx->d_lag[MELT_L_PTXAB_Q2], ctx->d_lag[MELT_L_PTXAB_TEMP], ctx->d_lag[MELT_L_PTXAB_Q3]}};
 }
@@ -1640,9 +1689,11 @@ int ibm_weights(melt_ctx* ctx, bool find) {
   return 0;
 }
 
-// Interpolation + spreading into the exact accumulators (mlsForce.f90, forc*).
+// Interpolation + spreading into the exact accumulators (mlsForce.f90, forc*);
+// with_probes (the fused substep, their coefficients ready): also the field part of
+// the gradient and pressure probes, their cell indices into pind2.
 template <typename R>
-static int ibm_force_scatter_t(melt_ctx* ctx) {
+static int ibm_force_scatter_t(melt_ctx* ctx, bool with_probes) {
   Grid g = make_grid(ctx);
   Win3 ef{{ctx->fwin[0], ctx->fwin[1], ctx->fwin[2]}}, et{{ctx->twin[0], ctx->twin[1], ctx->twin[2]}};
   if (!ctx->force_window_from_tag) {
@@ -1652,12 +1703,22 @@ static int ibm_force_scatter_t(melt_ctx* ctx) {
   }
   ForceArgs<R> F;
   F.fld[0] = fld<R>(ctx, MELT_VX); F.fld[1] = fld<R>(ctx, MELT_VY); F.fld[2] = fld<R>(ctx, MELT_TEMP); F.fld[3] = fld<R>(ctx, MELT_VZ);
-  F.phi[0] = ctx->d_lag[MELT_L_PTXAB_Q1]; F.phi[1] = ctx->d_lag[MELT_L_PTXAB_Q2];
-  F.phi[2] = ctx->d_lag[MELT_L_PTXAB_TEMP]; F.phi[3] = ctx->d_lag[MELT_L_PTXAB_Q3];
+  const PhiOut phi = phi_out(ctx);
+  for (int q = 0; q < 4; ++q) F.phi[q] = phi.q[q];
   F.vel_tri = ctx->d_lag[MELT_L_VEL_TRI]; F.cfac = ctx->d_lag[MELT_L_CFAC]; F.tmelt = ctx->cfg.tmelt;
+  F.bar = ctx->d_lag[MELT_L_TRI_BAR]; F.gf = ctx->d_gf; F.nf = ctx->nf; F.pind = ctx->d_pind;
+  F.win = ctx->d_win; F.ef = ef; F.acc = ctx->d_acc; F.cells = ctx->fwin_cells;
+  const ApplyArgs<R> Q = apply_args<R>(ctx, ctx->d_pind2);
+  const size_t items = with_probes ? apply_items(Q) : 0;
 #define MLS_FORCE(T, FPB)                                                                                                              \
-  hipLaunchKernelGGL((k_mls_force<R, T>), dim3(4 * nb(ctx->nf, FPB)), dim3(T), 0, ctx->stream, g, F, ctx->d_lag[MELT_L_TRI_BAR], ctx->d_gf, \
-                     ctx->nf, FPB, ctx->d_pind, ctx->d_win, ef, ctx->d_acc, ctx->fwin_cells, ctx->d_err)
+  do {                                                                                                                                 \
+    F.fpb = FPB;                                                                                                                       \
+    const unsigned nforce = 4 * nb(ctx->nf, FPB);                                                                                      \
+    if (items)                                                                                                                         \
+      hipLaunchKernelGGL((k_force_probes<R, T>), dim3(nforce + nb(items, T)), dim3(T), 0, ctx->stream, g, F, Q, (int)nforce, ctx->d_err); \
+    else                                                                                                                               \
+      hipLaunchKernelGGL((k_mls_force<R, T>), dim3(nforce), dim3(T), 0, ctx->stream, g, F, ctx->d_err);                                 \
+  } while (0)
   // Many faces: as many per block as share their cells best (20480 faces: 64
   // per block 27 us, 32 46, one update per face and cell 77).  Fewer faces: more
   // blocks and more faces at a time (1280 faces: 16 by 512 threads 6.7 us,
@@ -1750,18 +1811,14 @@ static int ibm_probe_coefs_t(melt_ctx* ctx) {
   return 0;
 }
 
+// The probes outside the fused substep: geometry and field part at once.
 template <typename R>
-static int ibm_probes_t(melt_ctx* ctx, int* pind_out, bool coefs_ready) {
+static int ibm_probes_t(melt_ctx* ctx) {
   ProbeArgs<R> P = probe_args<R>(ctx);
   int klo = P.heat ? 0 : 2, khi = P.loads ? 6 : 2;
-  int* pind = pind_out ? pind_out : ctx->d_pind;
-  if (khi > klo && coefs_ready) {
-    size_t threads = (size_t)ctx->nf * (khi - klo) * 3 + (P.loads ? ctx->nf : 0);
-    hipLaunchKernelGGL(k_probes_apply<R>, dim3(nb(threads, 256)), dim3(256), 0, ctx->stream, make_grid(ctx), P, ctx->d_pcoef, probe_ppw(ctx, P),
-                       ctx->d_probe, pind, klo, khi - klo, probe_coef_slots(P));
-  } else if (khi > klo) {
+  if (khi > klo) {
     const int ngrad = (int)nb((size_t)ctx->nf * (khi - klo) * 4, 256);
-    const GradArgs<R> Q{P, ctx->d_probe, pind, klo, khi - klo, nullptr, nullptr, ngrad};
+    const GradArgs<R> Q{P, ctx->d_probe, ctx->d_pind, klo, khi - klo, nullptr, nullptr, ngrad};
     hipLaunchKernelGGL((k_probes_grad<false, R>), dim3(ngrad), dim3(256), 0, ctx->stream, make_grid(ctx), Q, ctx->d_err);
     if (P.loads)
       hipLaunchKernelGGL(k_probes_point<R>, dim3(nb(ctx->nf, 64)), dim3(64), 0, ctx->stream, make_grid(ctx), P, ctx->d_probe, ctx->d_err);
@@ -1778,12 +1835,12 @@ int ibm_window_reset(melt_ctx* ctx) {
 
 // ------------------------------------------------- precision dispatch
 int ibm_tag(melt_ctx* ctx, bool wgt, bool coef) { return ctx->fp32 ? ibm_tag_t<float>(ctx, wgt, coef) : ibm_tag_t<double>(ctx, wgt, coef); }
-int ibm_force_scatter(melt_ctx* ctx) { return ctx->fp32 ? ibm_force_scatter_t<float>(ctx) : ibm_force_scatter_t<double>(ctx); }
+int ibm_force_scatter(melt_ctx* ctx, bool with_probes) {
+  return ctx->fp32 ? ibm_force_scatter_t<float>(ctx, with_probes) : ibm_force_scatter_t<double>(ctx, with_probes);
+}
 int ibm_force_drain(melt_ctx* ctx, int apply_now) { return ctx->fp32 ? ibm_force_drain_t<float>(ctx, apply_now) : ibm_force_drain_t<double>(ctx, apply_now); }
 int ibm_sub_mean(melt_ctx* ctx) { return ctx->fp32 ? ibm_sub_mean_t<float>(ctx) : ibm_sub_mean_t<double>(ctx); }
 int ibm_velforce(melt_ctx* ctx, int defer) { return ctx->fp32 ? ibm_velforce_t<float>(ctx, defer) : ibm_velforce_t<double>(ctx, defer); }
 int ibm_tempforce(melt_ctx* ctx) { return ctx->fp32 ? ibm_tempforce_t<float>(ctx) : ibm_tempforce_t<double>(ctx); }
-int ibm_probes(melt_ctx* ctx, int* pind_out, bool coefs_ready) {
-  return ctx->fp32 ? ibm_probes_t<float>(ctx, pind_out, coefs_ready) : ibm_probes_t<double>(ctx, pind_out, coefs_ready);
-}
+int ibm_probes(melt_ctx* ctx) { return ctx->fp32 ? ibm_probes_t<float>(ctx) : ibm_probes_t<double>(ctx); }
 int ibm_probe_coefs(melt_ctx* ctx) { return ctx->fp32 ? ibm_probe_coefs_t<float>(ctx) : ibm_probe_coefs_t<double>(ctx); }
