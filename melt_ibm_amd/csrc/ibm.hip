@@ -1721,10 +1721,11 @@ static int ibm_force_scatter_t(melt_ctx* ctx, bool with_probes) {
   } while (0)
   // Many faces: as many per block as share their cells best (20480 faces: 64
   // per block 27 us, 32 46, one update per face and cell 77).  Fewer faces: more
-  // blocks and more faces at a time (1280 faces: 16 by 512 threads 6.7 us,
-  // 8 by 256 8.1, 64 15.6; 5120 beside the probes: 32 by 512 15.7, 64 by 256 20.5).
+  // blocks (5120 faces with the probes: 32 by 256 threads 15 us, 16 24, 32 by 512, of
+  // which a CU holds two, 24), and more faces at a time (1280 faces alone: 16 by
+  // 512 threads 6.7 us, 8 by 256 8.1, 64 15.6).
   if (ctx->nf > 8192) MLS_FORCE(256, 64);
-  else if (ctx->nf > 2560) MLS_FORCE(512, 32);
+  else if (ctx->nf > 2560) MLS_FORCE(256, 32);
   else MLS_FORCE(512, 16);
 #undef MLS_FORCE
   MELT_HIP(hipGetLastError());
