@@ -135,6 +135,7 @@ struct melt_ctx {
   // through pinned memory, and the counters of melt_get_remesh_stats
   std::vector<int32_t> h_vof, h_eof, h_voe, h_foe, h_gv, h_ge, h_gf, h_anchor, h_flagged;
   double* d_xyz_melt = nullptr;
+  double* d_xold = nullptr;      // the vertices the rigid-body step starts from (scratch; without remeshing)
   int32_t* h_rm = nullptr;
   hipEvent_t ev_rm = nullptr;
   double remesh_stats[8] = {};

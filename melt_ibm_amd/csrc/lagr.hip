@@ -349,36 +349,71 @@ __global__ __launch_bounds__(256) void k_edge_len(LagArgs A, const double* __res
 
 __global__ void k_clear_rm(melt_body* b) { b->rm_flag = 0; }
 
+__device__ void mv3(const double* A, const double* x, double* y);
+
+// Relative vertex position against the centre of mass com before the
+// Newton-Euler step (RigidAuxRoutines.f90:20-35), and the vertex moved by its
+// rotation AA and new centre (update_xyz, :858-862).
+__device__ inline void move_vertex(const double* xold, const melt_body* __restrict__ b, const double* __restrict__ com,
+                                   const double* __restrict__ AA, double* rel_out, double* x) {
+  double rel[3], AT[9], u[3];
+  for (int d = 0; d < 3; ++d) rel[d] = xold[d] - com[d];
+  if (rel_out)
+    for (int d = 0; d < 3; ++d) rel_out[d] = rel[d];
+  for (int i = 0; i < 3; ++i) for (int j = 0; j < 3; ++j) AT[i + 3 * j] = AA[j + 3 * i];
+  mv3(AT, rel, u);
+  for (int d = 0; d < 3; ++d) x[d] = u[d] + b->pos_cm[d];
+}
+
 // calculate_area (triaux.f90:82-119), calc_centroids_from_vert (:308-323) and
 // update_tri_normal of every live face in one pass (the same expressions as
 // k_face_area and k_face_centroid_normal); thread 0 also clears the remesh
-// flag that k_edge_len then sets.  With vel, the face velocities too (as
-// k_face_vel, whose centroids are the same).
-__global__ __launch_bounds__(256) void k_face_geom(LagArgs A, const double* __restrict__ x, melt_body* b, int vel) {
+// flag that k_edge_len then sets.  With MOVE the rigid-body step itself too:
+// a face moves its own copies of its vertices (from xold, which nothing here
+// writes, so no launch has to separate the two), the vertices and relative
+// positions are stored by a thread each, and the faces get their velocities (as
+// k_rel_update and k_face_vel, whose centroids are the same): 4 + 5 us of launches
+// on the chain from the loads to the next tagging become 5.
+template <bool MOVE>
+__global__ __launch_bounds__(256) void k_face_geom(LagArgs A, const double* __restrict__ xold, melt_body* b, const double* __restrict__ com,
+                                                   const double* __restrict__ AA) {
   int f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f == 0) b->rm_flag = 0;
+  if (MOVE && f >= A.nf) {
+    const int v = f - A.nf;
+    if (v < A.nv && !A.gv[v]) move_vertex(&xold[3 * v], b, com, AA, &A.L[MELT_L_DXYZV_S][3 * v], &A.L[MELT_L_XYZV][3 * v]);
+    return;
+  }
   if (f >= A.nf || A.gf[f]) return;
-  int v[3] = {A.vof[3 * f], A.vof[3 * f + 1], A.vof[3 * f + 2]};
+  double x[3][3];
+  for (int k = 0; k < 3; ++k) {
+    const double* p = &xold[3 * A.vof[3 * f + k]];
+    if (MOVE) move_vertex(p, b, com, AA, nullptr, x[k]);
+    else
+      for (int d = 0; d < 3; ++d) x[k][d] = p[d];
+  }
   double dd[3];
   for (int e = 0; e < 3; ++e) {
-    int a = v[e], c = v[(e + 1) % 3];
-    double q0 = x[3 * a] - x[3 * c], q1 = x[3 * a + 1] - x[3 * c + 1], q2 = x[3 * a + 2] - x[3 * c + 2];
+    const double *a = x[e], *c = x[(e + 1) % 3];
+    double q0 = a[0] - c[0], q1 = a[1] - c[1], q2 = a[2] - c[2];
     dd[e] = sqrt(q0 * q0 + q1 * q1 + q2 * q2);
   }
   double sp = (dd[0] + dd[1] + dd[2]) / 2.;
   A.L[MELT_L_SUR][f] = sqrt(sp * (sp - dd[0]) * (sp - dd[1]) * (sp - dd[2]));
-  const int v1 = v[0], v2 = v[1], v3 = v[2];
-  for (int d = 0; d < 3; ++d) A.L[MELT_L_TRI_BAR][3 * f + d] = (A.L[MELT_L_XYZV][3 * v1 + d] + A.L[MELT_L_XYZV][3 * v2 + d] + A.L[MELT_L_XYZV][3 * v3 + d]) / 3.0;
+  double rel[3];
+  if (MOVE)
+    for (int d = 0; d < 3; ++d) A.L[MELT_L_DXYZ_S][3 * f + d] = rel[d] = A.L[MELT_L_TRI_BAR][3 * f + d] - com[d];
+  for (int d = 0; d < 3; ++d) A.L[MELT_L_TRI_BAR][3 * f + d] = (x[0][d] + x[1][d] + x[2][d]) / 3.0;
   double e1[3], e2[3], n[3];
-  for (int d = 0; d < 3; ++d) { e1[d] = x[3 * v2 + d] - x[3 * v1 + d]; e2[d] = x[3 * v3 + d] - x[3 * v1 + d]; }
+  for (int d = 0; d < 3; ++d) { e1[d] = x[1][d] - x[0][d]; e2[d] = x[2][d] - x[0][d]; }
   n[0] = e1[1] * e2[2] - e1[2] * e2[1];
   n[1] = e1[2] * e2[0] - e1[0] * e2[2];
   n[2] = e1[0] * e2[1] - e1[1] * e2[0];
   double s = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
   for (int d = 0; d < 3; ++d) A.L[MELT_L_TRI_NOR][3 * f + d] = n[d] / s;
-  if (vel) {
+  if (MOVE) {
     double om[3];
-    dcross(om, b->omega_c, &A.L[MELT_L_DXYZ_S][3 * f]);
+    dcross(om, b->omega_c, rel);
     for (int d = 0; d < 3; ++d) A.L[MELT_L_VEL_TRI][3 * f + d] = b->vel_cm[d] + om[d];
   }
 }
@@ -593,13 +628,19 @@ __device__ void newton_update(melt_body* b, double ga, double ro, double al, dou
 // [rigid 10], those present, quantity-major as in k_face_sums.
 template <bool L, bool V>
 __global__ __launch_bounds__(RB) void k_face_sums_motion(LagArgs A, const double* __restrict__ xyz, const double* __restrict__ rxp,
-                                                         const double* __restrict__ rxt, double* __restrict__ part) {
+                                                         const double* __restrict__ rxt, double* __restrict__ part, int G,
+                                                         double* __restrict__ xold) {
+  if ((int)blockIdx.x >= G) {
+    const int t = ((int)blockIdx.x - G) * RB + (int)threadIdx.x;
+    if (t < 3 * A.nv) xold[t] = xyz[t];
+    return;
+  }
   constexpr int QV = L ? 12 : 0, QG = QV + (V ? 1 : 0), NS = QG + (L ? 10 : 0);
   __shared__ double sm[NS][RB];
   double acc[NS];
 #pragma unroll
   for (int q = 0; q < NS; ++q) acc[q] = 0.0;
-  for (int f = blockIdx.x * RB + threadIdx.x; f < A.nf; f += gridDim.x * RB) {
+  for (int f = blockIdx.x * RB + threadIdx.x; f < A.nf; f += G * RB) {
     if (A.gf[f]) continue;
     if constexpr (L) {
       for (int d = 0; d < 3; ++d) {
@@ -627,7 +668,7 @@ __global__ __launch_bounds__(RB) void k_face_sums_motion(LagArgs A, const double
       for (int q = 0; q < NS; ++q) sm[q][threadIdx.x] = sm[q][threadIdx.x] + sm[q][threadIdx.x + w];
     __syncthreads();
   }
-  if ((int)threadIdx.x < NS) part[threadIdx.x * gridDim.x + blockIdx.x] = sm[threadIdx.x][0];
+  if ((int)threadIdx.x < NS) part[threadIdx.x * G + blockIdx.x] = sm[threadIdx.x][0];
 }
 
 // Stage 2 of k_face_sums_motion and the body updates that consume it, in the
@@ -654,22 +695,11 @@ __global__ __launch_bounds__(RB) void k_sum_motion(const double* __restrict__ pa
   }
 }
 
-// Relative vertex and face positions against the centre of mass com before
-// the Newton-Euler step (RigidAuxRoutines.f90:20-35), and the vertices moved
-// by its rotation AA and new centre (update_xyz, :858-862), in one pass.
 __global__ __launch_bounds__(256) void k_rel_update(LagArgs A, const melt_body* __restrict__ b, const double* __restrict__ com,
                                                     const double* __restrict__ AA) {
   int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < A.nv) {
-    if (A.gv[t]) return;
-    double* r = &A.L[MELT_L_DXYZV_S][3 * t];
-    double* x = &A.L[MELT_L_XYZV][3 * t];
-    double rel[3], AT[9], u[3];
-    for (int d = 0; d < 3; ++d) rel[d] = x[d] - com[d];
-    for (int d = 0; d < 3; ++d) r[d] = rel[d];
-    for (int i = 0; i < 3; ++i) for (int j = 0; j < 3; ++j) AT[i + 3 * j] = AA[j + 3 * i];
-    mv3(AT, rel, u);
-    for (int d = 0; d < 3; ++d) x[d] = u[d] + b->pos_cm[d];
+    if (!A.gv[t]) move_vertex(&A.L[MELT_L_XYZV][3 * t], b, com, AA, &A.L[MELT_L_DXYZV_S][3 * t], &A.L[MELT_L_XYZV][3 * t]);
   } else if (t < A.nv + A.nf) {
     int f = t - A.nv;
     if (!A.gf[f])
@@ -721,10 +751,14 @@ LagArgs lag_args(melt_ctx* ctx) {
 }
 
 // geometry refresh of particle.f90:163-193
-int refresh_geometry(melt_ctx* ctx, LagArgs& A, int vel = 0) {
+int refresh_geometry(melt_ctx* ctx, LagArgs& A, bool move = false) {
   const double* x = ctx->d_lag[MELT_L_XYZV];
   hipStream_t s = ctx->stream;
-  hipLaunchKernelGGL(k_face_geom, dim3(nb(ctx->nf, 256)), dim3(256), 0, s, A, x, ctx->d_body, vel);
+  if (move)
+    hipLaunchKernelGGL(k_face_geom<true>, dim3(nb((size_t)ctx->nf + ctx->nv, 256)), dim3(256), 0, s, A, ctx->d_xold, ctx->d_body, ctx->d_red + 48,
+                       ctx->d_red + 32);
+  else
+    hipLaunchKernelGGL(k_face_geom<false>, dim3(nb(ctx->nf, 256)), dim3(256), 0, s, A, x, ctx->d_body, nullptr, nullptr);
   // work that needs only the refreshed faces (the fused substep's next
   // tagging) forks here; the rest of the refresh does not touch what it reads
   if (const std::function<int()>* hook = ctx->after_faces) {
@@ -784,8 +818,9 @@ template <bool L, bool V>
 static void motion_sums(melt_ctx* ctx, const LagArgs& A) {
   const int G = std::max(1, std::min(64, (A.nf + RB - 1) / RB));
   double* part = ctx->d_red + 8192;
-  hipLaunchKernelGGL((k_face_sums_motion<L, V>), dim3(G), dim3(RB), 0, ctx->stream, A, ctx->d_lag[MELT_L_XYZV], ctx->d_rxp, ctx->d_rxt,
-                     part);
+  const unsigned copy = L && ctx->cfg.iremesh != 1 ? nb((size_t)3 * ctx->nv, RB) : 0;   // for k_face_geom<true>
+  hipLaunchKernelGGL((k_face_sums_motion<L, V>), dim3(G + copy), dim3(RB), 0, ctx->stream, A, ctx->d_lag[MELT_L_XYZV], ctx->d_rxp, ctx->d_rxt,
+                     part, G, ctx->d_xold);
   hipLaunchKernelGGL((k_sum_motion<L, V>), dim3(1), dim3(RB), 0, ctx->stream, part, G, ctx->d_red, ctx->d_body, ctx->cfg.dens_ratio, ctx->ga,
                      ctx->ro, ctx->al, ctx->dt, ctx->cfg.xlen, ctx->cfg.ylen, ctx->cfg.zlen, ctx->d_red + 32, ctx->d_red + 48, ctx->d_err);
 }
@@ -811,12 +846,12 @@ int lagr_after_force(melt_ctx* ctx, bool commit_pind) {
   if (loads && heat) motion_sums<true, true>(ctx, A);
   else if (loads) motion_sums<true, false>(ctx, A);
   else if (heat) motion_sums<false, true>(ctx, A);
-  if (loads) {
+  if (loads && ctx->cfg.iremesh == 1) {
     hipLaunchKernelGGL(k_rel_update, dim3(nb((size_t)ctx->nv + ctx->nf, 256)), dim3(256), 0, s, A, ctx->d_body, ctx->d_red + 48, ctx->d_red + 32);
-    if (ctx->cfg.iremesh == 1) hipLaunchKernelGGL(k_face_vel, dim3(nb(ctx->nf, 256)), dim3(256), 0, s, A, ctx->d_body);
+    hipLaunchKernelGGL(k_face_vel, dim3(nb(ctx->nf, 256)), dim3(256), 0, s, A, ctx->d_body);
   }
   MELT_HIP(hipGetLastError());
-  if (ctx->cfg.iremesh != 1) return refresh_geometry(ctx, A, loads);
+  if (ctx->cfg.iremesh != 1) return refresh_geometry(ctx, A, loads != 0);
   // calculate_eLengths (particle.f90:128): the short-edge flag goes to the host
   hipLaunchKernelGGL(k_clear_rm, dim3(1), dim3(1), 0, s, ctx->d_body);
   hipLaunchKernelGGL(k_edge_len, dim3(nb(ctx->ne, 256)), dim3(256), 0, s, A, ctx->d_lag[MELT_L_XYZV], ctx->d_body, ctx->h_body.e_thresh);
@@ -944,6 +979,7 @@ int lagr_alloc(melt_ctx* ctx, const double* xyz0, const int* voe, const int* eof
   rc |= dalloc((void**)&ctx->d_pcoef, sizeof(double) * 27 * 3 * 6 * nf);
   rc |= dalloc((void**)&ctx->d_foe, sizeof(int) * 2 * ne);
   if (ctx->cfg.iremesh == 1) rc |= dalloc((void**)&ctx->d_xyz_melt, sizeof(double) * 3 * nv);
+  else rc |= dalloc((void**)&ctx->d_xold, sizeof(double) * 3 * nv);
   if (rc) return MELT_ERR_HIP;
   if (ctx->cfg.iremesh == 1) {
     if (!ctx->h_rm) MELT_HIP(hipHostMalloc((void**)&ctx->h_rm, sizeof(int32_t)));
