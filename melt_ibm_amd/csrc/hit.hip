@@ -25,7 +25,6 @@
 
 namespace {
 
-constexpr int HIT_ZSEG = 32;   // z planes per synthesis thread
 
 __host__ __device__ inline unsigned long long hit_mix(unsigned long long seed, unsigned long long d) {
   unsigned long long z = seed + (d + 1ull) * 0x9E3779B97F4A7C15ull;
@@ -91,8 +90,8 @@ __global__ __launch_bounds__(1024) void k_hit_ou(HitArgs a, const int* __restric
 //
 // The x sum depends only on i: k_hit_xsum forms ax(c, n, m, i) =
 // sum_l Fhat(c,l,m,n) e^{i k_l x_i} once per grid line instead of once per
-// (i, j) column.  k_hit_synth then takes, per (i, j) column and 32-plane
-// segment, the y sum of those (75 complex products for nm = 5) and per plane
+// (i, j) column.  k_hit_synth then takes, per (i, j) column and segment
+// of planes, the y sum of those (75 complex products for nm = 5) and per plane
 // the z sum (15 real parts): about 40 FP64 FMAs per cell, so the pass is
 // bound by its field stores.
 template <int NM>
@@ -120,7 +119,7 @@ __global__ __launch_bounds__(256) void k_hit_xsum(int n1, const double* __restri
 // scalar loads.
 template <typename R, int NM>
 __global__ __launch_bounds__(256) void k_hit_synth(Grid g, const double* __restrict__ ax, const double* __restrict__ tab,
-                                                   R* __restrict__ fx, R* __restrict__ fy, R* __restrict__ fz, int bps) {
+                                                   R* __restrict__ fx, R* __restrict__ fy, R* __restrict__ fz, int bps, int zseg) {
   const int cols = g.n1 * g.n2;
   const int seg = (int)blockIdx.x / bps, col = ((int)blockIdx.x % bps) * 256 + (int)threadIdx.x;
   if (col >= cols) return;
@@ -147,7 +146,7 @@ __global__ __launch_bounds__(256) void k_hit_synth(Grid g, const double* __restr
     }
   }
   R* out[3] = {fx, fy, fz};
-  const int k0 = seg * HIT_ZSEG, k1 = min(n3, k0 + HIT_ZSEG);
+  const int k0 = seg * zseg, k1 = min(n3, k0 + zseg);
   for (int k = k0; k < k1; ++k) {
     const size_t o = (size_t)i + (size_t)n1 * ((size_t)j + (size_t)n2 * k);
 #pragma unroll
@@ -253,12 +252,18 @@ extern "C" int melt_hit_init(melt_ctx* ctx, double tl, double epsstar, double kf
 
 template <typename R, int NM>
 static int launch_hit_synth_nm(melt_ctx* ctx) {
-  const int nseg = (ctx->n3 + HIT_ZSEG - 1) / HIT_ZSEG;
   const int bps = (int)nblk((size_t)ctx->n1 * ctx->n2, 256);
+  // planes per block: each repeats its columns' y sums (150 loads a thread), so as
+  // many as leave 512 blocks, up to 64 (the whole synthesis, 8 / 16 / 32 / 64 planes:
+  // 256^3 FP32 142 / 98 / 81 / 68 us, FP64 164 / 121 / 99 / 96; 128^3 30 / 30 / 33 / 42;
+  // 64^3 24 / 26 / 31 / 40)
+  int zseg = 64;
+  while (zseg > 8 && bps * ((ctx->n3 + zseg - 1) / zseg) < 512) zseg /= 2;
+  const int nseg = (ctx->n3 + zseg - 1) / zseg;
   hipLaunchKernelGGL((k_hit_xsum<NM>), dim3(nblk((size_t)3 * NM * NM * ctx->n1, 256)), dim3(256), 0, ctx->stream, ctx->n1, ctx->d_hit_fhat,
                      ctx->d_hit_tab, ctx->d_hit_ax);
   hipLaunchKernelGGL((k_hit_synth<R, NM>), dim3((unsigned)(bps * nseg)), dim3(256), 0, ctx->stream, make_grid(ctx), ctx->d_hit_ax,
-                     ctx->d_hit_tab, fld<R>(ctx, MELT_FORCX), fld<R>(ctx, MELT_FORCY), fld<R>(ctx, MELT_FORCZ), bps);
+                     ctx->d_hit_tab, fld<R>(ctx, MELT_FORCX), fld<R>(ctx, MELT_FORCY), fld<R>(ctx, MELT_FORCZ), bps, zseg);
   MELT_HIP(hipGetLastError());
   return 0;
 }
