@@ -344,7 +344,8 @@ int melt_graph_enable(melt_ctx* ctx, int32_t on);
  * (BUFF_SIZE of pencil_rayTag.f90:84, n1m there; more faces raise
  * MELT_ERR_PENCIL_OVERFLOW as the reference aborts), 9 = 1 keeps one cell per
  * thread in the z-marching explicit pass of the precision form (default: two
- * x-neighbour cells per thread there); value 0 = built-in choice.
+ * x-neighbour cells per thread there, where n1m is a multiple of 128 from
+ * 256); value 0 = built-in choice.
  * Results do not depend on it (key 8: as long as no pencil overflows). */
 int melt_set_tuning(melt_ctx* ctx, int32_t key, int32_t value);
 void* melt_stream(melt_ctx* ctx);
