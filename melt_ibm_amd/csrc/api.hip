@@ -768,7 +768,9 @@ static int side2_run(melt_ctx* ctx, F&& work) {
 // as soon as the geometry refresh has written the face centroids and normals:
 // it reads only the vertices and faces and writes only VOFp, sdf, its own
 // scratch and the window box, none of which the rest of the refresh, the
-// probe stage or the pressure phase touches, so it overlaps them all; so
+// probe stage or the pressure phase touches, so it overlaps them all (sphere
+// tagging also reads the centre of mass, which the refresh writes last: it is
+// queued behind the refresh instead); so
 // does, with coef_next (every substep of tschem, also for the next call's
 // first substep: a caller's change of the faces or body in between cancels
 // it), the geometry part of the next substep's gradient probes (side stream,
@@ -851,9 +853,9 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
   timing_begin(ctx, SLOT_PH_MLS, &e_ph);
   // what the side stream queues after the Lagrangian update: the next
   // substep's tagging (tag_next) and probe geometry stage (coef_next).  The
-  // tagging needs only the refreshed faces (positions, centroids, normals):
-  // with a second side stream it forks there as soon as the refresh has
-  // written them, beside the rest of the refresh and the probe stage
+  // narrow-band tagging needs only the refreshed faces (positions, centroids,
+  // normals): with a second side stream it forks there as soon as the refresh
+  // has written them, beside the rest of the refresh and the probe stage
   auto tag_now = [&]() -> int {
     hipEvent_t et = nullptr;   // its own event: it may run inside the Lagrangian slot
     timing_begin(ctx, SLOT_TAG, &et);
@@ -944,7 +946,7 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
   // next substep's tagging and probe geometry stage
   if (ibm && (rc = side_continue(ctx, [&] {
                 timing_begin(ctx, SLOT_LAGR, &e);
-                if (tag_next && moving && !one_stream(ctx)) ctx->after_faces = &tag_fork;
+                if (tag_next && moving && c.tagtype != 0 && !one_stream(ctx)) ctx->after_faces = &tag_fork;
                 int r = lagr_after_force(ctx, true);
                 ctx->after_faces = nullptr;
                 timing_end(ctx, SLOT_LAGR, e);
