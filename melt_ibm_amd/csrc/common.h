@@ -451,7 +451,7 @@ __device__ inline void raise_error(int* err, int code) {
 // (block_max_to_slots: few atomics per address).  euler_fold_slots turns the
 // slots into one value and clears them.
 constexpr int REDUCE_SLOTS = 1024;
-__device__ inline double block_max(double v) {   // valid in thread 0
+__device__ inline double block_max(double v) {   // valid in thread 0; blocks of whole waves, all of whose threads call it
   __shared__ double wm[16];
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;

@@ -653,6 +653,9 @@ __global__ __launch_bounds__(rf_threads(P, Q, RF_NC), P * Q == 512 ? 2 : 1) void
 // 107 us, FP32 84 -> 70; at 192 16 pairs are slower, 40 -> 44 in FP32, at 128 and 384
 // the same).
 constexpr int x_pairs(int N) { return N == 64 || N == 256 ? 16 : N == 512 ? 4 : 8; }
+// Threads of a forward x block: whole waves, since its maximum of |div u| shuffles
+// over all 64 lanes of each (48 points: 8 pairs of 12 threads, 96, become 128).
+constexpr int x_fwd_threads(int P, int Q) { return (rf_threads(P, Q, x_pairs(P * Q)) + 63) / 64 * 64; }
 // Waves per SIMD the forward x pass asks for: 384 points in FP64 take 172 registers
 // by themselves, four above what three waves leave (486 -> 400 us).
 template <typename T>
@@ -664,12 +667,13 @@ constexpr int x_fwd_waves(int N) { return sizeof(T) == 8 && N == 384 ? 3 : 1; }
 // transform the two half spectra are separated with the mirror bins N-m,
 // exchanged through LDS.
 template <typename Rf, typename T, int P, int Q>
-__global__ __launch_bounds__(rf_threads(P, Q, x_pairs(P * Q)), x_fwd_waves<T>(P * Q)) void k_fft_x_fwd_reg(
+__global__ __launch_bounds__(x_fwd_threads(P, Q), x_fwd_waves<T>(P * Q)) void k_fft_x_fwd_reg(
     SpecArgs<T> S, const cx<T>* __restrict__ tw, const Rf* __restrict__ vx, const Rf* __restrict__ vy, const Rf* __restrict__ vz,
     const Rf* __restrict__ src, T usdtal, const int* __restrict__ gate, unsigned long long* __restrict__ div_slots) {
   if (gate && *gate == 0) return;
-  constexpr int N = P * Q, NPB = x_pairs(N), NT = rf_threads(P, Q, NPB), TB = NT / NPB;
+  constexpr int N = P * Q, NPB = x_pairs(N), NT = x_fwd_threads(P, Q), TB = NT / NPB;
   static_assert(N % (2 * NPB) == 0, "whole line pairs per block");
+  static_assert(NT % 64 == 0 && NT % NPB == 0, "whole waves, and as many threads for each pair");
   __shared__ RegFftLds<T, P, Q, NPB> L;
   static_assert(NPB * N <= (int)(sizeof(L.ex) / sizeof(L.ex[0])), "mirror exchange fits the transpose tile");
   const Grid& g = S.g;
@@ -922,7 +926,7 @@ int solve_t(melt_ctx* ctx, int fused_divg, const int* gate, unsigned long long* 
   if (!gate) timing_begin(ctx, SLOT_DIVG_FFTX, &ev);
   if (!with_reg_fft(ctx->n1, [&](auto P, auto Q) {
         constexpr int p = decltype(P)::value, q = decltype(Q)::value, npb = x_pairs(p * q);
-        hipLaunchKernelGGL((k_fft_x_fwd_reg<Rf, T, p, q>), dim3((unsigned)(ctx->n2 / (2 * npb) * ctx->n3)), dim3(rf_threads(p, q, npb)), 0,
+        hipLaunchKernelGGL((k_fft_x_fwd_reg<Rf, T, p, q>), dim3((unsigned)(ctx->n2 / (2 * npb) * ctx->n3)), dim3(x_fwd_threads(p, q)), 0,
                            ctx->stream, S, twx, fld<Rf>(ctx, MELT_VX), fld<Rf>(ctx, MELT_VY), fld<Rf>(ctx, MELT_VZ), src, usdtal, gate, dsl);
       }))
     hipLaunchKernelGGL((k_fft_x_fwd<Rf, T>), dim3(gx), dim3(FFT_NT), shx, ctx->stream, S, Px, twx, nlx, fld<Rf>(ctx, MELT_VX), fld<Rf>(ctx, MELT_VY),
