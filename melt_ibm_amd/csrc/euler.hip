@@ -1229,22 +1229,18 @@ __global__ __launch_bounds__(256) void k_interp_vof(Grid g, const R* __restrict_
 
 // Max reductions of cfl.f90:9-25 (what = 0), divgck divg.f90:36-50
 // (what = 1) and get_dt's advective measure cfl.f90:48-51 (what = 2, with dt),
-// in FP64 arithmetic whatever the storage type.  At most REDUCE_SLOTS blocks
-// walk the tiles of REDUCE_THREADS * V cells and store one (non-negative)
-// maximum each, so no slot has to be cleared beforehand.
-constexpr int REDUCE_THREADS = 512;
-inline unsigned reduce_tiles(size_t nc, int V) { return (unsigned)((nc / V + REDUCE_THREADS - 1) / REDUCE_THREADS); }
-inline unsigned reduce_blocks(size_t nc, int V) { return std::min(reduce_tiles(nc, V), (unsigned)REDUCE_SLOTS); }
+// in FP64 arithmetic whatever the storage type.  V cells a thread; the block's
+// maximum (non-negative) goes to a slot of its own while REDUCE_SLOTS blocks
+// cover the grid, else into slot blockIdx % REDUCE_SLOTS.
 template <typename R>
-__global__ __launch_bounds__(REDUCE_THREADS) void k_reduce_max(Grid g, const R* __restrict__ vx, const R* __restrict__ vy, const R* __restrict__ vz,
-                                                    int what, double dt, int nc, unsigned tiles, unsigned long long* __restrict__ slots) {
+__global__ __launch_bounds__(512) void k_reduce_max(Grid g, const R* __restrict__ vx, const R* __restrict__ vy, const R* __restrict__ vz,
+                                                    int what, double dt, int nc, unsigned long long* __restrict__ slots) {
   // V consecutive x cells per thread through 16-byte loads (n1 % V == 0)
   constexpr int V = 16 / sizeof(R);
   struct alignas(16) Vec { R v[V]; };
   double m = what == 0 ? 0.00000001 : 0.0;
-  for (unsigned t = blockIdx.x; t < tiles; t += gridDim.x) {
-    const unsigned at = (xcd_block(t, tiles) * blockDim.x + threadIdx.x) * V;
-    if (at >= (unsigned)nc) continue;
+  const unsigned at = (xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x) * V;
+  if (at < (unsigned)nc) {
     const int c = (int)at;
     const Cell s = make_cell(g, c);
     const Vec X = *reinterpret_cast<const Vec*>(vx + c), Y0 = *reinterpret_cast<const Vec*>(vy + c);
@@ -1264,8 +1260,11 @@ __global__ __launch_bounds__(REDUCE_THREADS) void k_reduce_max(Grid g, const R* 
       m = fmax(m, q);
     }
   }
-  block_max_store(m, slots + blockIdx.x);
+  if (gridDim.x <= REDUCE_SLOTS) block_max_store(m, slots + blockIdx.x);
+  else block_max_to_slots(m, slots);
 }
+// Threads per block: 512, for fewer partials, while their blocks have a slot each.
+inline int reduce_threads(size_t vecs) { return vecs <= (size_t)512 * REDUCE_SLOTS ? 512 : 256; }
 
 // The first `used` partial maxima into *out; all the slots are cleared for
 // the next reduction.  One block of FOLD_THREADS threads.
@@ -1671,11 +1670,13 @@ template <typename R>
 int launch_reduce_max(melt_ctx* ctx, int what, unsigned long long* d, double dt) {
   constexpr int V = 16 / sizeof(R);
   if (ctx->n1 % V) return melt_fail(ctx, MELT_ERR_ARG, "reduce_max", "n1m is not a multiple of the vector width");
-  const unsigned nb = reduce_blocks(ctx->nc, V);
-  hipLaunchKernelGGL(k_reduce_max<R>, dim3(nb), dim3(REDUCE_THREADS), 0, ctx->stream, make_grid(ctx), fld<R>(ctx, MELT_VX),
-                     fld<R>(ctx, MELT_VY), fld<R>(ctx, MELT_VZ), what, dt, (int)ctx->nc, reduce_tiles(ctx->nc, V), ctx->d_slots);
+  const size_t vecs = ctx->nc / V;
+  const int nt = reduce_threads(vecs);
+  const unsigned nb = nblocks(vecs, nt);
+  hipLaunchKernelGGL(k_reduce_max<R>, dim3(nb), dim3(nt), 0, ctx->stream, make_grid(ctx), fld<R>(ctx, MELT_VX), fld<R>(ctx, MELT_VY),
+                     fld<R>(ctx, MELT_VZ), what, dt, (int)ctx->nc, ctx->d_slots);
   MELT_HIP(hipGetLastError());
-  return euler_fold_slots(ctx, ctx->d_slots, d, (int)nb);
+  return euler_fold_slots(ctx, ctx->d_slots, d, (int)std::min(nb, (unsigned)REDUCE_SLOTS));
 }
 
 template <typename R>
@@ -1775,11 +1776,13 @@ int noalloc_scratch(unsigned long long** out) {
 template <typename R>
 int divgck_noalloc(const void* vx, const void* vy, const void* vz, const Grid& g, hipStream_t s, double* qmax, unsigned long long* slots) {
   constexpr int V = 16 / sizeof(R);
-  const size_t nc = (size_t)g.n1 * g.n2 * g.n3;
-  const unsigned nb = reduce_blocks(nc, V);
-  hipLaunchKernelGGL(k_reduce_max<R>, dim3(nb), dim3(REDUCE_THREADS), 0, s, g, static_cast<const R*>(vx), static_cast<const R*>(vy),
-                     static_cast<const R*>(vz), 1, 0.0, (int)nc, reduce_tiles(nc, V), slots);
-  hipLaunchKernelGGL(k_fold_slots, dim3(1), dim3(FOLD_THREADS), 0, s, slots, (int)nb, reinterpret_cast<unsigned long long*>(qmax));
+  const size_t nc = (size_t)g.n1 * g.n2 * g.n3, vecs = nc / V;
+  const int nt = reduce_threads(vecs);
+  const unsigned nb = nblocks(vecs, nt);
+  hipLaunchKernelGGL(k_reduce_max<R>, dim3(nb), dim3(nt), 0, s, g, static_cast<const R*>(vx), static_cast<const R*>(vy),
+                     static_cast<const R*>(vz), 1, 0.0, (int)nc, slots);
+  hipLaunchKernelGGL(k_fold_slots, dim3(1), dim3(FOLD_THREADS), 0, s, slots, (int)std::min(nb, (unsigned)REDUCE_SLOTS),
+                     reinterpret_cast<unsigned long long*>(qmax));
   return hipGetLastError() == hipSuccess ? 0 : MELT_ERR_HIP;
 }
 
