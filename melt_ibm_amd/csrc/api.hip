@@ -306,6 +306,11 @@ extern "C" int melt_sync(melt_ctx* ctx) {
 // second half converts while the first crosses the bus.  Bound by the bus (a
 // 256^3 field into pinned memory 2.4 ms; converted by the calling thread from
 // a temporary array it took 23 ms).
+//
+// Small fields convert on the calling thread instead, through ctx->h_conv: two
+// copies and two launches cost more than the conversion, and pageable memory
+// crosses at a third of the bus's rate, twice the bytes with it
+// (convert_on_host).
 template <typename R>
 __global__ __launch_bounds__(256) void k_from_double(R* __restrict__ dst, const double* __restrict__ src, size_t n) {
   for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (size_t)gridDim.x * blockDim.x) dst[c] = (R)src[c];
@@ -315,9 +320,31 @@ __global__ __launch_bounds__(256) void k_to_double(double* __restrict__ dst, con
 }
 static dim3 convert_grid(size_t n) { return dim3((unsigned)std::min<size_t>(2048, (n + 255) / 256)); }
 
+// Host or device conversion, us: pinned, download, 48^3 35 / 52, 64 x 64 x 48 55 /
+// 62, 64^3 98 / 73 (upload 28 / 53, 47 / 65, 78 / 75); pageable, download, 96^3 295 / 410,
+// 128^3 750 to 890 / 1000, 128 x 128 x 192 1500 / 1450; pageable, upload, 96^3 205 / 230,
+// 128 x 128 x 96 445 / 365 out of an array not in the caches (310 / 430 out of one
+// that is), 128^3 670 / 480 (485 / 560).  pageable_max: cells up to which pageable
+// memory converts on the host.
+static bool convert_on_host(const melt_ctx* ctx, const void* host, size_t pageable_max) {
+  if (ctx->nc < (size_t)64 * 64 * 64) return true;
+  if (ctx->nc > pageable_max) return false;
+  hipPointerAttribute_t at{};
+  const bool known = hipPointerGetAttributes(&at, host) == hipSuccess;
+  if (!known) (void)hipGetLastError();   // pageable memory is no error of the caller's
+  return !known || at.type == hipMemoryTypeUnregistered;
+}
+
 static int copy_to_device(melt_ctx* ctx, int field, const double* src) {
   if (!ctx->fp32) {
     MELT_HIP(hipMemcpy(ctx->f[field], src, sizeof(double) * ctx->nc, hipMemcpyHostToDevice));
+    return 0;
+  }
+  if (convert_on_host(ctx, src, (size_t)1 << 20)) {
+    ctx->h_conv.resize(ctx->nc);
+    float* t = ctx->h_conv.data();
+    for (size_t c = 0; c < ctx->nc; ++c) t[c] = (float)src[c];
+    MELT_HIP(hipMemcpy(ctx->f[field], t, sizeof(float) * ctx->nc, hipMemcpyHostToDevice));
     return 0;
   }
   const size_t m = ctx->nc / 2;   // nc is even
@@ -334,6 +361,13 @@ static int copy_to_device(melt_ctx* ctx, int field, const double* src) {
 static int copy_from_device(melt_ctx* ctx, int field, double* dst) {
   if (!ctx->fp32) {
     MELT_HIP(hipMemcpy(dst, ctx->f[field], sizeof(double) * ctx->nc, hipMemcpyDeviceToHost));
+    return 0;
+  }
+  if (convert_on_host(ctx, dst, (size_t)1 << 21)) {
+    ctx->h_conv.resize(ctx->nc);
+    float* t = ctx->h_conv.data();
+    MELT_HIP(hipMemcpy(t, ctx->f[field], sizeof(float) * ctx->nc, hipMemcpyDeviceToHost));
+    for (size_t c = 0; c < ctx->nc; ++c) dst[c] = (double)t[c];
     return 0;
   }
   const size_t m = ctx->nc / 2;

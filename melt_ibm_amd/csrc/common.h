@@ -181,6 +181,7 @@ struct melt_ctx {
 
   int* d_err = nullptr;    // device error word (first error wins)
   int* h_err = nullptr;    // pinned mirror
+  std::vector<float> h_conv;   // precision form: a small field on its way between the host's doubles and the device
   int defer_mean = 0;      // fused path: mean force applied in the projection
   int force_window_from_tag = 0;  // fused substep: tagging also places the forcing window
   int tag_ahead = 0;              // the next substep's tagging is already queued (side stream)
