@@ -335,6 +335,18 @@ static bool convert_on_host(const melt_ctx* ctx, const void* host, size_t pageab
   return !known || at.type == hipMemoryTypeUnregistered;
 }
 
+// Queues both halves of a field through their scratch buffer and waits, also
+// after an error: the caller's array is not in flight when the call returns.
+template <class F>
+static int through_halves(melt_ctx* ctx, F&& half) {
+  hipError_t e = hipSuccess;
+  for (int h = 0; h < 2 && e == hipSuccess; ++h) e = half(static_cast<double*>(ctx->tmp4[h]), h, ctx->nc / 2);   // nc is even
+  const hipError_t w = hipStreamSynchronize(ctx->stream);
+  MELT_HIP(e);
+  MELT_HIP(w);
+  return 0;
+}
+
 static int copy_to_device(melt_ctx* ctx, int field, const double* src) {
   if (!ctx->fp32) {
     MELT_HIP(hipMemcpy(ctx->f[field], src, sizeof(double) * ctx->nc, hipMemcpyHostToDevice));
@@ -347,15 +359,11 @@ static int copy_to_device(melt_ctx* ctx, int field, const double* src) {
     MELT_HIP(hipMemcpy(ctx->f[field], t, sizeof(float) * ctx->nc, hipMemcpyHostToDevice));
     return 0;
   }
-  const size_t m = ctx->nc / 2;   // nc is even
-  for (int h = 0; h < 2; ++h) {
-    double* st = static_cast<double*>(ctx->tmp4[h]);
-    MELT_HIP(hipMemcpyAsync(st, src + h * m, sizeof(double) * m, hipMemcpyHostToDevice, ctx->stream));
+  return through_halves(ctx, [&](double* st, int h, size_t m) {
+    if (hipError_t e = hipMemcpyAsync(st, src + h * m, sizeof(double) * m, hipMemcpyHostToDevice, ctx->stream)) return e;
     hipLaunchKernelGGL(k_from_double<float>, convert_grid(m), dim3(256), 0, ctx->stream, fld<float>(ctx, field) + h * m, st, m);
-  }
-  MELT_HIP(hipGetLastError());
-  MELT_HIP(hipStreamSynchronize(ctx->stream));
-  return 0;
+    return hipGetLastError();
+  });
 }
 
 static int copy_from_device(melt_ctx* ctx, int field, double* dst) {
@@ -370,15 +378,11 @@ static int copy_from_device(melt_ctx* ctx, int field, double* dst) {
     for (size_t c = 0; c < ctx->nc; ++c) dst[c] = (double)t[c];
     return 0;
   }
-  const size_t m = ctx->nc / 2;
-  for (int h = 0; h < 2; ++h) {
-    double* st = static_cast<double*>(ctx->tmp4[h]);
+  return through_halves(ctx, [&](double* st, int h, size_t m) {
     hipLaunchKernelGGL(k_to_double, convert_grid(m), dim3(256), 0, ctx->stream, st, fld<float>(ctx, field) + h * m, m);
-    MELT_HIP(hipGetLastError());
-    MELT_HIP(hipMemcpyAsync(dst + h * m, st, sizeof(double) * m, hipMemcpyDeviceToHost, ctx->stream));
-  }
-  MELT_HIP(hipStreamSynchronize(ctx->stream));
-  return 0;
+    if (hipError_t e = hipGetLastError()) return e;
+    return hipMemcpyAsync(dst + h * m, st, sizeof(double) * m, hipMemcpyDeviceToHost, ctx->stream);
+  });
 }
 
 extern "C" int melt_upload_field(melt_ctx* ctx, int field, const double* host, const melt_layout* lay) {
