@@ -905,9 +905,10 @@ static int substep_impl(melt_ctx* ctx, int32_t ns, bool tag_next, bool coef_next
     return r;
   };
   const std::function<int()> tag_fork = [&]() -> int { return side2_run(ctx, tag_now); };
-  // within a tschem call (tag_next) the main stream does not wait for the
-  // probe geometry stage: only the next substep's probes read its output, and
-  // they run on the side stream after it; the call's last substep joins it
+  // within a tschem call (tag_next) the substep's join does not wait for the probe
+  // geometry stage: only the field part of the next substep's probes reads its
+  // output, on the main stream with the spreading, which waits for ev_coef
+  // (coef_pending) there; the call's last substep queues it before its join
   const bool coef_after_join = tag_next && coef_next && probes && !one_stream(ctx);
   auto queue_coef = [&]() -> int {
     int r = coef_after_join ? side_coefs() : ibm_probe_coefs(ctx);
