@@ -169,7 +169,6 @@ extern "C" int melt_ctx_create(const melt_config* cfg, melt_ctx** out) {
   ctx->cfg = *cfg;
   ctx->fp32 = cfg->precision == 1;
   ctx->esz = ctx->fp32 ? sizeof(float) : sizeof(double);
-  ctx->spec64 = !ctx->fp32;
   ctx->n1 = cfg->n1m; ctx->n2 = cfg->n2m; ctx->n3 = cfg->n3m;
   ctx->nc = (size_t)ctx->n1 * ctx->n2 * ctx->n3;
   ctx->n1h = ctx->n1 / 2 + 1;

@@ -99,15 +99,14 @@ struct melt_ctx {
   // Eulerian fields: double, or float in the precision form (fp32 = 1); fld<R>()
   int fp32 = 0;
   size_t esz = sizeof(double);
-  // Poisson spectrum, twiddles and FFT arithmetic in FP64 (the FP64 form); the
-  // precision form keeps them in FP32 (an FP64 spectrum there was measured to
-  // leave its pressure difference to FP64 unchanged, at 0.28 ms per step)
-  int spec64 = 1;
   void* f[MELT_NFIELDS] = {};
   void* rhs4[4] = {};
   void* tmp4[4] = {};      // output of the y-direction Green filters (the z pass reads it)
   int no_green = 0;        // MELT_TUNE green=0: cyclic reduction for every line solve
-  void* spec = nullptr;                                    // complex, double if spec64 else float
+  // Poisson spectrum, twiddles and FFT arithmetic in the fields' precision (an FP64
+  // spectrum for the precision form was measured to leave its pressure difference
+  // to FP64 unchanged, at 0.28 ms per step)
+  void* spec = nullptr;                                    // complex
   double *ak1 = nullptr, *ak2 = nullptr, *ak3 = nullptr;   // 0-based wavenumber index
   void *tw1 = nullptr, *tw2 = nullptr, *tw3 = nullptr;     // exp(-2 pi i t / N), complex of the field type
   // precision-form pressure refinement: up to refine_max correction solves while

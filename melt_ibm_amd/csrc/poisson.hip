@@ -881,7 +881,7 @@ int poisson_init(melt_ctx* ctx) {
   for (int d = 0; d < 3; ++d) {
     FftPlan P;
     if (!make_plan(n[d], P)) return melt_fail(ctx, MELT_ERR_ARG, "poisson_init", "grid size must be 2^a 3^b");
-    int rc = ctx->spec64 ? upload_twiddles<double>(ctx, n[d], tw[d]) : upload_twiddles<float>(ctx, n[d], tw[d]);
+    int rc = ctx->fp32 ? upload_twiddles<float>(ctx, n[d], tw[d]) : upload_twiddles<double>(ctx, n[d], tw[d]);
     if (rc) return rc;
     // phini.f90:35-55, 0-based index m -> reference index m+1
     std::vector<double> a(n[d]);
@@ -894,7 +894,7 @@ int poisson_init(melt_ctx* ctx) {
     MELT_HIP(hipMalloc(ak[d], sizeof(double) * n[d]));
     MELT_HIP(hipMemcpy(*ak[d], a.data(), sizeof(double) * n[d], hipMemcpyHostToDevice));
   }
-  size_t sz = 2 * (ctx->spec64 ? sizeof(double) : sizeof(float)) * (size_t)ctx->n1hp * ctx->n2 * ctx->n3;
+  size_t sz = 2 * ctx->esz * (size_t)ctx->n1hp * ctx->n2 * ctx->n3;
   MELT_HIP(hipMalloc(&ctx->spec, sz));
   MELT_HIP(hipMemset(ctx->spec, 0, sz));
   return 0;
