@@ -703,7 +703,10 @@ extern "C" int melt_particle(melt_ctx* ctx) {
 // joins add (10 steps, one against several streams, eager / as a graph: 32^3 FP64 4.0
 // / 3.7 ms against 5.6 / 4.4; 64^3 with 1280 faces 5.0 / 5.1 against 6.0 / 5.3, with
 // 5120 5.7 / 5.8 against 6.2 / 5.8; 96^3 with 2880 8.1 / 8.2 against 8.2 / 7.9, with
-// 11520 9.4 / 9.4 against 9.2 / 9.2; FP32 alike).
+// 11520 9.4 / 9.4 against 9.2 / 9.2; FP32 alike).  So with remeshing, although one
+// stream's short-edge flag reaches the host behind the pressure phase (ms a step: 32^3
+// 0.46 against 0.54, 64^3 with 1280 faces 0.54 against 0.59, with 5120 0.59 / 0.61), and
+// with HIT forcing (64^3 without a body 0.210 / 0.219, with 1280 faces 0.49 / 0.50).
 static bool one_stream(const melt_ctx* ctx) {
   const int t = ctx->tune[TUNE_STREAMS];
   return t == 1 || (t == 0 && ctx->nc <= (size_t)64 * 64 * 64);

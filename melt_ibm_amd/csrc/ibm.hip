@@ -1665,7 +1665,10 @@ static int ibm_tag_t(melt_ctx* ctx, bool wgt, bool coef) {  // tagCells.f90:4-27
   // As many faces a group as keep the chip's blocks busy (20480 faces on 128^3:
   // 16 a group 42 us for the three passes, 8 50; 5120 faces: 8 22, 16 27; 1280: 4
   // 16, 8 17), with twice the cells a group of neighbours touches in its table
-  // (16 faces with 1024 cells often leave their distances: 62).
+  // (16 faces with 1024 cells often leave their distances: 62).  Beside the lines: a
+  // tagCells call of 9680 faces 46 us with 16 or 8, 11520 48 and 51, 14580 53 and 57; a
+  // step at 128^3 with 8000 faces 1.08 ms with 16, 1.05 with 8; with 2420 and 2880 4 and 8
+  // are level.
   if (ctx->nf > 8192) TAG_PASSES(16, 512, 2048);
   else if (ctx->nf > 2560) TAG_PASSES(8, 512, 1024);
   else TAG_PASSES(4, 512, 512);
@@ -1723,7 +1726,9 @@ static int ibm_force_scatter_t(melt_ctx* ctx, bool with_probes) {
   // per block 27 us, 32 46, one update per face and cell 77).  Fewer faces: more
   // blocks (5120 faces with the probes: 32 by 256 threads 15 us, 16 24, 32 by 512, of
   // which a CU holds two, 24), and more faces at a time (1280 faces alone: 16 by
-  // 512 threads 6.7 us, 8 by 256 8.1, 64 15.6).
+  // 512 threads 6.7 us, 8 by 256 8.1, 64 15.6).  Beside the lines, a step: 96^3 with
+  // 2420 faces 0.71 ms with 16 by 512, 0.69 with 32 by 256, with 2880 0.70 and 0.69; 128^3 in
+  // FP32 with 8000 0.76 with 64 or 32, with 8820 0.81 with 64, 0.82 with 32.
   if (ctx->nf > 8192) MLS_FORCE(256, 64);
   else if (ctx->nf > 2560) MLS_FORCE(256, 32);
   else MLS_FORCE(512, 16);
