@@ -1,8 +1,8 @@
 """Steps on several streams (tuning key streams = 2) on grids that take one by
 themselves: what is queued ahead across substeps and calls, its cancelling, graph
 replay, snapshots, remeshing and sphere tagging, as the checks of those parts do
-them; and replayed graphs and both places of the probes' geometry stage against
-one stream."""
+them; and replayed graphs, both places of the probes' geometry stage, the HIT
+forcing and remeshing against one stream, bit for bit."""
 import numpy as np
 import pytest
 
@@ -52,10 +52,25 @@ def test_sphere_tagging(gpu_lib, several, precision):
     test_gpu_parity.test_sphere_tagging_and_step(gpu_lib, precision)
 
 
+TUNES = (dict(streams=2), dict(streams=2, graph=1), dict(streams=2, coef=2), dict(streams=2, coef=2, graph=1))
+
+
 @pytest.mark.parametrize("precision", [0, 1])
-def test_graphs_and_coefficient_places_match_one_stream(gpu_lib, precision):
-    match_one_stream(gpu_lib, make_cfg(64, precision=precision),
-                     (dict(streams=2), dict(streams=2, graph=1), dict(streams=2, coef=2), dict(streams=2, coef=2, graph=1)))
+@pytest.mark.parametrize("kw", [{}, dict(imelt=0), dict(imlsstr=0)], ids=["melt+move", "move", "melt"])
+def test_graphs_and_coefficient_places_match_one_stream(gpu_lib, kw, precision):
+    match_one_stream(gpu_lib, make_cfg(64, precision=precision, **kw), TUNES)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_forcing_beside_the_step_matches_one_stream(gpu_lib, precision):
+    match_one_stream(gpu_lib, make_cfg(64, precision=precision), (dict(streams=2), dict(streams=2, graph=1)), hit=True)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_remeshing_matches_one_stream(gpu_lib, precision):
+    cfg = test_gpu_remesh.remesh_cfg()
+    cfg.precision = precision
+    match_one_stream(gpu_lib, cfg, (dict(streams=2), dict(streams=2, coef=2)), level=test_gpu_remesh.LEVEL, rad=test_gpu_remesh.RAD, steps=3)
 
 
 @pytest.mark.parametrize("precision", [0, 1])

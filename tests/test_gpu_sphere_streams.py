@@ -11,7 +11,7 @@ from tests.helpers import load_state, make_cfg, melt_case, with_body
 pytestmark = pytest.mark.gpu
 
 
-def match_one_stream(gpu_lib, cfg, tunes, level=3, rad=1.2, steps=5):
+def match_one_stream(gpu_lib, cfg, tunes, level=3, rad=1.2, steps=5, hit=False):
     """Steps of a moving body under each tuning (graph=1: replayed) equal those on one stream."""
     st, dt = melt_case(make_cfg(cfg.n1m, cfg.n3m), level, rad, seed=23)
     ctxs = {}
@@ -23,12 +23,16 @@ def match_one_stream(gpu_lib, cfg, tunes, level=3, rad=1.2, steps=5):
         c.upload("temp", inqpr_temperature(cfg, c.body().pos_cm[:], rad))
         c.set_dt(dt)
         c.tagCells()
+        if hit:
+            c.hit_init(0.5, 0.05, 2.5, seed=7)
         c.graph("graph" in tune)
     one = next(iter(ctxs.values()))
     fields = ("vx", "vy", "vz", "temp", "pr", "VOFp", "VOFx", "VOFy", "VOFz")
     for step in range(steps):
         print(f"# tagType {cfg.tagtype} precision {cfg.precision} step {step}", flush=True)
         for c in ctxs.values():
+            if hit:
+                c.hit_force()
             c.tschem()
         want = {q: one.download(q) for q in fields}
         xyz = one.lag("xyzv")
